@@ -84,7 +84,7 @@ def draw(rng):
                      "scan", "flash"])
     C = rng.choice([64, 64, 128])
     if op == "gdn":
-        B, H, T = _chains(rng, 1 << 20, 32768, C)
+        B, H, T = _chains(rng, 960000, 32768, C)
         return _gdn("bf16", B, H, T, gated=rng.random() < 0.8, h0=rng.random() < 0.5, C=C)
     if op == "gdn_fp32":
         B, H, T = _chains(rng, 1 << 17, 4096, C)
