@@ -57,19 +57,6 @@ bool gdn_shape_ok(int B, int H, int T, int C, int DK, int DV, int dtype) {
          DV == 128 && T % C == 0 && valid_dtype(dtype);
 }
 
-// CUs of the device current at the first call (queried once, thread-safe; 256, MI355X's count,
-// if the query fails).
-int device_cu_count() {
-  static const int cus = [] {
-    int dev = 0, n = 0;
-    if (hipGetDevice(&dev) == hipSuccess &&
-        hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0)
-      return n;
-    return 256;
-  }();
-  return cus;
-}
-
 template <typename E>
 void chunk_local_launch(const void* q, const void* k, const float* beta, const float* g,
                        float scale, char* base, size_t M, hipStream_t stream) {
@@ -94,7 +81,7 @@ void chunk_local_launch(const void* q, const void* k, const float* beta, const f
   } else {
     // fp32 with P: when the chunks fit one generation of workgroups (short sequences, few
     // chains), P gets workgroups of its own, which halves each workgroup's products
-    a.split_p = M <= (size_t)device_cu_count() ? 1 : 0;
+    a.split_p = M <= (size_t)pf::device_cu_count() ? 1 : 0;
     const unsigned grid = (unsigned)(a.split_p ? 2 * M : M);
     pf::chunk_local_kernel<E, E, C, DK, true, true><<<dim3(grid), dim3(256), 0, stream>>>(a);
   }
@@ -125,7 +112,7 @@ void scan_output_launch(const void* q, const void* k, const void* v, const float
     // bf16: one workgroup per (chain, 32-column slice), or 16-column slices when 32 would leave
     // CUs idle (fewer than 8 chains per 32 CUs: long sequences at small batch); four MFMA waves
     // split every chunk (pf_scan_split.h)
-    if ((size_t)BH * (DV / 32) < (size_t)device_cu_count())
+    if ((size_t)BH * (DV / 32) < (size_t)pf::device_cu_count())
       pf::scan_split_kernel<C, DK, DV, 1, kSplit16LoaderWaves>
           <<<dim3((unsigned)(BH * (DV / 16))), dim3(64 * (4 + kSplit16LoaderWaves)), 0, stream>>>(a);
     else

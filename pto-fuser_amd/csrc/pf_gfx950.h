@@ -26,6 +26,11 @@ __device__ __forceinline__ uint4 buf_load16(__amdgpu_buffer_rsrc_t r, uint32_t v
   return make_uint4(v[0], v[1], v[2], v[3]);
 }
 
+// Swz<RS, RM> names the swizzle of a row-major bf16 LDS tile: its 4-element column groups are
+// XOR-permuted by row bits, group' = group ^ ((row >> RS) & RM), so that the MFMA operand reads
+// (16 rows x one group) and the transposed reads spread over all banks.  With RM = 1 a 16-byte
+// vector (two groups) stays in place and only its two 8-byte halves swap.
+//
 // Store of a 16-byte row vector into a Swz<RS,1> tile slot whose 8-byte halves are swapped when
 // `swap` (a compile-time constant at every call): the halves change places in registers and the
 // LDS store stays one conflict-free 16-byte write (two 8-byte stores would conflict).

@@ -8,9 +8,7 @@
 //   qkv_flash_kernel  o = causal_incl(the same score) v, the score kept on chip
 //                     (qkv_flash_native*, qkv_fused.h:62-175; qkvp_flash_native*,
 //                     qkv_prologue_fused.h:99-187).
-//   scan_state_kernel chunk_h_scan: h_out[c] = S;  S = decay (.) S + k^T (u - w S), scalar decay
-//                     per chunk or a per-row (per key channel) decay vector
-//                     (scan_fused.h:198-262; vec_recurrence_perdim :143-180).
+// (The third stage, the resident-state scan, is in pf_state_scan.h.)
 //
 // Row addressing.  The reference runs these stages on two layouts: the native batch [M, C, D]
 // (heads outer) and the "mega" token layout [nc*C, H, D] (= [1, T, H, D]).  Both are described
@@ -18,8 +16,7 @@
 // layout.  Gates follow the same rule with row length 1, scores with row length C.
 //
 // gfx950 mapping: 256-thread workgroups (4 waves) per chunk for the two score kernels, every
-// 16x16 output block one MFMA chain (bf16 16x16x32 or fp32 16x16x4); the scan keeps its
-// [D x 16] state slice in registers across the whole chunk loop, one wave per 16 columns.
+// 16x16 output block one MFMA chain (bf16 16x16x32 or fp32 16x16x4).
 #pragma once
 
 #include "pf_device.h"
@@ -203,94 +200,6 @@ __global__ __launch_bounds__(256) void qkv_flash_kernel(QkvFlashArgs p) {
         r = Mfma<E>::rows(r, rx + (16 * bi + c) * LP, ry + (16 * bn + c) * VP, kb, g);
 #pragma unroll
     for (int ii = 0; ii < 4; ++ii) o[(size_t)(16 * bi + 4 * g + ii) * D + 16 * bn + c] = r[ii];
-  }
-}
-
-struct ScanStateArgs {
-  const void* w;        // [B, nc, C, H, D] E
-  const void* u;        // [B, nc, C, H, D] E
-  const void* k;        // [B, nc, C, H, D] E
-  const float* decay;   // [B, H, nc] (scalar) or [B, H, nc, D] (per row)
-  const float* h0;      // [B, H, D, D] or null (zero)
-  void* h_out;          // [B, nc, H, D, D] fp32 or bf16
-  float* final_state;   // [B, H, D, D] or null
-  int H, NC, perdim, out_f32;
-};
-
-// One workgroup per (b, h, 16*NW-column slice of the state); wave w owns 16 columns.
-template <typename E, int C, int D, int NW>
-__global__ __launch_bounds__(64 * NW) void scan_state_kernel(ScanStateArgs p) {
-  constexpr int PE = 16 / sizeof(E), KP = D + PE, TP = C + PE, VE = Vec16<E>::N;
-  constexpr int NKB_D = D / Mfma<E>::KB, NKB_C = C / Mfma<E>::KB, MB = C / 16, NTHR = 64 * NW;
-  constexpr int TW = 16 * NW, NT = D / TW;
-  using SW = Swz<0, 0>;
-  typedef typename VecT<E>::T V;
-  __shared__ __attribute__((aligned(16))) E ws[C * KP];
-  __shared__ __attribute__((aligned(16))) E kts[D * TP];
-  __shared__ __attribute__((aligned(16))) E us[C * TW];
-  __shared__ float dec[D];
-
-  const int bh = blockIdx.x / NT, tile = blockIdx.x % NT;
-  const int b = bh / p.H, h = bh % p.H;
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, g = lane >> 4, c = lane & 15;
-  const int col = tile * TW + w * 16 + c;
-  const size_t rs = (size_t)p.H * D;    // token row stride of [.., C, H, D]
-
-  floatx4 S[D / 16];
-#pragma unroll
-  for (int r = 0; r < D / 16; ++r)
-#pragma unroll
-    for (int ii = 0; ii < 4; ++ii)
-      S[r][ii] = p.h0 ? p.h0[((size_t)bh * D + 16 * r + 4 * g + ii) * D + col] : 0.f;
-
-  for (int ch = 0; ch < p.NC; ++ch) {
-    const size_t base = (((size_t)b * p.NC + ch) * C * p.H + h) * D;   // token 0 of chunk, head h
-    const E* wg = static_cast<const E*>(p.w) + base;
-    const E* ug = static_cast<const E*>(p.u) + base;
-    const E* kg = static_cast<const E*>(p.k) + base;
-    for (int i = tid; i < C * (D / VE); i += NTHR) {
-      const int t = i / (D / VE), d0 = (i % (D / VE)) * VE;
-      *reinterpret_cast<uint4*>(ws + t * KP + d0) = *reinterpret_cast<const uint4*>(wg + t * rs + d0);
-      const V x = __builtin_bit_cast(V, *reinterpret_cast<const uint4*>(kg + t * rs + d0));
-#pragma unroll
-      for (int e = 0; e < VE; ++e) kts[(d0 + e) * TP + t] = x[e];
-    }
-    for (int i = tid; i < C * TW; i += NTHR) us[i] = ug[(i / TW) * rs + tile * TW + (i % TW)];
-    for (int i = tid; i < D; i += NTHR)
-      dec[i] = p.perdim ? p.decay[((size_t)bh * p.NC + ch) * D + i] : p.decay[(size_t)bh * p.NC + ch];
-    lds_barrier();
-
-    // snapshot before the update
-    const size_t hbase = (((size_t)b * p.NC + ch) * p.H + h) * D * D;
-#pragma unroll
-    for (int r = 0; r < D / 16; ++r)
-#pragma unroll
-      for (int ii = 0; ii < 4; ++ii)
-        store_out(p.h_out, hbase + (size_t)(16 * r + 4 * g + ii) * D + col, S[r][ii], p.out_f32);
-    // vc = u - w S   (token rows 16mb + 4g + ii, column col)
-    floatx4 Vc[MB];
-#pragma unroll
-    for (int mb = 0; mb < MB; ++mb) {
-      const floatx4 X = chain<E, NKB_D, SW>(zero4(), ws, 16 * mb + c, KP, S, NKB_D, g);
-#pragma unroll
-      for (int ii = 0; ii < 4; ++ii) Vc[mb][ii] = to_f32(us[(16 * mb + 4 * g + ii) * TW + w * 16 + c]) - X[ii];
-    }
-    // S = decay (.) S + k^T vc   (per-row decay scales state row d)
-#pragma unroll
-    for (int r = 0; r < D / 16; ++r) {
-      floatx4 sd;
-#pragma unroll
-      for (int ii = 0; ii < 4; ++ii) sd[ii] = S[r][ii] * dec[16 * r + 4 * g + ii];
-      S[r] = chain<E, NKB_C, SW>(sd, kts, 16 * r + c, TP, Vc, NKB_C, g);
-    }
-    lds_barrier();
-  }
-  if (p.final_state) {
-#pragma unroll
-    for (int r = 0; r < D / 16; ++r)
-#pragma unroll
-      for (int ii = 0; ii < 4; ++ii)
-        p.final_state[((size_t)bh * D + 16 * r + 4 * g + ii) * D + col] = S[r][ii];
   }
 }
 

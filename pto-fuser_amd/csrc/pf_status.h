@@ -21,4 +21,17 @@ struct LaunchScope {
   }
 };
 
+// CUs of the device current at the first call (queried once, thread-safe; 256, MI355X's count,
+// if the query fails).
+inline int device_cu_count() {
+  static const int cus = [] {
+    int dev = 0, n = 0;
+    if (hipGetDevice(&dev) == hipSuccess &&
+        hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0)
+      return n;
+    return 256;
+  }();
+  return cus;
+}
+
 }  // namespace pf

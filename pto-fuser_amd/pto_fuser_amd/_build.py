@@ -32,9 +32,12 @@ ARCH = os.environ.get("PF_OFFLOAD_ARCH", "gfx950")
 # The iterative-ILP machine scheduler issues the LDS operand reads of the scan's MFMA chains
 # several instructions ahead (the default strategy serialises every MFMA behind its own read,
 # which leaves a one-wave-per-SIMD kernel latency-bound).
+# It keeps the register file full of hoisted reads; the stage kernels, whose waves hold a prefetched
+# chunk beside the state, spill under it, so their source is compiled with the default strategy.
 HIPCC_FLAGS = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}",
-               "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
-               "-mllvm", "-amdgpu-sched-strategy=iterative-ilp"]
+               "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
+ILP_FLAGS = ["-mllvm", "-amdgpu-sched-strategy=iterative-ilp"]
+DEFAULT_SCHED_SOURCES = ("pf_stages.hip",)
 OBJ_DIR = os.path.join(ROOT, "_build")
 
 
@@ -53,6 +56,11 @@ def headers() -> List[str]:
     return sorted(glob.glob(os.path.join(CSRC, "*.h")) + glob.glob(os.path.join(INCLUDE, "*.h")))
 
 
+def flags(path: str) -> List[str]:
+    """The hipcc flags of one source."""
+    return HIPCC_FLAGS + ([] if os.path.basename(path) in DEFAULT_SCHED_SOURCES else ILP_FLAGS)
+
+
 def source_hash() -> str:
     """16 hex digits of SHA-256 over every source and header (name and content) and the hipcc
     flags: what the library's ``pf_source_hash()`` must return for it to be current."""
@@ -62,7 +70,7 @@ def source_hash() -> str:
         with open(path, "rb") as f:
             h.update(f.read())
         h.update(b"\0")
-    h.update(" ".join(HIPCC_FLAGS).encode())
+    h.update("\n".join(" ".join(flags(s)) for s in sources()).encode())
     return h.hexdigest()[:16]
 
 
@@ -89,7 +97,7 @@ def build(verbose: bool = False, out: Optional[str] = None) -> str:
     tag = f'-DPF_SOURCE_HASH="{source_hash()}"'
     try:
         with ThreadPoolExecutor(jobs) as pool:
-            list(pool.map(lambda so: _run([hipcc, *HIPCC_FLAGS, tag, "-I", INCLUDE, "-c", so[0],
+            list(pool.map(lambda so: _run([hipcc, *flags(so[0]), tag, "-I", INCLUDE, "-c", so[0],
                                            "-o", so[1]], verbose), zip(srcs, objs)))
         tmp = out + f".tmp{os.getpid()}"
         _run([hipcc, "-shared", "-fPIC", f"--offload-arch={ARCH}", *objs, "-o", tmp], verbose)
@@ -109,7 +117,7 @@ def build_probe(verbose: bool = False) -> str:
     ``lib/pf_memfloor``; returns its path."""
     os.makedirs(LIB_DIR, exist_ok=True)
     tmp = PROBE_PATH + f".tmp{os.getpid()}"
-    _run([_hipcc(), *[f for f in HIPCC_FLAGS if f != "-fPIC"], PROBE_SRC, "-o", tmp], verbose)
+    _run([_hipcc(), *[f for f in flags(PROBE_SRC) if f != "-fPIC"], PROBE_SRC, "-o", tmp], verbose)
     os.replace(tmp, PROBE_PATH)
     return PROBE_PATH
 
