@@ -119,7 +119,7 @@ int pf_kda_exec(const void* q, const void* k, const void* v, const float* beta, 
     sa.h_final = h_final;
     sa.BH = B * H;
     sa.NC = T / kChunk;
-    pf::kda_scan_f32_kernel<KC, KD, KD><<<dim3((unsigned)(B * H * (KD / 32))), dim3(128), 0, s>>>(sa);
+    pf::kda_scan_f32_kernel<KC, KD, KD><<<dim3((unsigned)(B * H * (KD / 16))), dim3(256), 0, s>>>(sa);
     return scope.status();
   }
 

@@ -232,104 +232,203 @@ struct KdaScanF32Args {
   int BH, NC;
 };
 
+// One workgroup per (chain, 16-column slice), four waves; wave w owns state rows 32w .. 32w+31 (MFMA
+// D layout, in registers for the whole chain).  Per chunk:
+//
+//   1.  partial (W S)_w and (QE S)_w over the wave's rows for all 64 tokens              -> LDS
+//   2a. wave w: v_new of token tile w = U - sum of the partials -> LDS; the QE S partials of its
+//       o tile 3 - w summed
+//   2b. every wave reads all of v_new; wave w: o of token tile 3 - w = QE S + P v_new -> HBM;
+//       S_w <- e^{G_last} (.) S_w + KR[:, rows of w]^T v_new
+//
+// (64 + 4..16 + 32 products per wave and chunk).  Wave w reads only columns 32w .. 32w+31 of the W, QE
+// and KR rows, so it loads those slices itself and refills them after its own last read, with no
+// barrier; P is written between the barriers (its readers are past the first one), U after the
+// second.  Two barriers per chunk, the next chunk's loads in flight across both.
 template <int C, int DK, int DV>
-__global__ __launch_bounds__(128) void kda_scan_f32_kernel(KdaScanF32Args a) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
+void kda_scan_f32_kernel(KdaScanF32Args a) {
   static_assert(C == 64 && DK == 128 && DV == 128, "the fp32 KDA kernels are written for C 64, dk = dv = 128");
-  constexpr int RP = DK + 4, PP = C + 4, UP = 32 + 4;
+  constexpr int RP = DK + 4, UP = 16 + 4;
+  constexpr int TR = 20, TT = 16 * TR;                 // P: its ten lower 16x16 tiles, 20-float rows
   __shared__ __attribute__((aligned(16))) float Ws[C * RP];
   __shared__ __attribute__((aligned(16))) float Qs[C * RP];
   __shared__ __attribute__((aligned(16))) float Ks[C * RP];
-  __shared__ __attribute__((aligned(16))) float Ps[C * PP];
+  __shared__ __attribute__((aligned(16))) float Ps[10 * TT];
   __shared__ __attribute__((aligned(16))) float Us[C * UP];
-  __shared__ __attribute__((aligned(16))) float Ds[DK];
+  __shared__ __attribute__((aligned(16))) floatx4 YP[4 * 4 * 64];   // [wave][token tile][lane]
+  __shared__ __attribute__((aligned(16))) floatx4 QP[4 * 4 * 64];
+  __shared__ __attribute__((aligned(16))) floatx4 VX[4 * 64];       // v_new, [token tile][lane]
 
-  const int bh = blockIdx.x / (DV / 32), slice = blockIdx.x % (DV / 32);
+  constexpr int NS = DV / 16;
+  int bh, slice;
+  const int bid = blockIdx.x;
+  if (a.BH % 8 == 0) {  // the slices of one chain share an XCD: they read the same W, QE, KR, P
+    const int grp = bid / (8 * NS), within = bid % (8 * NS);
+    bh = grp * 8 + (within % 8);
+    slice = within / 8;
+  } else {
+    bh = bid / NS;
+    slice = bid % NS;
+  }
+  const int col0 = 16 * slice;
   const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, c = lane & 15;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int col0 = 32 * slice, mycol = col0 + 16 * w + c;   // this lane's state / o column
-  const size_t Tlen = (size_t)a.NC * C;
+  const int NC = a.NC, last = NC - 1;
+  const size_t m0 = (size_t)bh * NC, t0 = m0 * C;
 
-  floatx4 S[DK / 16];                                  // rows 16 r + 4g + ii, column mycol
+  // chunk data: global -> registers -> LDS.  Lane u of a wave's slice: row u / 8, columns 32w + 4 (u % 8)
+  floatx4 rw[8], rq[8], rk[8], rp[4], ru, rd[2];
+  const int srow = lane >> 3, scol = 32 * w + 4 * (lane & 7);
+  auto load_slice = [&](floatx4 (&r)[8], const float* src, int ch) {
+    const float* s = src + (t0 + (size_t)ch * C + srow) * DK + scol;
 #pragma unroll
-  for (int r = 0; r < DK / 16; ++r)
+    for (int i = 0; i < 8; ++i) r[i] = *reinterpret_cast<const floatx4*>(s + i * 8 * DK);
+  };
+  auto store_slice = [&](float* dst, const floatx4 (&r)[8]) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) *reinterpret_cast<floatx4*>(dst + (srow + 8 * i) * RP + scol) = r[i];
+  };
+  // thread tid holds P rows 16 i + tid / 16, columns 4 (tid % 16) ..: tile (i, (tid % 16) / 4)
+  const int p_row = tid >> 4, p_jb = (tid & 15) >> 2, p_col = 4 * (tid & 3);
+  auto load_p = [&](int ch) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      rp[i] = *reinterpret_cast<const floatx4*>(a.P + ((m0 + ch) * C + 16 * i + p_row) * C + 4 * (tid & 15));
+  };
+  auto store_p = [&]() {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (p_jb <= i) *reinterpret_cast<floatx4*>(Ps + score_tile_index(i, p_jb) * TT + p_row * TR + p_col) = rp[i];
+  };
+  auto load_u = [&](int ch) {
+    ru = *reinterpret_cast<const floatx4*>(a.U + (t0 + (size_t)ch * C + (tid >> 2)) * DV + col0 + 4 * (tid & 3));
+  };
+  auto store_u = [&]() { *reinterpret_cast<floatx4*>(Us + (tid >> 2) * UP + 4 * (tid & 3)) = ru; };
+  auto load_d = [&](int ch) {
+#pragma unroll
+    for (int r = 0; r < 2; ++r)
+      rd[r] = *reinterpret_cast<const floatx4*>(a.DEC + (m0 + ch) * DK + 32 * w + 16 * r + 4 * g);
+  };
+
+  floatx4 S[2];                                        // rows 32w + 16r + 4g + ii, column col0 + c
+#pragma unroll
+  for (int r = 0; r < 2; ++r)
 #pragma unroll
     for (int ii = 0; ii < 4; ++ii)
-      S[r][ii] = a.h0 ? a.h0[((size_t)bh * DK + 16 * r + 4 * g + ii) * DV + mycol] : 0.f;
+      S[r][ii] = a.h0 ? a.h0[((size_t)bh * DK + 32 * w + 16 * r + 4 * g + ii) * DV + col0 + c] : 0.f;
 
-  for (int ch = 0; ch < a.NC; ++ch) {
-    const size_t m = (size_t)bh * a.NC + ch;
-    // ---- the chunk's images into LDS (128 threads, 16-byte copies) ----
-    for (int u = tid; u < C * DK / 4; u += 128) {
-      const int r = u / (DK / 4), q4 = u % (DK / 4);
-      *reinterpret_cast<floatx4*>(Ws + r * RP + 4 * q4) = *reinterpret_cast<const floatx4*>(a.W + (m * C + r) * DK + 4 * q4);
-      *reinterpret_cast<floatx4*>(Qs + r * RP + 4 * q4) = *reinterpret_cast<const floatx4*>(a.QE + (m * C + r) * DK + 4 * q4);
-      *reinterpret_cast<floatx4*>(Ks + r * RP + 4 * q4) = *reinterpret_cast<const floatx4*>(a.KR + (m * C + r) * DK + 4 * q4);
-    }
-    for (int u = tid; u < C * C / 4; u += 128) {
-      const int r = u / (C / 4), q4 = u % (C / 4);
-      *reinterpret_cast<floatx4*>(Ps + r * PP + 4 * q4) = *reinterpret_cast<const floatx4*>(a.P + (m * C + r) * C + 4 * q4);
-    }
-    for (int u = tid; u < C * 8; u += 128) {
-      const int r = u / 8, q4 = u % 8;
-      *reinterpret_cast<floatx4*>(Us + r * UP + 4 * q4) = *reinterpret_cast<const floatx4*>(a.U + (m * C + r) * DV + col0 + 4 * q4);
-    }
-    if (tid < DK / 4) *reinterpret_cast<floatx4*>(Ds + 4 * tid) = *reinterpret_cast<const floatx4*>(a.DEC + m * DK + 4 * tid);
-    lds_barrier();
+  load_slice(rw, a.W, 0);
+  load_slice(rq, a.QE, 0);
+  load_slice(rk, a.KR, 0);
+  load_u(0);
+  store_slice(Ws, rw);
+  store_slice(Qs, rq);
+  store_slice(Ks, rk);
+  store_u();
+  load_p(0);
+  load_d(0);
+  load_slice(rw, a.W, min(1, last));
+  load_slice(rq, a.QE, min(1, last));
+  load_slice(rk, a.KR, min(1, last));
+  load_u(min(1, last));
+  lds_barrier();
 
-    // ---- Y = W S, (QE S), v_new = U - Y (token tile ib: lane (c, g) rows 16 ib + 4g + ii) ----
-    floatx4 VN[C / 16], QS[C / 16];
+  // Past the end the loads repeat the last chunk and the copies write what no one reads again, so
+  // the loop is straight-line code and a copy waits only for its own loads.
+  for (int ch = 0; ch < NC; ++ch) {
+    const int nx1 = min(ch + 1, last), nx2 = min(ch + 2, last);
+    // ---- 1. partial products over this wave's 32 state rows ----
 #pragma unroll
-    for (int ib = 0; ib < C / 16; ++ib) {
-      floatx4 y = zero4(), qs = zero4();
+    for (int ib = 0; ib < 4; ++ib) {
+      floatx4 y = zero4(), qy = zero4();
 #pragma unroll
-      for (int r = 0; r < DK / 16; ++r) {
-        const floatx4 wa = *reinterpret_cast<const floatx4*>(Ws + (16 * ib + c) * RP + 16 * r + 4 * g);
-        const floatx4 qa = *reinterpret_cast<const floatx4*>(Qs + (16 * ib + c) * RP + 16 * r + 4 * g);
+      for (int r = 0; r < 2; ++r) {
+        const int off = (16 * ib + c) * RP + 32 * w + 16 * r + 4 * g;
+        const floatx4 wa = *reinterpret_cast<const floatx4*>(Ws + off);
+        const floatx4 qa = *reinterpret_cast<const floatx4*>(Qs + off);
 #pragma unroll
         for (int ii = 0; ii < 4; ++ii) {
           y = __builtin_amdgcn_mfma_f32_16x16x4f32(wa[ii], S[r][ii], y, 0, 0, 0);
-          qs = __builtin_amdgcn_mfma_f32_16x16x4f32(qa[ii], S[r][ii], qs, 0, 0, 0);
+          qy = __builtin_amdgcn_mfma_f32_16x16x4f32(qa[ii], S[r][ii], qy, 0, 0, 0);
         }
       }
-#pragma unroll
-      for (int ii = 0; ii < 4; ++ii) VN[ib][ii] = Us[(16 * ib + 4 * g + ii) * UP + 16 * w + c] - y[ii];
-      QS[ib] = qs;
+      YP[(w * 4 + ib) * 64 + lane] = y;
+      QP[(w * 4 + ib) * 64 + lane] = qy;
     }
-    // ---- o = QE S + P v_new (P lower triangular by 16-token blocks) -> HBM ----
+    store_slice(Ws, rw);                               // this wave's W and QE slices are read
+    store_slice(Qs, rq);
+    load_slice(rw, a.W, nx2);
+    load_slice(rq, a.QE, nx2);
+    lds_barrier();                                     // B1: partials written; P and VX read
+    store_p();
+    load_p(nx1);
+    // ---- 2a. v_new of token tile w; the QE S partials of o tile 3 - w ----
+    const int ot = 3 - w;
+    floatx4 O = QP[ot * 64 + lane];
 #pragma unroll
-    for (int ib = 0; ib < C / 16; ++ib) {
-      floatx4 o4 = QS[ib];
+    for (int w2 = 1; w2 < 4; ++w2) O += QP[(w2 * 4 + ot) * 64 + lane];
+    {
+      floatx4 Y = YP[w * 64 + lane];
 #pragma unroll
-      for (int jb = 0; jb <= ib; ++jb) {
-        const floatx4 pa = *reinterpret_cast<const floatx4*>(Ps + (16 * ib + c) * PP + 16 * jb + 4 * g);
+      for (int w2 = 1; w2 < 4; ++w2) Y += YP[(w2 * 4 + w) * 64 + lane];
+      floatx4 V;
 #pragma unroll
-        for (int ii = 0; ii < 4; ++ii) o4 = __builtin_amdgcn_mfma_f32_16x16x4f32(pa[ii], VN[jb][ii], o4, 0, 0, 0);
+      for (int ii = 0; ii < 4; ++ii) V[ii] = Us[(16 * w + 4 * g + ii) * UP + c] - Y[ii];
+      VX[w * 64 + lane] = V;
+    }
+    lds_barrier();                                     // B2: v_new and P written, U read
+    store_u();
+    load_u(nx2);
+    // ---- 2b. o of token tile 3 - w; the update of rows 32w .. ----
+    floatx4 VN[4];
+#pragma unroll
+    for (int ib = 0; ib < 4; ++ib) VN[ib] = VX[ib * 64 + lane];
+    {
+      floatx4 O2 = zero4();
+#pragma unroll
+      for (int jb = 0; jb < 4; ++jb) {
+        if (jb <= ot) {
+          const floatx4 pa = *reinterpret_cast<const floatx4*>(Ps + score_tile_index(ot, jb) * TT + c * TR + 4 * g);
+#pragma unroll
+          for (int ii = 0; ii < 4; ++ii) {
+            if (ii & 1) O2 = __builtin_amdgcn_mfma_f32_16x16x4f32(pa[ii], VN[jb][ii], O2, 0, 0, 0);
+            else O = __builtin_amdgcn_mfma_f32_16x16x4f32(pa[ii], VN[jb][ii], O, 0, 0, 0);
+          }
+        }
       }
+      O += O2;
 #pragma unroll
       for (int ii = 0; ii < 4; ++ii)
-        __builtin_nontemporal_store(o4[ii], a.o + ((size_t)bh * Tlen + (size_t)ch * C + 16 * ib + 4 * g + ii) * DV + mycol);
+        a.o[(t0 + (size_t)ch * C + 16 * ot + 4 * g + ii) * DV + col0 + c] = O[ii];
     }
-    // ---- S <- diag(e^{G_last}) S + KR^T v_new  (A operand lane (c, g): KR[t][16 r + c]) ----
 #pragma unroll
-    for (int r = 0; r < DK / 16; ++r) {
-      floatx4 acc;
+    for (int r = 0; r < 2; ++r) {
+      floatx4 acc, acc2 = zero4();                     // two accumulators: shorter chains
 #pragma unroll
-      for (int ii = 0; ii < 4; ++ii) acc[ii] = Ds[16 * r + 4 * g + ii] * S[r][ii];
+      for (int ii = 0; ii < 4; ++ii) acc[ii] = rd[r][ii] * S[r][ii];
 #pragma unroll
-      for (int jb = 0; jb < C / 16; ++jb)
+      for (int jb = 0; jb < 4; ++jb)
 #pragma unroll
-        for (int ii = 0; ii < 4; ++ii)
-          acc = __builtin_amdgcn_mfma_f32_16x16x4f32(Ks[(16 * jb + 4 * g + ii) * RP + 16 * r + c], VN[jb][ii], acc, 0, 0, 0);
-      S[r] = acc;
+        for (int ii = 0; ii < 4; ++ii) {
+          const float kx = Ks[(16 * jb + 4 * g + ii) * RP + 32 * w + 16 * r + c];
+          if (ii & 1) acc2 = __builtin_amdgcn_mfma_f32_16x16x4f32(kx, VN[jb][ii], acc2, 0, 0, 0);
+          else acc = __builtin_amdgcn_mfma_f32_16x16x4f32(kx, VN[jb][ii], acc, 0, 0, 0);
+        }
+      S[r] = acc + acc2;
     }
-    lds_barrier();                                     // the images are read: next chunk's copies
+    load_d(nx1);
+    store_slice(Ks, rk);                               // this wave's KR slice is read
+    load_slice(rk, a.KR, nx2);
+    // no third barrier: the next step 1 writes YP and QP (last read before B2), its B1 precedes the
+    // next writes of VX and P
   }
   if (a.h_final) {
 #pragma unroll
-    for (int r = 0; r < DK / 16; ++r)
+    for (int r = 0; r < 2; ++r)
 #pragma unroll
       for (int ii = 0; ii < 4; ++ii)
-        a.h_final[((size_t)bh * DK + 16 * r + 4 * g + ii) * DV + mycol] = S[r][ii];
+        a.h_final[((size_t)bh * DK + 32 * w + 16 * r + 4 * g + ii) * DV + col0 + c] = S[r][ii];
   }
 }
 
