@@ -9,11 +9,10 @@
 // with QE = scale q e^G, KR = k e^{G_last - G}, P = causal_incl(QE b^T).
 //
 // Stage 1 (kda_local_f32_kernel): one 256-thread workgroup per chunk; a, b and qe in LDS (fp32,
-// 132-float rows, so that the 16 rows of an MFMA operand read fall in 16 different bank groups),
+// 68-float rows, so that the 16 rows of an MFMA operand read fall in 16 different bank groups),
 // the 20 score blocks over the GDN chunk-local kernel's lists, the inverse in place, then W and U
-// with the T rows as the A operand.  Stage 2 (kda_scan_f32_kernel): one workgroup of two waves per
-// (chain, 32-column slice); each wave holds 16 state columns (fp32, MFMA D layout) through the
-// chain, and every chunk's W, QE, KR, P and U slice are copied into LDS before its products.
+// with the T rows as the A operand.  Stage 2 (kda_scan_f32_kernel): one workgroup of four waves per
+// (chain, 16-column slice), the products of every chunk split over the state rows.
 #pragma once
 
 #include <type_traits>
@@ -38,15 +37,20 @@ struct KdaLocalF32Args {
   float* DEC;           // [M, DK]     e^{G_last}
 };
 
+// The row tiles hold 64 of the 128 channels at a time (69.8 KB of LDS with A): two workgroups share a
+// CU, so that one's loads and stores run beside the other's products: 1024 chunks (287 MB) in 66 us,
+// 83 with full-width tiles and one workgroup per CU.
 template <int C, int DK>
-__global__ __launch_bounds__(256) void kda_local_f32_kernel(KdaLocalF32Args a) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void kda_local_f32_kernel(KdaLocalF32Args a) {
   static_assert(C == 64 && DK == 128, "the fp32 KDA kernels are written for C 64, dk = dv = 128");
-  constexpr int RP = DK + 4;           // fp32 row tiles
-  constexpr int CP = C + 4;            // A / T
+  constexpr int HD = DK / 2, RP = HD + 4;   // half-width row tiles
+  constexpr int CP = C + 4;                 // A / T
   constexpr int TILE = C * RP;
-  // LDS: a | b | qe row tiles, then A; the g staging [C][DK] aliases a and b until the gated
-  // operands are formed; after the scores T replaces A in place and the v tile takes b's rows.
-  static_assert(C * DK <= 2 * TILE, "g staging fits the a and b tiles");
+  // LDS: a | b | qe row tiles of one channel half, then A; the g staging [C][DK] aliases the tiles
+  // until the gated operands are formed; after the scores T replaces A in place and the tiles
+  // hold a (second half), a (first half) and v.
+  static_assert(C * DK <= 3 * TILE, "g staging fits the tiles");
   __shared__ __attribute__((aligned(16))) float tiles[3 * TILE];
   __shared__ __attribute__((aligned(16))) float As[C * CP];
   __shared__ __attribute__((aligned(16))) float Bs[C];
@@ -54,28 +58,26 @@ __global__ __launch_bounds__(256) void kda_local_f32_kernel(KdaLocalF32Args a) {
   float* bt = tiles + TILE;
   float* qt = tiles + 2 * TILE;
   float* gsm = tiles;
-  float* vt = bt;
 
   const int m = blockIdx.x;
   const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, c = lane & 15;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const size_t row0 = (size_t)m * C;
-  const int rb = tid >> 4, vc = (tid & 15) * 8;    // rows rb + 16 i, columns vc .. vc+7
+  const int rb = tid >> 4, vc = (tid & 15) * 4;    // rows rb + 16 i, columns 64 h + vc .. vc+3
 
   // ---- 1. loads; g to LDS ----------------------------------------------------------------
   floatx4 kr[4][2], qr[4][2], vr[4][2];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const size_t e = (row0 + rb + 16 * i) * DK + vc;
+  for (int i = 0; i < 4; ++i)
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      kr[i][h] = *reinterpret_cast<const floatx4*>(a.k + e + 4 * h);
-      qr[i][h] = *reinterpret_cast<const floatx4*>(a.q + e + 4 * h);
-      vr[i][h] = *reinterpret_cast<const floatx4*>(a.v + e + 4 * h);
-      *reinterpret_cast<floatx4*>(gsm + (rb + 16 * i) * DK + vc + 4 * h) =
-          *reinterpret_cast<const floatx4*>(a.g + e + 4 * h);
+      const size_t e = (row0 + rb + 16 * i) * DK + HD * h + vc;
+      kr[i][h] = *reinterpret_cast<const floatx4*>(a.k + e);
+      qr[i][h] = *reinterpret_cast<const floatx4*>(a.q + e);
+      vr[i][h] = *reinterpret_cast<const floatx4*>(a.v + e);
+      *reinterpret_cast<floatx4*>(gsm + (rb + 16 * i) * DK + HD * h + vc) =
+          *reinterpret_cast<const floatx4*>(a.g + e);
     }
-  }
   if (tid < C) Bs[tid] = a.beta[row0 + tid];
   lds_barrier();
 
@@ -93,59 +95,59 @@ __global__ __launch_bounds__(256) void kda_local_f32_kernel(KdaLocalF32Args a) {
   }
   lds_barrier();
 
-  // ---- 3. gated operands ------------------------------------------------------------------
-  float G[4][8], gl[8];
+  // ---- 3. the cumulative gates of this thread's elements ------------------------------------
+  floatx4 G[4][2], gl[2];
 #pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    const float half = gsm[(C / 2 - 1) * DK + vc + e];
-    gl[e] = gsm[(C - 1) * DK + vc + e] + half;         // G_last of column vc + e
+  for (int h = 0; h < 2; ++h) {
+    const floatx4 half = *reinterpret_cast<const floatx4*>(gsm + (C / 2 - 1) * DK + HD * h + vc);
+    gl[h] = *reinterpret_cast<const floatx4*>(gsm + (C - 1) * DK + HD * h + vc) + half;   // G_last
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      G[i][e] = gsm[(rb + 16 * i) * DK + vc + e] + ((rb + 16 * i) >= C / 2 ? half : 0.f);
+    for (int i = 0; i < 4; ++i) {
+      G[i][h] = *reinterpret_cast<const floatx4*>(gsm + (rb + 16 * i) * DK + HD * h + vc);
+      if (i >= 2) G[i][h] += half;
+    }
+    if (tid < 16)
+      *reinterpret_cast<floatx4*>(a.DEC + (size_t)m * DK + HD * h + vc) =
+          floatx4{__expf(gl[h][0]), __expf(gl[h][1]), __expf(gl[h][2]), __expf(gl[h][3])};
   }
-  lds_barrier();                                       // the g staging is overwritten below
-  if (tid < 16) {
+
+  // ---- 4. gated operands and scores, one channel half at a time: the GDN chunk-local kernel's block
+  //         lists (score_code with P): A = beta_i (a_i . b_j) strictly lower into As,
+  //         P = qe_i . b_j (lower, with its diagonal) to HBM
+  floatx4 a0[4];                                       // a of the first half, for W
+  constexpr int N = 5;
+  floatx4 acc[N];
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
-      *reinterpret_cast<floatx4*>(a.DEC + (size_t)m * DK + vc + 4 * h) =
-          floatx4{__expf(gl[4 * h]), __expf(gl[4 * h + 1]), __expf(gl[4 * h + 2]), __expf(gl[4 * h + 3])};
-  }
+  for (int b = 0; b < N; ++b) acc[b] = zero4();
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int r = rb + 16 * i;
+  for (int h = 0; h < 2; ++h) {
+    lds_barrier();                                     // the g staging / the first half is read
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
+    for (int i = 0; i < 4; ++i) {
+      const int r = rb + 16 * i;
       floatx4 av, bv, qv, rv;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const float gg = G[i][4 * h + e];
+        const float gg = G[i][h][e];
         const float eg = __expf(gg), ebg = __expf(-gg);
         av[e] = kr[i][h][e] * eg;
         bv[e] = kr[i][h][e] * ebg;
         qv[e] = a.scale * qr[i][h][e] * eg;
-        rv[e] = kr[i][h][e] * __expf(gl[4 * h + e] - gg);
+        rv[e] = kr[i][h][e] * __expf(gl[h][e] - gg);
       }
-      const size_t e0 = (row0 + r) * DK + vc + 4 * h;
+      const size_t e0 = (row0 + r) * DK + HD * h + vc;
       *reinterpret_cast<floatx4*>(a.QE + e0) = qv;
       *reinterpret_cast<floatx4*>(a.KR + e0) = rv;
-      *reinterpret_cast<floatx4*>(at + r * RP + vc + 4 * h) = av;
-      *reinterpret_cast<floatx4*>(bt + r * RP + vc + 4 * h) = bv;
-      *reinterpret_cast<floatx4*>(qt + r * RP + vc + 4 * h) = qv;
+      *reinterpret_cast<floatx4*>(at + r * RP + vc) = av;
+      *reinterpret_cast<floatx4*>(bt + r * RP + vc) = bv;
+      *reinterpret_cast<floatx4*>(qt + r * RP + vc) = qv;
+      if (h == 0) a0[i] = av;
     }
-  }
-  lds_barrier();
-
-  // ---- 4. scores: the GDN chunk-local kernel's block lists (score_code with P): A = beta_i
-  //         (a_i . b_j) strictly lower into As, P = qe_i . b_j (lower, with its diagonal) to HBM
-  {
-    constexpr int N = 5;
-    floatx4 acc[N];
-#pragma unroll
-    for (int b = 0; b < N; ++b) acc[b] = zero4();
+    lds_barrier();
     auto products = [&](auto wtag) {
       constexpr int WW = decltype(wtag)::value;
 #pragma unroll
-      for (int kb = 0; kb < DK / 16; ++kb) {
+      for (int kb = 0; kb < HD / 16; ++kb) {
 #pragma unroll
         for (int b = 0; b < N; ++b) {
           const int code = score_code(kScoreAP, WW, b);
@@ -161,62 +163,65 @@ __global__ __launch_bounds__(256) void kda_local_f32_kernel(KdaLocalF32Args a) {
       case 2: products(std::integral_constant<int, 2>{}); break;
       default: products(std::integral_constant<int, 3>{}); break;
     }
-    // each product is formed transposed: acc[ii] = (x_i . b_j), i = 16 bi + c, j = 16 bj + 4g + ii
+  }
+  // each product is formed transposed: acc[ii] = (x_i . b_j), i = 16 bi + c, j = 16 bj + 4g + ii
 #pragma unroll
-    for (int b = 0; b < N; ++b) {
-      const int code = score_code(kScoreAP, w, b);
-      const int i = 16 * ((code >> 2) & 3) + c, j0 = 16 * (code & 3) + 4 * g;
-      floatx4 out;
-      if (!(code & 16)) {
-        const float bi = Bs[i];
+  for (int b = 0; b < N; ++b) {
+    const int code = score_code(kScoreAP, w, b);
+    const int i = 16 * ((code >> 2) & 3) + c, j0 = 16 * (code & 3) + 4 * g;
+    floatx4 out;
+    if (!(code & 16)) {
+      const float bi = Bs[i];
 #pragma unroll
-        for (int ii = 0; ii < 4; ++ii) out[ii] = (i > j0 + ii) ? bi * acc[b][ii] : 0.f;
-        *reinterpret_cast<floatx4*>(As + i * CP + j0) = out;
-      } else {
+      for (int ii = 0; ii < 4; ++ii) out[ii] = (i > j0 + ii) ? bi * acc[b][ii] : 0.f;
+      *reinterpret_cast<floatx4*>(As + i * CP + j0) = out;
+    } else {
 #pragma unroll
-        for (int ii = 0; ii < 4; ++ii) out[ii] = (i >= j0 + ii) ? acc[b][ii] : 0.f;
-        *reinterpret_cast<floatx4*>(a.P + (size_t)m * C * C + i * C + j0) = out;
-      }
+      for (int ii = 0; ii < 4; ++ii) out[ii] = (i >= j0 + ii) ? acc[b][ii] : 0.f;
+      *reinterpret_cast<floatx4*>(a.P + (size_t)m * C * C + i * C + j0) = out;
     }
   }
   lds_barrier();
 
-  // ---- 5. T = (I + A)^-1 in place; the v tile into b's rows ---------------------------------
+  // ---- 5. a (first half) and v (first half) into the b and qe tiles; T = (I + A)^-1 in place -----
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    *reinterpret_cast<floatx4*>(bt + (rb + 16 * i) * RP + vc) = a0[i];
+    *reinterpret_cast<floatx4*>(qt + (rb + 16 * i) * RP + vc) = vr[i][0];
+  }
   unit_lower_inverse64(As, As);
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int h = 0; h < 2; ++h) *reinterpret_cast<floatx4*>(vt + (rb + 16 * i) * RP + vc + 4 * h) = vr[i][h];
-  lds_barrier();
 
-  // ---- 6. W = T diag(beta) a, U = T diag(beta) v: wave w owns column blocks 2w, 2w+1 ---------
-  //         (A operand = T rows, lane (c, g) T[16 ib + c][4 kk + g]; B = beta_j x[j][16 db + c])
+  // ---- 6. W = T diag(beta) a, U = T diag(beta) v: wave w owns column block w of each tile ---------
+  //         (A operand = T rows, lane (c, g) T[16 ib + c][4 kk + g]; B = beta_j x[j][16 w + c])
+  auto wy = [&](auto ntag, const float* const (&tile)[decltype(ntag)::value],
+                float* const (&dst)[decltype(ntag)::value]) {
+    constexpr int NT = decltype(ntag)::value;
 #pragma unroll
-  for (int ib = 0; ib < 4; ++ib) {
-    floatx4 accW[2], accU[2];
+    for (int ib = 0; ib < 4; ++ib) {
+      floatx4 d[NT];
 #pragma unroll
-    for (int d2 = 0; d2 < 2; ++d2) accW[d2] = accU[d2] = zero4();
-    for (int kk = 0; kk < 4 * ib + 4; ++kk) {        // T lower triangular: j <= 16 ib + 15
-      const int j = 4 * kk + g;
-      const float t = As[(16 * ib + c) * CP + j];
-      const float bj = Bs[j];
+      for (int t = 0; t < NT; ++t) d[t] = zero4();
+#pragma unroll 4
+      for (int kk = 0; kk < 4 * ib + 4; ++kk) {        // T lower triangular: j <= 16 ib + 15
+        const int j = 4 * kk + g;
+        const float tv = As[(16 * ib + c) * CP + j], bj = Bs[j];
 #pragma unroll
-      for (int d2 = 0; d2 < 2; ++d2) {
-        const int col = 16 * (2 * w + d2) + c;
-        accW[d2] = __builtin_amdgcn_mfma_f32_16x16x4f32(t, bj * at[j * RP + col], accW[d2], 0, 0, 0);
-        accU[d2] = __builtin_amdgcn_mfma_f32_16x16x4f32(t, bj * vt[j * RP + col], accU[d2], 0, 0, 0);
+        for (int t = 0; t < NT; ++t)
+          d[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(tv, bj * tile[t][j * RP + 16 * w + c], d[t], 0, 0, 0);
       }
+      // lane (c, g) holds D[4g + ii][c] of the tile: rows 16 ib + 4g + ii, column 16 w + c
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int ii = 0; ii < 4; ++ii) dst[t][(row0 + 16 * ib + 4 * g + ii) * DK + 16 * w + c] = d[t][ii];
     }
-    // lane (c, g) holds D[4g + ii][c] of the tile: rows 16 ib + 4g + ii, column 16 db + c
+  };
+  wy(std::integral_constant<int, 3>{}, {at, bt, qt}, {a.W + HD, a.W, a.U});
+  lds_barrier();
 #pragma unroll
-    for (int d2 = 0; d2 < 2; ++d2)
-#pragma unroll
-      for (int ii = 0; ii < 4; ++ii) {
-        const size_t e = ((size_t)m * C + 16 * ib + 4 * g + ii) * DK + 16 * (2 * w + d2) + c;
-        a.W[e] = accW[d2][ii];
-        a.U[e] = accU[d2][ii];
-      }
-  }
+  for (int i = 0; i < 4; ++i) *reinterpret_cast<floatx4*>(at + (rb + 16 * i) * RP + vc) = vr[i][1];
+  lds_barrier();
+  wy(std::integral_constant<int, 1>{}, {at}, {a.U + HD});
 }
 
 struct KdaScanF32Args {
@@ -244,7 +249,9 @@ struct KdaScanF32Args {
 // (64 + 4..16 + 32 products per wave and chunk).  Wave w reads only columns 32w .. 32w+31 of the W, QE
 // and KR rows, so it loads those slices itself and refills them after its own last read, with no
 // barrier; P is written between the barriers (its readers are past the first one), U after the
-// second.  Two barriers per chunk, the next chunk's loads in flight across both.
+// second.  Two barriers per chunk, the next chunk's loads in flight across both.  Bound by the chunk
+// step's chain, 3.6 us, of which the fp32 products take 1.4 (32 chains x 32 chunks: 115-123 us; 480
+// for the earlier two-wave form, which copied every image with the products waiting).
 template <int C, int DK, int DV>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
 void kda_scan_f32_kernel(KdaScanF32Args a) {
