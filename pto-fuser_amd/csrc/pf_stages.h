@@ -15,11 +15,22 @@
 // by one rule: chunk m = c*H + h, token i of it lives at row (c*C + i)*H + h.  H = 1 is the native
 // layout.  Gates follow the same rule with row length 1, scores with row length C.
 //
-// gfx950 mapping: 256-thread workgroups (4 waves) per chunk for the two score kernels, every
-// 16x16 output block one MFMA chain (bf16 16x16x32 or fp32 16x16x4).
+// gfx950 mapping.  256-thread workgroups (4 waves), one per chunk.  A wave owns whole 16-token query
+// blocks: their rows go straight from HBM into its registers as MFMA operands (no other wave reads
+// them); only the key side (and v) is staged in LDS, unpadded with XOR-permuted 16-byte slots.
+// Every score tile is formed transposed, P^T = k_jb q_ib^T, so a lane holds P[16 ib + c][16 jb + 4g ..
+// +3]: four consecutive columns of one row, which is a vector to store (gated_qk) and, two tiles
+// together, the B operand of o^T = v^T P^T as it stands (qkv_flash; v^T by transposed reads of the
+// row-major tile, fp32 by element reads): the score never passes through LDS.
+//
+// What bounds them: the memory system (1024 chunks of C = D = 128 bf16: qkv_flash 30-37 us for 168 MB,
+// 56-66 with the score and a transposed v staged in LDS by 2-byte writes; 2048 causal scores 37 us for
+// 203 MB, 76 with 2-byte stores), below ~500 chunks the call itself.
 #pragma once
 
-#include "pf_device.h"
+#include <type_traits>
+
+#include "pf_gfx950.h"
 
 // Barriers are LDS-only (lds_barrier): waves exchange data through LDS alone, so a barrier need
 // not wait for this wave's global stores to be acknowledged (a full __syncthreads would).
@@ -30,37 +41,53 @@ template <typename E> struct VecT;
 template <> struct VecT<bf16> { typedef bf16x8 T; };
 template <> struct VecT<float> { typedef floatx4 T; };
 
-// Copy a C x D tile (rows `row_stride` elements apart) into LDS with row pitch `pitch`,
-// multiplying element-wise by `scale` (same addressing, fp32) when it is given.
-template <typename E, int C, int D, int NTHR>
-__device__ __forceinline__ void stage_tile(const E* src, size_t row_stride, const float* scale,
-                                           E* dst, int pitch) {
-  constexpr int VE = Vec16<E>::N, PER_ROW = D / VE;
+// 16 bytes of operand rows at element offset `off`, times `scale` (fp32, same addressing) if given.
+template <typename E>
+__device__ __forceinline__ typename VecT<E>::T load_scaled(const E* src, const float* scale, size_t off) {
   typedef typename VecT<E>::T V;
-  for (int u = threadIdx.x; u < C * PER_ROW; u += NTHR) {
-    const int i = u / PER_ROW, d0 = (u % PER_ROW) * VE;
-    V x = __builtin_bit_cast(V, *reinterpret_cast<const uint4*>(src + i * row_stride + d0));
-    if (scale) {
-      const float* s = scale + i * row_stride + d0;
+  V x = *reinterpret_cast<const V*>(src + off);
+  if (scale) {
 #pragma unroll
-      for (int e = 0; e < VE; ++e) x[e] = from_f32<E>(to_f32(x[e]) * s[e]);
-    }
-    *reinterpret_cast<V*>(dst + i * pitch + d0) = x;
+    for (int e = 0; e < Vec16<E>::N; ++e) x[e] = from_f32<E>(to_f32(x[e]) * scale[off + e]);
   }
+  return x;
 }
 
-__device__ __forceinline__ void store_out(void* base, size_t idx, float v, int out_f32) {
-  if (out_f32) static_cast<float*>(base)[idx] = v;
-  else static_cast<bf16*>(base)[idx] = (bf16)v;
+// Physical slot of 16-byte slot `s` of row `row`: a key tile read one row per lane c, and a v tile
+// read transposed (4 rows x 2 slots per lane group) or, fp32, as 4 rows x 16 floats.
+template <typename E, int D>
+__device__ __forceinline__ int key_slot(int row, int s) {
+  return sizeof(E) == 2 && D == 64 ? s ^ ((row >> 1) & 7) : s ^ (row & 15);
+}
+template <typename E, int D>
+__device__ __forceinline__ int val_slot(int row, int s) {
+  if (sizeof(E) == 4) return s ^ (((row >> 2) & 3) << 2);
+  return D == 64 ? s ^ (row & 2) : s ^ ((row & 3) << 1);
 }
 
-// Lower-triangular block (bi >= bj) number x of an NB x NB block grid, row-major over the
-// triangle: 0 -> (0,0), 1 -> (1,0), 2 -> (1,1), 3 -> (2,0) ...
-__device__ __forceinline__ void tri_block(int x, int& bi, int& bj) {
-  bi = 0;
-  while (x > bi) { x -= bi + 1; ++bi; }
-  bj = x;
+// The four-column score tile of query block rows `q` (one row per lane c, K-blocks in `q`) against key
+// block jb of the staged tile.
+template <typename E, int D>
+__device__ __forceinline__ floatx4 score_tile(const E* ks, int jb, const typename VecT<E>::T* q, int c, int g) {
+  floatx4 acc = zero4();
+  const E* row = ks + (16 * jb + c) * D;
+#pragma unroll
+  for (int kb = 0; kb < D / Mfma<E>::KB; ++kb) {
+    const auto k = *reinterpret_cast<const typename VecT<E>::T*>(row + Vec16<E>::N * key_slot<E, D>(c, 4 * kb + g));
+    if constexpr (sizeof(E) == 2) {
+      acc = mfma_bf16(k, q[kb], acc);
+    } else {
+#pragma unroll
+      for (int ii = 0; ii < 4; ++ii) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(k[ii], q[kb][ii], acc, 0, 0, 0);
+    }
+  }
+  return acc;
 }
+
+// Query block s (0 or 1) of wave w: the last blocks, with most key blocks behind them, go to the
+// waves with the first ones.
+template <int NB>
+__device__ __forceinline__ int query_block(int s, int w) { return s == 0 ? w : NB - 1 - w; }
 
 struct GatedQkArgs {
   const void* a;        // rows of a  (E)
@@ -78,39 +105,87 @@ struct GatedQkArgs {
 
 template <typename E, int C, int D>
 __global__ __launch_bounds__(256) void gated_qk_kernel(GatedQkArgs p) {
-  constexpr int PE = 16 / sizeof(E), KP = D + PE, NB = C / 16;
-  __shared__ __attribute__((aligned(16))) E sa[C * KP];
-  __shared__ __attribute__((aligned(16))) E sb[C * KP];
-  __shared__ float Gs[C], Ls[C];
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, g = lane >> 4, c = lane & 15;
+  typedef typename VecT<E>::T V;
+  constexpr int VE = Vec16<E>::N, SLOTS = D / VE, NB = C / 16, NKB = D / Mfma<E>::KB;
+  constexpr int NBW = (NB + 3) / 4, NV = (C * SLOTS + 255) / 256;
+  __shared__ __attribute__((aligned(16))) E sb[C * D];
+  __shared__ __attribute__((aligned(16))) float Gs[C], Ls[C];
+  const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, c = lane & 15;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int m = blockIdx.x, ch = m / p.H, h = m % p.H;
   const size_t rs = (size_t)p.H * D, base = ((size_t)ch * C * p.H + h) * D;
-  stage_tile<E, C, D, 256>(static_cast<const E*>(p.a) + base, rs, p.a_scale ? p.a_scale + base : nullptr, sa, KP);
-  stage_tile<E, C, D, 256>(static_cast<const E*>(p.b) + base, rs, p.b_scale ? p.b_scale + base : nullptr, sb, KP);
+  const E* ag = static_cast<const E*>(p.a) + base;
+  const E* bg = static_cast<const E*>(p.b) + base;
+  const float* as = p.a_scale ? p.a_scale + base : nullptr;
+  const float* bs = p.b_scale ? p.b_scale + base : nullptr;
+
+  V br[NV], q[NBW][NKB];
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const int u = tid + 256 * i;
+    if (C * SLOTS >= 256 * (i + 1) || u < C * SLOTS)
+      br[i] = load_scaled(bg, bs, (u / SLOTS) * rs + (u % SLOTS) * VE);
+  }
+#pragma unroll
+  for (int s = 0; s < NBW; ++s)
+    if (w < NB)
+#pragma unroll
+      for (int kb = 0; kb < NKB; ++kb)
+        q[s][kb] = load_scaled(ag, as, (16 * query_block<NB>(s, w) + c) * rs + Mfma<E>::KB * kb + VE * g);
   if (tid < C) {
     const size_t gi = ((size_t)ch * C + tid) * p.H + h;
     Gs[tid] = p.g ? p.g[gi] : 0.f;
     Ls[tid] = p.beta ? __logf(p.beta[gi]) : 0.f;
   }
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const int u = tid + 256 * i, row = u / SLOTS;
+    if (C * SLOTS >= 256 * (i + 1) || u < C * SLOTS)
+      *reinterpret_cast<V*>(sb + row * D + VE * key_slot<E, D>(row, u % SLOTS)) = br[i];
+  }
   lds_barrier();
+  if (w >= NB) return;
   const size_t lrs = (size_t)p.H * C, lbase = ((size_t)ch * C * p.H + h) * C;
-  for (int x = w; x < NB * NB; x += 4) {
-    const int bi = x / NB, bj = x % NB, j = 16 * bj + c;
-    if (bj > bi && !p.mask) {            // strictly-upper blocks of a triangular mask are zero
 #pragma unroll
-      for (int ii = 0; ii < 4; ++ii) store_out(p.L, lbase + (16 * bi + 4 * g + ii) * lrs + j, 0.f, p.out_f32);
-      continue;
-    }
-    floatx4 acc = zero4();
+  for (int s = 0; s < NBW; ++s) {
+    const int ib = query_block<NB>(s, w), i = 16 * ib + c;
+    const float gi = Gs[i] + Ls[i];
+    auto tile = [&](int jb) -> floatx4 {   // strictly-upper tiles of a triangular mask are zero
+      if (jb > ib && !p.mask) return zero4();
+      const floatx4 acc = score_tile<E, D>(sb, jb, q[s], c, g);
+      const int j0 = 16 * jb + 4 * g;
+      const floatx4 gj = *reinterpret_cast<const floatx4*>(Gs + j0);
+      floatx4 out;
 #pragma unroll
-    for (int kb = 0; kb < D / Mfma<E>::KB; ++kb)
-      acc = Mfma<E>::rows(acc, sa + (16 * bi + c) * KP, sb + (16 * bj + c) * KP, kb, g);
+      for (int ii = 0; ii < 4; ++ii) {
+        const float mk = p.mask ? p.mask[i * C + j0 + ii] : ((p.causal ? i >= j0 + ii : i > j0 + ii) ? 1.f : 0.f);
+        out[ii] = mk == 0.f ? 0.f : acc[ii] * __expf(fminf(gi - gj[ii], 0.f)) * mk;
+      }
+      return out;
+    };
+    const size_t row = lbase + i * lrs;
+    if (p.out_f32) {
 #pragma unroll
-    for (int ii = 0; ii < 4; ++ii) {
-      const int i = 16 * bi + 4 * g + ii;
-      const float mk = p.mask ? p.mask[i * C + j] : ((p.causal ? i >= j : i > j) ? 1.f : 0.f);
-      const float coef = __expf(fminf(Gs[i] + Ls[i] - Gs[j], 0.f));
-      store_out(p.L, lbase + i * lrs + j, mk == 0.f ? 0.f : acc[ii] * coef * mk, p.out_f32);
+      for (int jb = 0; jb < NB; ++jb)
+        *reinterpret_cast<floatx4*>(static_cast<float*>(p.L) + row + 16 * jb + 4 * g) = tile(jb);
+    } else {
+      bf16* L = static_cast<bf16*>(p.L) + row;
+#pragma unroll
+      for (int jp = 0; jp < NB / 2; ++jp) {
+        // lane groups 2x and 2x+1 exchange halves of two tiles: each lane then holds eight consecutive
+        // columns, groups 0 and 2 of tile 2 jp and 1 and 3 of tile 2 jp + 1
+        const floatx4 t0 = tile(2 * jp), t1 = tile(2 * jp + 1);
+        typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+        const u32x2 x = __builtin_bit_cast(u32x2, bf16x4{(bf16)t0[0], (bf16)t0[1], (bf16)t0[2], (bf16)t0[3]});
+        const u32x2 y = __builtin_bit_cast(u32x2, bf16x4{(bf16)t1[0], (bf16)t1[1], (bf16)t1[2], (bf16)t1[3]});
+        const u32x2 e0 = __builtin_amdgcn_permlane16_swap(x[0], y[0], false, false);
+        const u32x2 e1 = __builtin_amdgcn_permlane16_swap(x[1], y[1], false, false);
+        *reinterpret_cast<u32x4*>(L + 32 * jp + 16 * (g & 1) + 8 * (g >> 1)) = u32x4{e0[0], e1[0], e0[1], e1[1]};
+      }
+      if constexpr (NB == 1) {
+        const floatx4 t0 = tile(0);
+        store4(L + 4 * g, t0[0], t0[1], t0[2], t0[3]);
+      }
     }
   }
 }
@@ -126,80 +201,118 @@ struct QkvFlashArgs {
   float* o;             // [M, C, D] fp32
 };
 
-template <int A, int B> struct MaxI { static constexpr int v = A > B ? A : B; };
-
 template <typename E, int C, int D>
-__global__ __launch_bounds__(256) void qkv_flash_kernel(QkvFlashArgs p) {
-  constexpr int PE = 16 / sizeof(E), KP = D + PE, LP = C + PE, VP = C + PE, VE = Vec16<E>::N;
-  constexpr int NB = C / 16, NL = NB * (NB + 1) / 2, NPW = (NL + 3) / 4;
-  // phase 1: rx = q tile, ry = k tile;  phase 2: rx = score (operand type), ry = v^T
-  __shared__ __attribute__((aligned(16))) E rx[MaxI<C * KP, C * LP>::v];
-  __shared__ __attribute__((aligned(16))) E ry[MaxI<C * KP, D * VP>::v];
-  __shared__ float Gs[C], Ls[C];
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, g = lane >> 4, c = lane & 15;
-  const size_t m = blockIdx.x, row0 = m * C;
-  stage_tile<E, C, D, 256>(static_cast<const E*>(p.q) + row0 * D, D, p.q_scale ? p.q_scale + row0 * D : nullptr, rx, KP);
-  stage_tile<E, C, D, 256>(static_cast<const E*>(p.k) + row0 * D, D, p.k_scale ? p.k_scale + row0 * D : nullptr, ry, KP);
+__global__ __launch_bounds__(256)
+__attribute__((amdgpu_waves_per_eu(C * D * sizeof(E) > 32 * 1024 ? 1 : 2, 8)))
+void qkv_flash_kernel(QkvFlashArgs p) {
+  typedef typename VecT<E>::T V;
+  constexpr bool B16 = sizeof(E) == 2;
+  constexpr int VE = Vec16<E>::N, SLOTS = D / VE, NB = C / 16, NKB = D / Mfma<E>::KB;
+  constexpr int NBW = (NB + 3) / 4, NV = (C * SLOTS + 255) / 256;
+  __shared__ __attribute__((aligned(16))) E sk[C * D];
+  __shared__ __attribute__((aligned(16))) E sv[C * D];
+  __shared__ __attribute__((aligned(16))) float Gs[C], Ls[C];
+  const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, c = lane & 15;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const size_t row0 = (size_t)blockIdx.x * C;
+  const E* qg = static_cast<const E*>(p.q) + row0 * D;
+  const E* kg = static_cast<const E*>(p.k) + row0 * D;
+  const E* vg = static_cast<const E*>(p.v) + row0 * D;
+  const float* qsc = p.q_scale ? p.q_scale + row0 * D : nullptr;
+  const float* ksc = p.k_scale ? p.k_scale + row0 * D : nullptr;
+
+  // every load is issued before the first LDS store; v's stay in flight while the score is formed
+  V kr[NV], vr[NV], q[NBW][NKB];
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const int u = tid + 256 * i;
+    if (C * SLOTS >= 256 * (i + 1) || u < C * SLOTS) kr[i] = load_scaled(kg, ksc, (size_t)u * VE);
+  }
+#pragma unroll
+  for (int s = 0; s < NBW; ++s)
+    if (w < NB)
+#pragma unroll
+      for (int kb = 0; kb < NKB; ++kb)
+        q[s][kb] = load_scaled(qg, qsc, (size_t)(16 * query_block<NB>(s, w) + c) * D + Mfma<E>::KB * kb + VE * g);
   if (tid < C) {
     Gs[tid] = p.g ? p.g[row0 + tid] : 0.f;
     Ls[tid] = p.beta ? __logf(p.beta[row0 + tid]) : 0.f;
   }
-  lds_barrier();
-  floatx4 acc[NPW];
 #pragma unroll
-  for (int s = 0; s < NPW; ++s) {
-    acc[s] = zero4();
-    const int x = w + 4 * s;
-    if (x < NL) {
-      int bi, bj;
-      tri_block(x, bi, bj);
+  for (int i = 0; i < NV; ++i) {
+    const int u = tid + 256 * i;
+    if (C * SLOTS >= 256 * (i + 1) || u < C * SLOTS) vr[i] = *reinterpret_cast<const V*>(vg + (size_t)u * VE);
+  }
 #pragma unroll
-      for (int kb = 0; kb < D / Mfma<E>::KB; ++kb)
-        acc[s] = Mfma<E>::rows(acc[s], rx + (16 * bi + c) * KP, ry + (16 * bj + c) * KP, kb, g);
-    }
+  for (int i = 0; i < NV; ++i) {
+    const int u = tid + 256 * i, row = u / SLOTS;
+    if (C * SLOTS >= 256 * (i + 1) || u < C * SLOTS)
+      *reinterpret_cast<V*>(sk + row * D + VE * key_slot<E, D>(row, u % SLOTS)) = kr[i];
   }
   lds_barrier();
+
+  // the score rows of this wave's query blocks, in the operand type
+  constexpr int NP = B16 ? (NB + 1) / 2 : NB;
+  typedef typename std::conditional<B16, bf16x8, floatx4>::type PV;
+  PV P[NBW][NP];
 #pragma unroll
-  for (int s = 0; s < NPW; ++s) {
-    const int x = w + 4 * s;
-    if (x < NL) {
-      int bi, bj;
-      tri_block(x, bi, bj);
-      const int j = 16 * bj + c;
+  for (int s = 0; s < NBW; ++s) {
+    const int ib = query_block<NB>(s, w), i = 16 * ib + c;
+    if (w < NB) {
+      const float gi = Gs[i] + Ls[i];
+      auto tile = [&](int jb) -> floatx4 {
+        if (jb > ib) return zero4();
+        const floatx4 acc = score_tile<E, D>(sk, jb, q[s], c, g);
+        const floatx4 gj = *reinterpret_cast<const floatx4*>(Gs + 16 * jb + 4 * g);
+        floatx4 out;
 #pragma unroll
-      for (int ii = 0; ii < 4; ++ii) {
-        const int i = 16 * bi + 4 * g + ii;
-        const float coef = __expf(fminf(Gs[i] + Ls[i] - Gs[j], 0.f));
-        rx[i * LP + j] = from_f32<E>(i >= j ? acc[s][ii] * coef : 0.f);
+        for (int ii = 0; ii < 4; ++ii)
+          out[ii] = i >= 16 * jb + 4 * g + ii ? acc[ii] * __expf(fminf(gi - gj[ii], 0.f)) : 0.f;
+        return out;
+      };
+#pragma unroll
+      for (int x = 0; x < NP; ++x) {
+        if constexpr (B16) P[s][x] = pack8(tile(2 * x), tile(2 * x + 1));
+        else P[s][x] = tile(x);
       }
     }
   }
-  for (int e = tid; e < C * C; e += 256) {
-    const int i = e / C, j = e % C;
-    if ((j >> 4) > (i >> 4)) rx[i * LP + j] = from_f32<E>(0.f);
-  }
-  {
-    typedef typename VecT<E>::T V;
-    const E* vg = static_cast<const E*>(p.v) + row0 * D;
-    for (int u = tid; u < C * (D / VE); u += 256) {
-      const int t = u / (D / VE), n0 = (u % (D / VE)) * VE;
-      const V x = __builtin_bit_cast(V, *reinterpret_cast<const uint4*>(vg + (size_t)t * D + n0));
 #pragma unroll
-      for (int e = 0; e < VE; ++e) ry[(n0 + e) * VP + t] = x[e];
-    }
+  for (int i = 0; i < NV; ++i) {
+    const int u = tid + 256 * i, row = u / SLOTS;
+    if (C * SLOTS >= 256 * (i + 1) || u < C * SLOTS)
+      *reinterpret_cast<V*>(sv + row * D + VE * val_slot<E, D>(row, u % SLOTS)) = vr[i];
   }
   lds_barrier();
-  // o[t, n] = sum_{t' <= t} S[t, t'] v[t', n]: (C/16) x (D/16) blocks over the four waves
-  float* o = p.o + row0 * D;
-  for (int x = w; x < NB * (D / 16); x += 4) {
-    const int bi = x / (D / 16), bn = x % (D / 16);
-    floatx4 r = zero4();
+  if (w >= NB) return;
+  // o^T tiles: lane (c, g) gets o[16 ib + c][16 r + 4g .. +3]
 #pragma unroll
-    for (int kb = 0; kb < C / Mfma<E>::KB; ++kb)
-      if (kb * Mfma<E>::KB <= 16 * bi + 15)
-        r = Mfma<E>::rows(r, rx + (16 * bi + c) * LP, ry + (16 * bn + c) * VP, kb, g);
+  for (int s = 0; s < NBW; ++s) {
+    const int ib = query_block<NB>(s, w);
+    float* o = p.o + (row0 + 16 * ib + c) * D + 4 * g;
 #pragma unroll
-    for (int ii = 0; ii < 4; ++ii) o[(size_t)(16 * bi + 4 * g + ii) * D + 16 * bn + c] = r[ii];
+    for (int r = 0; r < D / 16; ++r) {
+      floatx4 acc = zero4();
+#pragma unroll
+      for (int x = 0; x < NP; ++x) {
+        if constexpr (B16) {
+          if (2 * x <= ib) {
+            const int row = 32 * x + 4 * g + (c >> 2);
+            const int off = VE * val_slot<E, D>(c >> 2, 2 * r + ((c & 3) >> 1)) + 4 * (c & 1);
+            acc = mfma_bf16(cat8(lds_read_tr(sv + row * D + off), lds_read_tr(sv + (row + 16) * D + off)), P[s][x], acc);
+          }
+        } else {
+          if (x <= ib) {
+#pragma unroll
+            for (int ii = 0; ii < 4; ++ii) {
+              const float vx = sv[(16 * x + 4 * g + ii) * D + 4 * val_slot<E, D>(4 * g, 4 * r + (c >> 2)) + (c & 3)];
+              acc = __builtin_amdgcn_mfma_f32_16x16x4f32(vx, P[s][x][ii], acc, 0, 0, 0);
+            }
+          }
+        }
+      }
+      *reinterpret_cast<floatx4*>(o + 16 * r) = acc;
+    }
   }
 }
 
