@@ -41,16 +41,17 @@ template <typename E> struct VecT;
 template <> struct VecT<bf16> { typedef bf16x8 T; };
 template <> struct VecT<float> { typedef floatx4 T; };
 
-// 16 bytes of operand rows at element offset `off`, times `scale` (fp32, same addressing) if given.
+// 16 bytes of operand rows at element offset `off`, and the same times their prescales (fp32, same
+// addressing).  Callers load every vector first and prescale in one uniform branch: a branch per
+// vector would make each load wait for the one before.
 template <typename E>
-__device__ __forceinline__ typename VecT<E>::T load_scaled(const E* src, const float* scale, size_t off) {
-  typedef typename VecT<E>::T V;
-  V x = *reinterpret_cast<const V*>(src + off);
-  if (scale) {
+__device__ __forceinline__ typename VecT<E>::T load_vec(const E* src, size_t off) {
+  return *reinterpret_cast<const typename VecT<E>::T*>(src + off);
+}
+template <typename E>
+__device__ __forceinline__ void prescale(typename VecT<E>::T& x, const float* scale, size_t off) {
 #pragma unroll
-    for (int e = 0; e < Vec16<E>::N; ++e) x[e] = from_f32<E>(to_f32(x[e]) * scale[off + e]);
-  }
-  return x;
+  for (int e = 0; e < Vec16<E>::N; ++e) x[e] = from_f32<E>(to_f32(x[e]) * scale[off + e]);
 }
 
 // Physical slot of 16-byte slot `s` of row `row`: a key tile read one row per lane c, and a v tile
@@ -99,11 +100,11 @@ struct GatedQkArgs {
   const float* mask;    // [C, C] multiplier, or null (use `causal`)
   void* L;              // scores, row length C, fp32 or bf16
   int H;                // heads interleaved in the row index (1 = native [M, C, D])
-  int causal;           // without mask: 1 keeps i >= j, 0 keeps i > j
+  int causal;           // without mask: 1 keeps i >= j, 0 keeps i > j (0 or 1)
   int out_f32;          // 1: L is fp32, 0: bf16
 };
 
-template <typename E, int C, int D>
+template <typename E, int C, int D, bool MASK>
 __global__ __launch_bounds__(256) void gated_qk_kernel(GatedQkArgs p) {
   typedef typename VecT<E>::T V;
   constexpr int VE = Vec16<E>::N, SLOTS = D / VE, NB = C / 16, NKB = D / Mfma<E>::KB;
@@ -120,18 +121,29 @@ __global__ __launch_bounds__(256) void gated_qk_kernel(GatedQkArgs p) {
   const float* bs = p.b_scale ? p.b_scale + base : nullptr;
 
   V br[NV], q[NBW][NKB];
+  auto b_off = [&](int i) {
+    const int u = tid + 256 * i;                       // vectors past the tile repeat its last one
+    return (min(u, C * SLOTS - 1) / SLOTS) * rs + (u % SLOTS) * VE;
+  };
+  auto a_off = [&](int s, int kb) {
+    return (16 * (query_block<NB>(s, w) & (NB - 1)) + c) * rs + Mfma<E>::KB * kb + VE * g;
+  };
 #pragma unroll
-  for (int i = 0; i < NV; ++i) {
-    const int u = tid + 256 * i;
-    if (C * SLOTS >= 256 * (i + 1) || u < C * SLOTS)
-      br[i] = load_scaled(bg, bs, (u / SLOTS) * rs + (u % SLOTS) * VE);
-  }
+  for (int i = 0; i < NV; ++i) br[i] = load_vec(bg, b_off(i));
 #pragma unroll
   for (int s = 0; s < NBW; ++s)
-    if (w < NB)
 #pragma unroll
-      for (int kb = 0; kb < NKB; ++kb)
-        q[s][kb] = load_scaled(ag, as, (16 * query_block<NB>(s, w) + c) * rs + Mfma<E>::KB * kb + VE * g);
+    for (int kb = 0; kb < NKB; ++kb) q[s][kb] = load_vec(ag, a_off(s, kb));
+  if (bs) {
+#pragma unroll
+    for (int i = 0; i < NV; ++i) prescale<E>(br[i], bs, b_off(i));
+  }
+  if (as) {
+#pragma unroll
+    for (int s = 0; s < NBW; ++s)
+#pragma unroll
+      for (int kb = 0; kb < NKB; ++kb) prescale<E>(q[s][kb], as, a_off(s, kb));
+  }
   if (tid < C) {
     const size_t gi = ((size_t)ch * C + tid) * p.H + h;
     Gs[tid] = p.g ? p.g[gi] : 0.f;
@@ -151,14 +163,14 @@ __global__ __launch_bounds__(256) void gated_qk_kernel(GatedQkArgs p) {
     const int ib = query_block<NB>(s, w), i = 16 * ib + c;
     const float gi = Gs[i] + Ls[i];
     auto tile = [&](int jb) -> floatx4 {   // strictly-upper tiles of a triangular mask are zero
-      if (jb > ib && !p.mask) return zero4();
+      if (!MASK && jb > ib) return zero4();
       const floatx4 acc = score_tile<E, D>(sb, jb, q[s], c, g);
       const int j0 = 16 * jb + 4 * g;
       const floatx4 gj = *reinterpret_cast<const floatx4*>(Gs + j0);
       floatx4 out;
 #pragma unroll
       for (int ii = 0; ii < 4; ++ii) {
-        const float mk = p.mask ? p.mask[i * C + j0 + ii] : ((p.causal ? i >= j0 + ii : i > j0 + ii) ? 1.f : 0.f);
+        const float mk = MASK ? p.mask[i * C + j0 + ii] : (i + p.causal > j0 + ii ? 1.f : 0.f);
         out[ii] = mk == 0.f ? 0.f : acc[ii] * __expf(fminf(gi - gj[ii], 0.f)) * mk;
       }
       return out;
@@ -223,25 +235,31 @@ void qkv_flash_kernel(QkvFlashArgs p) {
 
   // every load is issued before the first LDS store; v's stay in flight while the score is formed
   V kr[NV], vr[NV], q[NBW][NKB];
+  auto off = [&](int i) { return (size_t)min(tid + 256 * i, C * SLOTS - 1) * VE; };
+  auto q_off = [&](int s, int kb) {
+    return (size_t)(16 * (query_block<NB>(s, w) & (NB - 1)) + c) * D + Mfma<E>::KB * kb + VE * g;
+  };
 #pragma unroll
-  for (int i = 0; i < NV; ++i) {
-    const int u = tid + 256 * i;
-    if (C * SLOTS >= 256 * (i + 1) || u < C * SLOTS) kr[i] = load_scaled(kg, ksc, (size_t)u * VE);
-  }
+  for (int i = 0; i < NV; ++i) kr[i] = load_vec(kg, off(i));
 #pragma unroll
   for (int s = 0; s < NBW; ++s)
-    if (w < NB)
 #pragma unroll
-      for (int kb = 0; kb < NKB; ++kb)
-        q[s][kb] = load_scaled(qg, qsc, (size_t)(16 * query_block<NB>(s, w) + c) * D + Mfma<E>::KB * kb + VE * g);
+    for (int kb = 0; kb < NKB; ++kb) q[s][kb] = load_vec(qg, q_off(s, kb));
   if (tid < C) {
     Gs[tid] = p.g ? p.g[row0 + tid] : 0.f;
     Ls[tid] = p.beta ? __logf(p.beta[row0 + tid]) : 0.f;
   }
 #pragma unroll
-  for (int i = 0; i < NV; ++i) {
-    const int u = tid + 256 * i;
-    if (C * SLOTS >= 256 * (i + 1) || u < C * SLOTS) vr[i] = *reinterpret_cast<const V*>(vg + (size_t)u * VE);
+  for (int i = 0; i < NV; ++i) vr[i] = load_vec(vg, off(i));
+  if (ksc) {
+#pragma unroll
+    for (int i = 0; i < NV; ++i) prescale<E>(kr[i], ksc, off(i));
+  }
+  if (qsc) {
+#pragma unroll
+    for (int s = 0; s < NBW; ++s)
+#pragma unroll
+      for (int kb = 0; kb < NKB; ++kb) prescale<E>(q[s][kb], qsc, q_off(s, kb));
   }
 #pragma unroll
   for (int i = 0; i < NV; ++i) {

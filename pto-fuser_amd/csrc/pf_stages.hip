@@ -48,7 +48,8 @@ struct GatedQkLaunch {
   template <typename E, int C, int D>
   int operator()() {
     pf::LaunchScope scope;
-    pf::gated_qk_kernel<E, C, D><<<dim3(grid), dim3(256), 0, s>>>(a);
+    if (a.mask) pf::gated_qk_kernel<E, C, D, true><<<dim3(grid), dim3(256), 0, s>>>(a);
+    else pf::gated_qk_kernel<E, C, D, false><<<dim3(grid), dim3(256), 0, s>>>(a);
     return scope.status();
   }
 };

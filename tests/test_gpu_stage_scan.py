@@ -21,11 +21,12 @@ SHAPES = [(32, 64, 2, 3, 3), (64, 64, 1, 8, 2), (128, 64, 1, 1, 1), (32, 128, 1,
           (128, 128, 2, 64, 2)]                                                # 64-column slices
 
 
-@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("C,D,B,H,nc", SHAPES + [(16, 64, 1, 3, 3), (16, 128, 2, 65, 2)])
+CASES = [(torch.float32, *x) for x in SHAPES + [(16, 64, 1, 3, 3), (16, 128, 2, 65, 2)]] + \
+        [(torch.bfloat16, *x) for x in SHAPES]           # bf16 stages take C >= 32
+
+
+@pytest.mark.parametrize("dtype,C,D,B,H,nc", CASES)
 def test_chunk_scan_dispatch_edges(dtype, C, D, B, H, nc):
-    if dtype == torch.bfloat16 and C < 32:
-        pytest.skip("bf16 stages take C >= 32")
     perdim, out16, with_h0 = (B + H + nc) % 2 == 0, H % 2 == 1, nc != 2
     announce(f"chunk_scan C={C} D={D} B={B} H={H} nc={nc} {dtype} perdim={perdim} out16={out16}")
     rng = np.random.default_rng(C + D + B * H + nc)
