@@ -59,6 +59,9 @@ const char* pf_source_hash(void);
  *   32-bit; a longer sequence is PF_ERR_ARG).  The kernels run 64-token chunks; C = 128
  *   (the reference's chunk) is served by them over T / 64 chunks — the chunked forward's result
  *   does not depend on the chunk size, only the blocking of its arithmetic does.
+ *   bf16 operands, few long chains: a chain runs as segments side by side, joined through their
+ *   state maps, when the workspace holds those (pf_gdn_workspace_bytes and pf_gdn_setup include them);
+ *   on a smaller workspace the same call runs whole chains.
  * ------------------------------------------------------------------------------------------ */
 size_t pf_gdn_workspace_bytes(int B, int H, int T, int C, int DK, int DV, int dtype);
 void* pf_gdn_setup(int B, int H, int T, int C, int DK, int DV, int dtype);
@@ -68,7 +71,7 @@ void* pf_gdn_setup(int B, int H, int T, int C, int DK, int DV, int dtype);
  * for an unsupported shape, PF_ERR_ALLOC).  A reserve that does not grow allocates nothing and is
  * safe under HIP graph capture; one that grows waits for the device and must run outside it.
  * Growing frees the old buffer: a HIP graph captured on the handle before a growth still
- * addresses it and must be captured again.  The fp32 layout of a shape holds its bf16 layout, so
+ * addresses it and must be captured again.  The fp32 size of a shape covers its bf16 size, so
  * a handle reserved for the fp32 size serves both dtypes of that shape without growing.
  * pf_gdn_setup(shape) == pf_gdn_create() + pf_gdn_reserve(shape); pf_gdn_teardown frees either. */
 void* pf_gdn_create(void);

@@ -30,20 +30,72 @@ size_t elem_size(int dtype) { return dtype == PF_DTYPE_BF16 ? 2 : 4; }
 
 bool valid_dtype(int dtype) { return dtype == PF_DTYPE_F32 || dtype == PF_DTYPE_BF16; }
 
-// Byte layout of the fused-forward workspace:
-//   [ T (M*C*C E) | P (M*C*C E, pre-scaled; fp32 only) | G (M*C fp32) | output scale (fp32, 256 B) ].
+// How a chain of NC chunks is run: `seg` segments of `len` chunks (the last may have fewer).
+struct Segments {
+  int seg, len;
+};
+
+int generations(long wgs) { return (int)((wgs + pf::device_cu_count() - 1) / pf::device_cu_count()); }
+
+// Column slices of the bf16 scan: 16 columns (a chunk step of 1.2 us) while eight slices per unit fit
+// one generation of workgroups, else 32 (1.45 us, half the workgroups).
+bool narrow_slices(long units) { return units * 8 <= pf::device_cu_count(); }
+double scan_us(long units, int chunks) {
+  return narrow_slices(units) ? 1.2 * chunks : 1.45 * chunks * generations(units * 4);
+}
+
+// Segments of a bf16 chain.  A chain's time is its chunk count while chains leave CUs idle; in
+// segments it is the segment's length twice (its map, 2.5 us per chunk step on one workgroup per CU,
+// and the scan) plus a composition step of 1.9 us per segment, and 9 us for the two more launches.  The
+// times are per generation of workgroups, as measured; segments are taken where they come out 10 %
+// ahead.  Measured, whole forward, one chain against its segments: 4 chains x 512 chunks 577 -> 157 us,
+// 8 x 256 300 -> 132, 16 x 128 160 -> 119, 8 x 64 82 -> 59, 1 x 128 147 -> 68, 2 x 32 44 -> 42; not taken:
+// 32 x 128 (173, 190 in segments), 15 x 23 (37, 53), 32 x 512 (666, 693).
+Segments gdn_segments(int BH, int NC, int dtype) {
+  Segments best{1, NC};
+  if (dtype != PF_DTYPE_BF16 || NC < 16) return best;
+  double t = 0.9 * scan_us(BH, NC);
+  for (int want = 4; want <= 64 && want * 4 <= NC; want += want < 8 ? 2 : want / 4) {
+    const int len = (NC + want - 1) / want, seg = (NC + len - 1) / len;
+    const double x = 9.0 + 2.5 * len * generations((long)BH * (2 * seg - 3)) + 1.9 * (seg - 2) +
+                     scan_us((long)BH * seg, len);
+    if (x < t) {
+      t = x;
+      best = {seg, len};
+    }
+  }
+  return best;
+}
+
+// Byte layout of the fused-forward workspace, M = BH * NC chunks:
+//   [ T (M*C*C E) | P (M*C*C E, pre-scaled; fp32 only) | G (M*C fp32) | output scale (fp32, 256 B) |
+//     D, Mx (BH*(seg-1)*128*128 fp32 each; segmented chains only) ].
 // The bf16 scan forms P from the q and k rows it stages, so the bf16 layout has no P.
 struct GdnLayout {
-  size_t t_off, p_off, g_off, s_off, total;
-  GdnLayout(size_t M, int C, int dtype) {
+  size_t t_off, p_off, g_off, s_off, d_off, m_off, base, total;
+  GdnLayout(int BH, int NC, int dtype, Segments sg) {
+    constexpr size_t C = 64, DD = 128 * 128;
+    const size_t M = (size_t)BH * NC;
     const size_t cc = M * C * C * elem_size(dtype);
     t_off = 0;
     p_off = align256(cc);
     g_off = p_off + (dtype == PF_DTYPE_BF16 ? 0 : align256(cc));
     s_off = g_off + align256(M * C * sizeof(float));
-    total = s_off + 256;
+    base = s_off + 256;                       // all an unsegmented run needs
+    d_off = base;
+    m_off = d_off + (size_t)BH * (sg.seg - 1) * DD * sizeof(float);
+    total = m_off + (size_t)BH * (sg.seg - 1) * DD * sizeof(float);
   }
 };
+
+// The workspace a shape asks for.  The fp32 size is at least the bf16 one, so that a handle reserved
+// for fp32 serves both types of a shape without growing.
+size_t gdn_workspace_total(int BH, int NC, int dtype) {
+  const size_t b16 = GdnLayout(BH, NC, PF_DTYPE_BF16, gdn_segments(BH, NC, PF_DTYPE_BF16)).total;
+  if (dtype == PF_DTYPE_BF16) return b16;
+  const size_t f32 = GdnLayout(BH, NC, PF_DTYPE_F32, {1, NC}).total;
+  return f32 > b16 ? f32 : b16;
+}
 
 // The kernels' chunk: every forward runs 64-token chunks.  A caller's chunk size of 128 (the
 // reference's) is served by the same kernels over T / 64 chunks: the chunked forward's result does
@@ -59,9 +111,10 @@ bool gdn_shape_ok(int B, int H, int T, int C, int DK, int DV, int dtype) {
 
 template <typename E>
 void chunk_local_launch(const void* q, const void* k, const float* beta, const float* g,
-                       float scale, char* base, size_t M, hipStream_t stream) {
+                       float scale, char* base, int BH, int NC, hipStream_t stream) {
   constexpr int C = 64, DK = 128;
-  const GdnLayout lay(M, C, std::is_same<E, bf16>::value ? PF_DTYPE_BF16 : PF_DTYPE_F32);
+  const size_t M = (size_t)BH * NC;
+  const GdnLayout lay(BH, NC, std::is_same<E, bf16>::value ? PF_DTYPE_BF16 : PF_DTYPE_F32, {1, NC});
   pf::ChunkLocalArgs a{};
   a.k = k;
   a.q = q;
@@ -90,10 +143,12 @@ void chunk_local_launch(const void* q, const void* k, const float* beta, const f
 template <typename E>
 void scan_output_launch(const void* q, const void* k, const void* v, const float* beta,
                        const float* h0, float* o, float* h_final, int BH, int NC,
-                       char* base, hipStream_t stream) {
+                       char* base, size_t bytes, hipStream_t stream) {
   constexpr int C = 64, DK = 128, DV = 128;
-  const size_t M = (size_t)BH * NC;
-  const GdnLayout lay(M, C, std::is_same<E, bf16>::value ? PF_DTYPE_BF16 : PF_DTYPE_F32);
+  constexpr int dtype = std::is_same<E, bf16>::value ? PF_DTYPE_BF16 : PF_DTYPE_F32;
+  Segments sg = gdn_segments(BH, NC, dtype);
+  if (GdnLayout(BH, NC, dtype, sg).total > bytes) sg = {1, NC};   // a smaller buffer: whole chains
+  const GdnLayout lay(BH, NC, dtype, sg);
   pf::ScanOutArgs a{};
   a.q = q;
   a.k = k;
@@ -108,16 +163,35 @@ void scan_output_launch(const void* q, const void* k, const void* v, const float
   a.BH = BH;
   a.NC = NC;
   a.scale = reinterpret_cast<const float*>(base + lay.s_off);
+  a.hseg = reinterpret_cast<const float*>(base + lay.d_off);
+  a.SEG = sg.seg;
+  a.L = sg.len;
   if constexpr (std::is_same<E, bf16>::value) {
-    // bf16: one workgroup per (chain, 32-column slice), or 16-column slices when 32 would leave
-    // CUs idle (fewer than 8 chains per 32 CUs: long sequences at small batch); four MFMA waves
-    // split every chunk (pf_scan_split.h)
-    if ((size_t)BH * (DV / 32) < (size_t)pf::device_cu_count())
+    if (sg.seg > 1) {
+      pf::SegMapArgs m{};
+      m.k = static_cast<const bf16*>(k);
+      m.v = static_cast<const bf16*>(v);
+      m.beta = beta;
+      m.G = a.G;
+      m.Tm = static_cast<const bf16*>(a.Tm);
+      m.h0 = h0;
+      m.D = reinterpret_cast<float*>(base + lay.d_off);
+      m.M = reinterpret_cast<float*>(base + lay.m_off);
+      m.BH = BH;
+      m.NC = NC;
+      m.SEG = sg.seg;
+      m.L = sg.len;
+      pf::seg_states_launch(m, stream);
+    }
+    const int units = BH * sg.seg;
+    // bf16: one workgroup per (segment or whole chain, 32- or 16-column slice); four MFMA waves split
+    // every chunk (pf_scan_split.h)
+    if (narrow_slices(units))
       pf::scan_split_kernel<C, DK, DV, 1, kSplit16LoaderWaves>
-          <<<dim3((unsigned)(BH * (DV / 16))), dim3(64 * (4 + kSplit16LoaderWaves)), 0, stream>>>(a);
+          <<<dim3((unsigned)(units * (DV / 16))), dim3(64 * (4 + kSplit16LoaderWaves)), 0, stream>>>(a);
     else
       pf::scan_split_kernel<C, DK, DV, 2, kSplitLoaderWaves>
-          <<<dim3((unsigned)(BH * (DV / 32))), dim3(64 * (4 + kSplitLoaderWaves)), 0, stream>>>(a);
+          <<<dim3((unsigned)(units * (DV / 32))), dim3(64 * (4 + kSplitLoaderWaves)), 0, stream>>>(a);
   } else {
     // fp32: one workgroup per (chain, 16-column slice), every chunk split over four waves
     // (pf_scan_split_f32.h)
@@ -126,17 +200,17 @@ void scan_output_launch(const void* q, const void* k, const void* v, const float
 }
 
 // Both stages of the forward on the workspace at `base` (the layout of GdnLayout).
-int gdn_forward_on(char* base, const void* q, const void* k, const void* v, const float* beta,
+int gdn_forward_on(char* base, size_t bytes, const void* q, const void* k, const void* v, const float* beta,
                    const float* g, const float* h0, float* o, float* h_final, int B, int H, int T,
                    int C, int dtype, float scale, hipStream_t s) {
-  const size_t M = (size_t)B * H * (T / kChunk);
+  const int BH = B * H, NC = T / kChunk;
   pf::LaunchScope scope;
   if (dtype == PF_DTYPE_BF16) {
-    chunk_local_launch<bf16>(q, k, beta, g, scale, base, M, s);
-    scan_output_launch<bf16>(q, k, v, beta, h0, o, h_final, B * H, T / kChunk, base, s);
+    chunk_local_launch<bf16>(q, k, beta, g, scale, base, BH, NC, s);
+    scan_output_launch<bf16>(q, k, v, beta, h0, o, h_final, BH, NC, base, bytes, s);
   } else {
-    chunk_local_launch<float>(q, k, beta, g, scale, base, M, s);
-    scan_output_launch<float>(q, k, v, beta, h0, o, h_final, B * H, T / kChunk, base, s);
+    chunk_local_launch<float>(q, k, beta, g, scale, base, BH, NC, s);
+    scan_output_launch<float>(q, k, v, beta, h0, o, h_final, BH, NC, base, bytes, s);
   }
   return scope.status();
 }
@@ -145,7 +219,7 @@ int gdn_forward_on(char* base, const void* q, const void* k, const void* v, cons
 int gdn_check(int B, int H, int T, int C, int DK, int DV, int dtype, const void* ws) {
   if (!gdn_shape_ok(B, H, T, C, DK, DV, dtype)) return PF_ERR_ARG;
   const GdnWorkspace* w = static_cast<const GdnWorkspace*>(ws);
-  if (!w || !w->base || w->bytes < GdnLayout((size_t)B * H * (T / kChunk), kChunk, dtype).total)
+  if (!w || !w->base || w->bytes < GdnLayout(B * H, T / kChunk, dtype, {1, T / kChunk}).base)
     return PF_ERR_WORKSPACE;
   return PF_OK;
 }
@@ -210,7 +284,7 @@ const char* pf_source_hash(void) { return PF_SOURCE_HASH; }
 
 size_t pf_gdn_workspace_bytes(int B, int H, int T, int C, int DK, int DV, int dtype) {
   if (!gdn_shape_ok(B, H, T, C, DK, DV, dtype)) return 0;
-  return GdnLayout((size_t)B * H * (T / kChunk), kChunk, dtype).total;
+  return gdn_workspace_total(B * H, T / kChunk, dtype);
 }
 
 void* pf_gdn_create(void) { return pf::workspace_create(); }
@@ -240,13 +314,13 @@ int pf_gdn_chunk_local_exec(const void* q, const void* k, const float* beta, con
   if (st != PF_OK) return st;
   if (!q || !k || !beta) return PF_ERR_ARG;
   const GdnWorkspace* w = static_cast<const GdnWorkspace*>(ws);
-  const size_t M = (size_t)B * H * (T / kChunk);
+  const int BH = B * H, NC = T / kChunk;
   hipStream_t s = static_cast<hipStream_t>(stream);
   pf::LaunchScope scope;
   if (dtype == PF_DTYPE_BF16)
-    chunk_local_launch<bf16>(q, k, beta, g, scale, static_cast<char*>(w->base), M, s);
+    chunk_local_launch<bf16>(q, k, beta, g, scale, static_cast<char*>(w->base), BH, NC, s);
   else
-    chunk_local_launch<float>(q, k, beta, g, scale, static_cast<char*>(w->base), M, s);
+    chunk_local_launch<float>(q, k, beta, g, scale, static_cast<char*>(w->base), BH, NC, s);
   return scope.status();
 }
 
@@ -261,10 +335,10 @@ int pf_gdn_scan_output_exec(const void* q, const void* k, const void* v, const f
   pf::LaunchScope scope;
   if (dtype == PF_DTYPE_BF16)
     scan_output_launch<bf16>(q, k, v, beta, h0, o, h_final, B * H, T / kChunk,
-                             static_cast<char*>(w->base), s);
+                             static_cast<char*>(w->base), w->bytes, s);
   else
     scan_output_launch<float>(q, k, v, beta, h0, o, h_final, B * H, T / kChunk,
-                              static_cast<char*>(w->base), s);
+                              static_cast<char*>(w->base), w->bytes, s);
   return scope.status();
 }
 
@@ -274,8 +348,8 @@ int pf_gdn_exec(const void* q, const void* k, const void* v, const float* beta, 
   const int st = gdn_check(B, H, T, C, DK, DV, dtype, ws);
   if (st != PF_OK) return st;
   if (!q || !k || !v || !beta || !o) return PF_ERR_ARG;
-  return gdn_forward_on(static_cast<char*>(static_cast<GdnWorkspace*>(ws)->base), q, k, v, beta,
-                        g, h0, o, h_final, B, H, T, C, dtype, scale,
+  const GdnWorkspace* w = static_cast<const GdnWorkspace*>(ws);
+  return gdn_forward_on(static_cast<char*>(w->base), w->bytes, q, k, v, beta, g, h0, o, h_final, B, H, T, C, dtype, scale,
                         static_cast<hipStream_t>(stream));
 }
 
@@ -283,13 +357,13 @@ int pf_gdn_exec_static(const void* q, const void* k, const void* v, const float*
                        const float* g, const float* h0, float* o, float* h_final, int B, int H,
                        int T, int C, int DK, int DV, int dtype, float scale, void* stream) {
   if (!gdn_shape_ok(B, H, T, C, DK, DV, dtype)) return PF_ERR_ARG;
-  if (GdnLayout((size_t)B * H * (T / kChunk), kChunk, dtype).total > kStaticScratchBytes)
+  if (GdnLayout(B * H, T / kChunk, dtype, {1, T / kChunk}).base > kStaticScratchBytes)
     return PF_ERR_SCRATCH;
   if (!q || !k || !v || !beta || !o) return PF_ERR_ARG;
   int st = PF_OK;
   void* base = scratch_on_current_device(&st);
   if (!base) return st;
-  return gdn_forward_on(static_cast<char*>(base), q, k, v, beta, g, h0, o, h_final, B, H, T, C,
+  return gdn_forward_on(static_cast<char*>(base), kStaticScratchBytes, q, k, v, beta, g, h0, o, h_final, B, H, T, C,
                         dtype, scale, static_cast<hipStream_t>(stream));
 }
 

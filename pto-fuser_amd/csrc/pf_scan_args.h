@@ -20,6 +20,25 @@ struct ScanOutArgs {
   int BH;
   int NC;               // chunks per chain
   const float* scale;   // device scalar: the output scale (written by stage 1)
+  // segmented chains (bf16): each chain runs as SEG segments of L chunks (the last may have fewer),
+  // segment s > 0 from the state hseg[bh][s - 1]; SEG = 1, L = NC otherwise
+  const float* hseg;    // [BH, SEG - 1, DK, DV]
+  int SEG, L;
 };
+
+// Arguments of the segmented chains' first two steps (pf_seg_scan.h) and their launch (pf_seg.hip).
+struct SegMapArgs {
+  const bf16* k;        // [BH*T, DK]
+  const bf16* v;        // [BH*T, DV]
+  const float* beta;    // [BH*T]
+  const float* G;       // [BH*T] within-chunk cumsum of the log decay, from stage 1
+  const bf16* Tm;       // [M, C, C] (I + A)^-1, from stage 1
+  const float* h0;      // [BH, DK, DV] or null
+  float* D;             // [BH, SEG - 1, DK, DV]
+  float* M;             // [BH, SEG - 1, DK, DK]   (segment 0's is not written)
+  int BH, NC;           // chains, chunks per chain
+  int SEG, L;           // segments per chain, chunks per segment (the last may have fewer)
+};
+void seg_states_launch(const SegMapArgs& m, hipStream_t stream);
 
 }  // namespace pf

@@ -1,0 +1,16 @@
+// Launches of the segmented-chain kernels (pf_seg_scan.h), in a source of their own: they are compiled
+// with the default machine scheduler.
+#include <hip/hip_runtime.h>
+
+#include "pf_seg_scan.h"
+
+namespace pf {
+
+void seg_states_launch(const SegMapArgs& m, hipStream_t stream) {
+  const unsigned units = (unsigned)(m.BH * (m.SEG - 1));
+  seg_map_kernel<64, 128, 128><<<dim3((units + 7) / 8 * 16), dim3(512), 0, stream>>>(m);
+  if (m.SEG > 2)
+    seg_compose_kernel<128, 128><<<dim3((unsigned)((m.BH + 7) / 8 * 64)), dim3(256), 0, stream>>>(m.D, m.M, m.BH, m.SEG);
+}
+
+}  // namespace pf

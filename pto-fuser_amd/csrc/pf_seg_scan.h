@@ -1,0 +1,297 @@
+// Segmented chains (bf16 operands, few long chains): what turns one chain of NC sequential chunks into
+// SEG segments that run side by side.
+//
+// Over a segment of chunks the delta rule is affine in its incoming state, H_out = M H_in + D, so
+//
+//   1. seg_map_kernel     for every segment but the last, D (128 columns, from a zero state; the first
+//                         segment from h0, which makes its D the true state) and M (the state
+//                         recurrence without v, from the identity; not needed for the first);
+//   2. seg_compose_kernel H_{s+1} = D_s + M_s H_s along each chain, fp32 products, in place of D_s;
+//   3. the scan (pf_scan_split.h) over all segments at once, each from its own H_s.
+//
+// Step 1 repeats the state part of the chunk loop on 256 columns instead of 128, so segments pay
+// where chains leave the chip idle or their length is the bound, not where every CU is busy
+// (gdn_segments in pf_abi.hip has the rule and its measurements).
+//
+// seg_map_kernel: state columns are independent, so a wave owns 16 of them for the whole segment and
+// every product feeds the next from registers: S (packed pairs of D tiles) is the B operand of k S,
+// r = beta v - beta e^G (k S) that of T r, v_new e^{G_last - G} that of the update
+// S <- e^{G_last} S + k^T (.).  The eight waves of a workgroup (D or M of one segment) share only
+// the chunk's k, T, v and gate images in LDS (two), loaded into registers three chunks ahead.  Tile pair (2x, 2x + 1) holds rows (state
+// rows or tokens) 32x + 8g + 0..7 per lane group, so k and T rows are read as natural-order 16-byte
+// fragments and k^T by transposed reads of the same image.  fp32 state and accumulators, bf16
+// operands, as in the scan itself.
+#pragma once
+
+#include "pf_gfx950.h"
+#include "pf_scan_args.h"
+
+namespace pf {
+
+// Row of tile t (a pair's half t & 1) held in register ii of lane group g, and the row lane c supplies
+// as the A operand of that tile.
+__device__ __forceinline__ constexpr int seg_row(int t, int g, int ii) { return 32 * (t >> 1) + 8 * g + 4 * (t & 1) + ii; }
+
+// Physical 16-byte slot of slot `s` of row `row`: k (16 slots a row; read as 16 rows x one slot and,
+// transposed, as 4 rows x 4 slots) and T (8 slots a row; 16 rows x one slot).
+__device__ __forceinline__ int seg_k_slot(int row, int s) { return s ^ (((row & 3) << 2) | ((row >> 3) & 3)); }
+__device__ __forceinline__ int seg_t_slot(int row, int s) { return s ^ ((((row >> 1) & 1) << 2) | ((row >> 3) & 3)); }
+
+// M is kept in the operand order of seg_compose_kernel: 16x16 tiles, each 64 lanes x four consecutive
+// columns, so that its loads are contiguous (row-major, 64-byte pieces of 16 rows, a step took 2.6 us).
+__device__ __forceinline__ constexpr int seg_m_index(int row, int col) {
+  return (((row >> 4) * 8 + (col >> 4)) * 64 + ((col >> 2) & 3) * 16 + (row & 15)) * 4 + (col & 3);
+}
+
+struct SegImage {                                      // one chunk in LDS
+  bf16 ks[64 * 128], ts[64 * 64], vs[8 * 64 * 16];     // v: per wave [64][16]
+  struct {
+    float BT[64], BEG[64], EL[64];                     // beta, beta e^G, e^{G_last - G}
+  } gate[8];                                           // per wave: no branch around the tables
+};
+
+// D (MAP false) or M (MAP true) of segment `seg` of chain bh.  MAP is a template parameter so that the
+// chunk is straight-line code (a uniform branch around v splits it, and every LDS read is then waited
+// for where it is issued).
+template <int C, int DK, int DV, bool MAP>
+__device__ __forceinline__ void seg_map_run(const SegMapArgs& a, SegImage (&img)[2], int bh, int seg) {
+  const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, c = lane & 15;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int col = 16 * w + c;
+  const size_t m0 = (size_t)bh * a.NC + (size_t)seg * a.L, t0 = m0 * C;
+  const bf16* kg = a.k + t0 * DK;
+  const bf16* vg = a.v + t0 * DV;
+  const bf16* tg = a.Tm + m0 * C * C;
+  const float* Gg = a.G + t0;
+  const float* Bg = a.beta + t0;
+
+  // one chunk in registers: 16-byte vectors u = tid + 512 i of k and v (16 a row), tid of T (8 a row)
+  struct Regs {
+    u32x4 k[2], t, v[2];
+    float g, b;
+  };
+  auto load = [&](Regs& x, int ch) {
+    ch = min(ch, a.L - 1);                             // past the end: the last chunk again, unused
+#pragma unroll
+    for (int i = 0; i < 2; ++i) x.k[i] = *reinterpret_cast<const u32x4*>(kg + (size_t)ch * C * DK + (tid + 512 * i) * 8);
+    x.t = *reinterpret_cast<const u32x4*>(tg + (size_t)ch * C * C + tid * 8);
+    if constexpr (!MAP) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) x.v[i] = *reinterpret_cast<const u32x4*>(vg + (size_t)ch * C * DV + (tid + 512 * i) * 8);
+    }
+    x.g = Gg[(size_t)ch * C + lane];
+    x.b = Bg[(size_t)ch * C + lane];
+  };
+  auto store = [&](SegImage& im, const Regs& x) -> float {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int u = tid + 512 * i, row = u >> 4, s = u & 15;
+      *reinterpret_cast<u32x4*>(im.ks + row * DK + 8 * seg_k_slot(row, s)) = x.k[i];
+      if constexpr (!MAP) *reinterpret_cast<u32x4*>(im.vs + (s >> 1) * C * 16 + row * 16 + 8 * (s & 1)) = x.v[i];
+    }
+    *reinterpret_cast<u32x4*>(im.ts + (tid >> 3) * C + 8 * seg_t_slot(tid >> 3, tid & 7)) = x.t;
+    const float gl = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x.g), C - 1));
+    im.gate[w].BT[lane] = x.b;                         // lane = token
+    im.gate[w].BEG[lane] = x.b * __expf(x.g);
+    im.gate[w].EL[lane] = __expf(gl - x.g);
+    return __expf(gl);                                 // the chunk's decay
+  };
+
+  floatx4 S[8];
+#pragma unroll
+  for (int r = 0; r < 8; ++r)
+#pragma unroll
+    for (int ii = 0; ii < 4; ++ii) S[r][ii] = MAP && seg_row(r, g, ii) == col ? 1.f : 0.f;
+  if (!MAP && seg == 0 && a.h0) {                      // one branch around all loads
+    const float* h = a.h0 + (size_t)bh * DK * DV + col;
+#pragma unroll
+    for (int r = 0; r < 8; ++r)
+#pragma unroll
+      for (int ii = 0; ii < 4; ++ii) S[r][ii] = h[seg_row(r, g, ii) * DV];
+  }
+
+  const int crow = 8 * (c >> 2) + (c & 3);             // + 32x + 4h: the row lane c supplies
+  const int trow = 8 * g + (c >> 2);                   // transposed reads: + 32x + 4h
+  // chunk m in register set m % 3 until it is written to LDS, three chunks of lead
+  Regs r0, r1, r2;
+  load(r0, 0);
+  load(r1, 1);
+  load(r2, 2);
+  float dl = store(img[0], r0), dl_next = 0.f;
+  load(r0, 3);
+  lds_barrier();
+  auto chunk = [&](Regs& nx, int ch) {                 // nx holds chunk ch + 1
+    const SegImage& im = img[ch & 1];
+    const bf16 *ks = im.ks, *ts = im.ts, *vs = im.vs;
+    bf16x8 Sb[4];
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb) Sb[kb] = pack8(S[2 * kb], S[2 * kb + 1]);
+    // r = beta v - beta e^G (k S)
+    bf16x8 Rb[2];
+#pragma unroll
+    for (int x = 0; x < 2; ++x) {
+      floatx4 r[2];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        floatx4 Y = zero4();
+        const int row = 32 * x + 4 * h + crow;
+#pragma unroll
+        for (int kb = 0; kb < 4; ++kb)
+          Y = mfma_bf16(*reinterpret_cast<const bf16x8*>(ks + row * DK + 8 * seg_k_slot(row, 4 * kb + g)), Sb[kb], Y);
+        const int t4 = 32 * x + 8 * g + 4 * h;
+        const floatx4 beg = *reinterpret_cast<const floatx4*>(im.gate[w].BEG + t4);
+        if constexpr (MAP) {
+#pragma unroll
+          for (int ii = 0; ii < 4; ++ii) r[h][ii] = -beg[ii] * Y[ii];
+        } else {
+          const floatx4 bt = *reinterpret_cast<const floatx4*>(im.gate[w].BT + t4);
+          const bf16x4 v4 = lds_read_tr(vs + w * C * 16 + (32 * x + 4 * h + trow) * 16 + 4 * (c & 3));
+#pragma unroll
+          for (int ii = 0; ii < 4; ++ii) r[h][ii] = fmaf(-beg[ii], Y[ii], bt[ii] * (float)v4[ii]);
+        }
+      }
+      Rb[x] = pack8(r[0], r[1]);
+    }
+    dl_next = store(img[(ch + 1) & 1], nx);                      // last read a barrier ago
+    load(nx, ch + 4);
+    // v_new = T r (T lower triangular by 32-token blocks), scaled by e^{G_last - G}
+    bf16x8 Vb[2];
+#pragma unroll
+    for (int x = 0; x < 2; ++x) {
+      floatx4 V[2];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        V[h] = zero4();
+        const int row = 32 * x + 4 * h + crow;
+#pragma unroll
+        for (int xb = 0; xb <= x; ++xb)
+          V[h] = mfma_bf16(*reinterpret_cast<const bf16x8*>(ts + row * C + 8 * seg_t_slot(row, 4 * xb + g)), Rb[xb], V[h]);
+        V[h] *= *reinterpret_cast<const floatx4*>(im.gate[w].EL + 32 * x + 8 * g + 4 * h);
+      }
+      Vb[x] = pack8(V[0], V[1]);
+    }
+    // S <- e^{G_last} S + k^T (.)
+#pragma unroll
+    for (int r = 0; r < 8; ++r) {
+      floatx4 acc = S[r] * dl;
+#pragma unroll
+      for (int x = 0; x < 2; ++x) {
+        const int r0 = 32 * x + trow, off = 8 * seg_k_slot(trow, 4 * (r >> 1) + (c & 3)) + 4 * (r & 1);
+        // rows r0 and r0 + 4 share their slot permutation (row bits 0, 1, 3, 4)
+        acc = mfma_bf16(cat8(lds_read_tr(ks + r0 * DK + off), lds_read_tr(ks + (r0 + 4) * DK + off)), Vb[x], acc);
+      }
+      S[r] = acc;
+    }
+    dl = dl_next;
+    lds_barrier();                                     // the next image written, this one read
+  };
+  int ch = 0;
+  for (; ch + 2 < a.L; ch += 3) {
+    chunk(r1, ch);
+    chunk(r2, ch + 1);
+    chunk(r0, ch + 2);
+  }
+  if (ch < a.L) chunk(r1, ch);
+  if (ch + 1 < a.L) chunk(r2, ch + 1);
+  float* out = (MAP ? a.M : a.D) + ((size_t)bh * (a.SEG - 1) + seg) * DK * DV;
+#pragma unroll
+  for (int r = 0; r < 8; ++r)
+#pragma unroll
+    for (int ii = 0; ii < 4; ++ii) {
+      const int row = seg_row(r, g, ii);
+      out[MAP ? seg_m_index(row, col) : row * DV + col] = S[r][ii];
+    }
+}
+
+template <int C, int DK, int DV>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void seg_map_kernel(SegMapArgs a) {
+  static_assert(C == 64 && DK == 128 && DV == 128, "the forward's tile: C 64, dk = dv = 128");
+  __shared__ __attribute__((aligned(16))) SegImage img[2];
+  // the workgroups of D and M of one segment on one XCD: they read the same k and T
+  const int units = a.BH * (a.SEG - 1), bid = blockIdx.x;
+  const int unit = (bid / 16) * 8 + bid % 8;
+  const bool map = bid % 16 >= 8;
+  if (unit >= units) return;
+  const int bh = unit / (a.SEG - 1), seg = unit % (a.SEG - 1);
+  if (!map) seg_map_run<C, DK, DV, false>(a, img, bh, seg);
+  else if (seg > 0) seg_map_run<C, DK, DV, true>(a, img, bh, seg);
+}
+
+// H_{s+1} = D_s + M_s H_s for s = 1 .. SEG - 2 (H_1 = D_0 is final), written over D_s.  One workgroup per
+// (chain, 16 columns); wave w forms rows 32w .. 32w+31 with fp32 products (two 16-row tiles, the
+// four-element K order of the D layout), its rows of M_s loaded a step ahead; H_s passes through LDS as
+// D tiles.
+template <int DK, int DV>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
+void seg_compose_kernel(float* D, const float* M, int BH, int SEG) {
+  constexpr int NS = DV / 16;
+  __shared__ __attribute__((aligned(16))) floatx4 H[2][8 * 64];
+  // the slices of one chain on one XCD: they read the same M
+  const int bh = (blockIdx.x / (8 * NS)) * 8 + blockIdx.x % 8, col0 = 16 * (blockIdx.x % (8 * NS) / 8);
+  if (bh >= BH) return;
+  const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, c = lane & 15;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  float* Dc = D + (size_t)bh * (SEG - 1) * DK * DV + col0 + c;
+  const float* Mc = M + (size_t)bh * (SEG - 1) * DK * DK;
+  struct Step {
+    floatx4 m[2][8], d[2];
+  };
+  auto load = [&](Step& x, int s) {
+    s = min(s, SEG - 2);                               // past the end: the last step again, unused
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+#pragma unroll
+      for (int kk = 0; kk < 8; ++kk)
+        x.m[r][kk] = *reinterpret_cast<const floatx4*>(Mc + (size_t)s * DK * DK + (((2 * w + r) * 8 + kk) * 64 + lane) * 4);
+#pragma unroll
+      for (int ii = 0; ii < 4; ++ii) x.d[r][ii] = Dc[((size_t)s * DK + 32 * w + 16 * r + 4 * g + ii) * DV];
+    }
+  };
+  Step st[3];                                          // step s in set (s - 1) % 3: two steps of lead
+  load(st[0], 1);
+  load(st[1], 2);
+  load(st[2], 3);
+#pragma unroll
+  for (int r = 0; r < 2; ++r) {
+    floatx4 x;
+#pragma unroll
+    for (int ii = 0; ii < 4; ++ii) x[ii] = Dc[(size_t)(32 * w + 16 * r + 4 * g + ii) * DV];
+    H[1][(2 * w + r) * 64 + lane] = x;
+  }
+  lds_barrier();
+  auto step = [&](Step& x, int s) {
+    const floatx4* h = H[s & 1];
+    floatx4 acc[2][2] = {{x.d[0], zero4()}, {x.d[1], zero4()}}, hv[8];
+#pragma unroll
+    for (int kk = 0; kk < 8; ++kk) hv[kk] = h[kk * 64 + lane];
+    __builtin_amdgcn_sched_barrier(0);                 // all eight reads issued before the first use
+#pragma unroll
+    for (int kk = 0; kk < 8; ++kk) {
+#pragma unroll
+      for (int r = 0; r < 2; ++r)
+#pragma unroll
+        for (int ii = 0; ii < 4; ++ii)
+          acc[r][ii & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.m[r][kk][ii], hv[kk][ii], acc[r][ii & 1], 0, 0, 0);
+    }
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+      const floatx4 y = acc[r][0] + acc[r][1];
+      H[(s + 1) & 1][(2 * w + r) * 64 + lane] = y;
+#pragma unroll
+      for (int ii = 0; ii < 4; ++ii) Dc[((size_t)s * DK + 32 * w + 16 * r + 4 * g + ii) * DV] = y[ii];
+    }
+    load(x, s + 3);
+    lds_barrier();                                     // H of the next step written, this step's read
+  };
+  int s = 1;
+  for (; s + 2 < SEG - 1; s += 3) {
+    step(st[0], s);
+    step(st[1], s + 1);
+    step(st[2], s + 2);
+  }
+  if (s < SEG - 1) step(st[0], s);
+  if (s + 1 < SEG - 1) step(st[1], s + 1);
+}
+
+}  // namespace pf

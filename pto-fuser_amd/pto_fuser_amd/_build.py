@@ -32,12 +32,13 @@ ARCH = os.environ.get("PF_OFFLOAD_ARCH", "gfx950")
 # The iterative-ILP machine scheduler issues the LDS operand reads of the scan's MFMA chains
 # several instructions ahead (the default strategy serialises every MFMA behind its own read,
 # which leaves a one-wave-per-SIMD kernel latency-bound).
-# It keeps the register file full of hoisted reads; the stage kernels, whose waves hold a prefetched
-# chunk beside the state, spill under it, so their source is compiled with the default strategy.
+# It keeps the register file full of hoisted reads; the stage and the segment kernels, whose
+# waves hold prefetched chunks beside the state, spill under it (or crash the compiler), so their
+# sources are compiled with the default strategy.
 HIPCC_FLAGS = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}",
                "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 ILP_FLAGS = ["-mllvm", "-amdgpu-sched-strategy=iterative-ilp"]
-DEFAULT_SCHED_SOURCES = ("pf_stages.hip",)
+DEFAULT_SCHED_SOURCES = ("pf_seg.hip", "pf_stages.hip")
 OBJ_DIR = os.path.join(ROOT, "_build")
 
 

@@ -80,6 +80,22 @@ def test_workspace_sizing_contract(lib):
     assert not lib.pf_gdn_setup(1, 1, 100, 64, 128, 128, 1)
 
 
+def test_gdn_workspace_of_segmented_chains():
+    """Few long chains ask for the segments' maps and states (two 128 x 128 fp32 matrices each) on top of
+    what whole chains need, and the fp32 size of a shape always covers its bf16 one."""
+    lib = _hip.load()
+
+    def size(B, H, T, dt):
+        return lib.pf_gdn_workspace_bytes(B, H, T, 64, 128, 128, dt)
+
+    base = (1 << 15) // 64 * 4 * (64 * 64 * 2 + 64 * 4) + 256
+    extra = size(1, 4, 1 << 15, _hip.PF_DTYPE_BF16) - base
+    assert extra > 0 and extra % (4 * 2 * 128 * 128 * 4) == 0
+    for B, H, T in ((1, 1, 64), (1, 1, 1024), (1, 4, 1 << 15), (1, 8, 4096), (2, 5, 5120), (4, 16, 4096),
+                    (1, 1, 1 << 22), (1, 32, 1 << 15)):
+        assert size(B, H, T, _hip.PF_DTYPE_F32) >= size(B, H, T, _hip.PF_DTYPE_BF16) > 0
+
+
 @pytest.mark.parametrize("B,H,T,C", [(1, 1, 64, 64), (4, 16, 4096, 64), (1, 32, 32768, 128),
                                      (3, 5, 192, 64)])
 def test_fp32_workspace_holds_bf16(lib, B, H, T, C):

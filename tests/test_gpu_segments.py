@@ -1,0 +1,86 @@
+"""Segmented chains of the bf16 GDN forward (few long chains): against the fp64 oracle where the segments
+divide the chain and where the last one is shorter, with and without a gate and an initial state,
+against the same call on a workspace too small for segments (which runs whole chains), and with a
+NaN in one value column.  Bound of the forward tests: max abs 2e-2 on o and the final state."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from conftest import announce, record_error
+from oracle.gdn_oracle import gdn_reference
+from pto_fuser_amd import _hip, gdn_chunk_forward
+from pto_fuser_amd.forwards import as_oracle_inputs, make_delta_inputs
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda:0")
+D = 128
+
+
+def _base_bytes(chunks):
+    """T (bf16, 64 x 64) and G (fp32) of every chunk and the scale: what whole chains need."""
+    return chunks * (64 * 64 * 2 + 64 * 4) + 256
+
+
+def _segmented(B, H, T):
+    return _hip.load().pf_gdn_workspace_bytes(B, H, T, 64, D, D, _hip.PF_DTYPE_BF16) > _base_bytes(B * H * T // 64)
+
+
+@pytest.mark.parametrize("B,H,T,kind,h0_std", [
+    (1, 1, 8192, "gdn", 0.02), (1, 2, 64 * 67, "gdn", None), (1, 3, 64 * 59, "deltanet", 0.02),
+    (2, 4, 4096, "deltanet", None), (1, 9, 64 * 97, "gdn", 0.02)])
+def test_segmented_forward(B, H, T, kind, h0_std):
+    announce(f"segmented {kind} B{B} H{H} T{T} h0={h0_std}")
+    assert _segmented(B, H, T), "the shape is meant to run in segments"
+    inp = make_delta_inputs(B, H, T, kind=kind, dtype=torch.bfloat16, seed=T + H, h0_std=h0_std)
+    d = {n: (None if t is None else t.to(DEV)) for n, t in inp.items()}
+    o, h = gdn_chunk_forward(d["q"], d["k"], d["v"], d["beta"], d["g"], h0=d["h0"])
+    o2, h2 = gdn_chunk_forward(d["q"], d["k"], d["v"], d["beta"], d["g"], h0=d["h0"])
+    torch.cuda.synchronize()
+    assert torch.equal(o, o2) and torch.equal(h, h2)
+    x = as_oracle_inputs(inp)
+    g = x["g"] if x["g"] is not None else np.zeros_like(x["beta"])
+    ro, rh = gdn_reference(x["q"], x["k"], x["v"], x["beta"], g, h0=x["h0"], C=64, dtype=np.float64)
+    for name, got, ref in (("o", o, ro), ("h", h, rh)):
+        e = record_error(f"segments {kind} B{B} H{H} T{T}", name, got.cpu().numpy(), ref, "max abs <= 0.02")
+        assert e["abs"] <= 2e-2, (name, e)
+
+
+def test_small_workspace_runs_whole_chains():
+    """A handle that holds what whole chains need (reserved for another shape of as many chunks) still
+    serves the call; both routes agree within their bf16 rounding."""
+    B, H, T = 1, 2, 8192
+    announce(f"whole chains on a small workspace B{B} H{H} T{T}")
+    lib = _hip.load()
+    assert _segmented(B, H, T) and not _segmented(16, 16, T // 128)
+    d = make_delta_inputs(B, H, T, kind="gdn", dtype=torch.bfloat16, seed=5, h0_std=0.02, device=DEV)
+    seg = gdn_chunk_forward(d["q"], d["k"], d["v"], d["beta"], d["g"], h0=d["h0"])
+    ws = ctypes.c_void_p(lib.pf_gdn_create())
+    try:
+        assert lib.pf_gdn_reserve(ws, 16, 16, T // 128, 64, D, D, _hip.PF_DTYPE_BF16) == _hip.PF_OK
+        o, h = torch.empty_like(seg[0]), torch.empty_like(seg[1])
+        st = lib.pf_gdn_exec(*(_hip.ptr(t) for t in (d["q"], d["k"], d["v"], d["beta"], d["g"], d["h0"], o, h)),
+                             B, H, T, 64, D, D, _hip.PF_DTYPE_BF16, D ** -0.5, ws, _hip.current_stream_handle(DEV))
+        _hip.check("pf_gdn_exec", st)
+        torch.cuda.synchronize()
+    finally:
+        lib.pf_gdn_teardown(ws)
+    for a, b in zip(seg, (o, h)):
+        assert not torch.equal(a, b)                     # the other route ran
+        # two correct bf16 forwards lie 2.9e-3 from float64 each: sqrt(2) of that apart, times two
+        assert float((a - b).norm() / b.norm()) <= 8.2e-3
+
+
+def test_nan_stays_in_its_column_and_behind_its_token():
+    B, H, T, tok, col = 1, 2, 8192, 5000, 17
+    announce(f"segmented NaN containment B{B} H{H} T{T}")
+    d = make_delta_inputs(B, H, T, kind="gdn", dtype=torch.bfloat16, seed=6, device=DEV)
+    d["v"][0, 0, tok, col] = float("nan")
+    o, h = gdn_chunk_forward(d["q"], d["k"], d["v"], d["beta"], d["g"])
+    torch.cuda.synchronize()
+    bad = torch.isnan(o)
+    assert bad[0, 0, tok:, col].all() and bool(torch.isnan(h)[0, 0, :, col].all())
+    assert not bad[0, 1].any() and not bad[0, 0, :tok // 64 * 64].any()
+    others = [c for c in range(D) if c != col]
+    assert not bad[0, 0][:, others].any() and not torch.isnan(h)[0, 0][:, others].any()
