@@ -17,8 +17,7 @@
 
 namespace {
 
-// loader waves of the bf16 split scan kernel for 32-column and for 16-column slices
-constexpr int kSplitLoaderWaves = 4, kSplit16LoaderWaves = 4;
+constexpr int kSplitLoaderWaves = 4;   // loader waves of the bf16 split scan kernel
 
 using pf::bf16;
 
@@ -37,11 +36,19 @@ struct Segments {
 
 int generations(long wgs) { return (int)((wgs + pf::device_cu_count() - 1) / pf::device_cu_count()); }
 
-// Column slices of the bf16 scan: 16 columns (a chunk step of 1.2 us) while eight slices per unit fit
-// one generation of workgroups, else 32 (1.45 us, half the workgroups).
-bool narrow_slices(long units) { return units * 8 <= pf::device_cu_count(); }
+// Column slices of the bf16 scan, one workgroup per CU: 16 columns (a chunk step of 1.2 us) while eight
+// slices per unit fit one generation of workgroups, 32 (1.45 us) while four do, else 64 (2.0-2.3 us,
+// half the workgroups of 32 and half their reads of k, q and T).  Whole forward at 16 / 32 / 64 columns:
+// 32 chains x 128 chunks 176 / 193 / 272 us, 64 x 64 178 / 113 / 150, 65 x 64 339 / 250 / 150,
+// 96 x 64 265 / 207 / 160, 128 x 64 349 / 240 / 194, 192 x 32 283 / 180 / 164, 512 x 8 235 / 157 / 116.
+// The three give the same bits.
+int slice_columns(long units) {
+  const int cus = pf::device_cu_count();
+  return units * 8 <= cus ? 16 : units * 4 <= cus ? 32 : 64;
+}
 double scan_us(long units, int chunks) {
-  return narrow_slices(units) ? 1.2 * chunks : 1.45 * chunks * generations(units * 4);
+  const int cols = slice_columns(units);
+  return (cols == 16 ? 1.2 : cols == 32 ? 1.45 : 2.25) * chunks * generations(units * (128 / cols));
 }
 
 // Segments of a bf16 chain.  A chain's time is its chunk count while chains leave CUs idle; in
@@ -184,14 +191,15 @@ void scan_output_launch(const void* q, const void* k, const void* v, const float
       pf::seg_states_launch(m, stream);
     }
     const int units = BH * sg.seg;
-    // bf16: one workgroup per (segment or whole chain, 32- or 16-column slice); four MFMA waves split
+    // bf16: one workgroup per (segment or whole chain, column slice); four MFMA waves split
     // every chunk (pf_scan_split.h)
-    if (narrow_slices(units))
-      pf::scan_split_kernel<C, DK, DV, 1, kSplit16LoaderWaves>
-          <<<dim3((unsigned)(units * (DV / 16))), dim3(64 * (4 + kSplit16LoaderWaves)), 0, stream>>>(a);
-    else
-      pf::scan_split_kernel<C, DK, DV, 2, kSplitLoaderWaves>
-          <<<dim3((unsigned)(units * (DV / 32))), dim3(64 * (4 + kSplitLoaderWaves)), 0, stream>>>(a);
+    const int cols = slice_columns(units);
+    const dim3 grid((unsigned)(units * (DV / cols))), block(64 * (4 + kSplitLoaderWaves));
+    switch (cols) {
+      case 16: pf::scan_split_kernel<C, DK, DV, 1, kSplitLoaderWaves><<<grid, block, 0, stream>>>(a); break;
+      case 32: pf::scan_split_kernel<C, DK, DV, 2, kSplitLoaderWaves><<<grid, block, 0, stream>>>(a); break;
+      default: pf::scan_split_kernel<C, DK, DV, 4, kSplitLoaderWaves><<<grid, block, 0, stream>>>(a); break;
+    }
   } else {
     // fp32: one workgroup per (chain, 16-column slice), every chunk split over four waves
     // (pf_scan_split_f32.h)

@@ -44,7 +44,7 @@
 // or at a raised priority, was measured to stall the compute waves sharing the SIMDs (one phase
 // lost up to 1 000 cycles; q's loads in the first phase beside k's cost 5 % of the kernel).
 // The compute waves store their o rows themselves, 16-byte stores: with 32-column slices two per
-// lane, non-temporal, after lanes c and c + 8 swap the halves of a token's 128-byte row so that
+// lane (64: four), non-temporal, after lanes c and c + 8 swap the halves of a token's 128-byte row so that
 // every store instruction writes whole lines; with 16-column slices one per lane, through the
 // cache (the line's other half comes from the neighbouring slice's workgroup).  The loaders also carry the deferred state decay: the compute waves hold
 // S~ = S / f with a running factor f folded into the gate tables, and multiply it back only when
@@ -102,8 +102,8 @@ void scan_split_kernel(ScanOutArgs a) {
   constexpr int KP = Stage::KP, TP = Stage::TP, VP = Stage::VP;
   constexpr int NS = DV / NCOL;                 // slices per chain
   constexpr int FRAG = 64 * 8;                  // bf16 elements of one operand fragment
-  static_assert(C == 64 && DK == 128 && (NT == 1 || NT == 2) && (NLW == 2 || NLW == 4),
-                "tile shapes of the split scan kernel: C 64, DK 128, 16 or 32 columns");
+  static_assert(C == 64 && DK == 128 && (NT == 1 || NT == 2 || NT == 4) && (NLW == 2 || NLW == 4),
+                "tile shapes of the split scan kernel: C 64, DK 128, 16, 32 or 64 columns");
 
   __shared__ __attribute__((aligned(16))) Stage st[2];
   __shared__ __attribute__((aligned(16))) bf16 SB[4 * NT * FRAG];
@@ -523,31 +523,33 @@ void scan_split_kernel(ScanOutArgs a) {
         // non-temporal (o is never read here; streaming it past L2 leaves the cache to the k, q
         // and T lines the chain's other column slices read: 7 % of the kernel's time)
         const float egs = s.EGS[tok0 + c];
-        if constexpr (NT == 2) {
-          // a token's 32 columns are one 128-byte line: lanes c and c + 8 of a row swap halves
+        if constexpr (NT >= 2) {
+          // 32 columns of a token are one 128-byte line: lanes c and c + 8 of a row swap halves
           // (DPP row rotate by 8) so that each store instruction writes eight whole lines, tokens
           // 0..7 then 8..15 of the block (two half-line stores reach memory apart when streamed)
-          floatx4 v0, v1;
-#pragma unroll
-          for (int ii = 0; ii < 4; ++ii) {
-            v0[ii] = fmaf(egs, QT[0][ii], OT[0][ii]);
-            v1[ii] = fmaf(egs, QT[1][ii], OT[1][ii]);
-          }
           const bool hi = c >= 8;
-          floatx4 sa, sb;
 #pragma unroll
-          for (int ii = 0; ii < 4; ++ii) {
-            const float send = hi ? v0[ii] : v1[ii];
-            const float recv = __int_as_float(__builtin_amdgcn_update_dpp(
-                __float_as_int(send), __float_as_int(send), 0x128, 0xf, 0xf, false));   // row_ror:8
-            sa[ii] = hi ? recv : v0[ii];                 // token c & 7, columns 16 hi + 4g ..
-            sb[ii] = hi ? v1[ii] : recv;                 // token 8 + (c & 7), same columns
+          for (int p = 0; p < NT / 2; ++p) {
+            floatx4 v0, v1, sa, sb;
+#pragma unroll
+            for (int ii = 0; ii < 4; ++ii) {
+              v0[ii] = fmaf(egs, QT[2 * p][ii], OT[2 * p][ii]);
+              v1[ii] = fmaf(egs, QT[2 * p + 1][ii], OT[2 * p + 1][ii]);
+            }
+#pragma unroll
+            for (int ii = 0; ii < 4; ++ii) {
+              const float send = hi ? v0[ii] : v1[ii];
+              const float recv = __int_as_float(__builtin_amdgcn_update_dpp(
+                  __float_as_int(send), __float_as_int(send), 0x128, 0xf, 0xf, false));   // row_ror:8
+              sa[ii] = hi ? recv : v0[ii];               // token c & 7, columns 32 p + 16 hi + 4g ..
+              sb[ii] = hi ? v1[ii] : recv;               // token 8 + (c & 7), same columns
+            }
+            const uint32_t col = col0 + 32 * p + (hi ? 16 : 0) + 4 * g;
+            const uint32_t ra = (uint32_t)(((size_t)ch * C + tok0 + (c & 7)) * DV + col) * 4;
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, sa), ro, ra, 0, kCachePolicyNT);
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, sb), ro, ra + 8 * DV * 4, 0,
+                                                   kCachePolicyNT);
           }
-          const uint32_t col = col0 + (hi ? 16 : 0) + 4 * g;
-          const uint32_t ra = (uint32_t)(((size_t)ch * C + tok0 + (c & 7)) * DV + col) * 4;
-          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, sa), ro, ra, 0, kCachePolicyNT);
-          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, sb), ro, ra + 8 * DV * 4, 0,
-                                                 kCachePolicyNT);
         } else {
           // 16-column slices: the other half of each 128-byte line comes from the neighbouring
           // slice's workgroup (same XCD), so o is stored through the cache, where the halves

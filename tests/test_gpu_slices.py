@@ -1,0 +1,44 @@
+"""The bf16 scan's column slices: 16, 32 and 64 columns, chosen by how many chains a call has.  A state
+column is computed the same way in all three, so a chain's outputs do not depend on how many chains
+run beside it: the first 40 and the first 8 of 72 chains give the same bits as within the 72, with
+every score-gate path, one chunk to five, and 72 and 69 chains (grouped by XCD and not)."""
+import pytest
+import torch
+
+from conftest import announce
+from pto_fuser_amd import gdn_chunk_forward
+from pto_fuser_amd.forwards import make_delta_inputs
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda:0")
+
+
+def _gate(name, shape, seed):
+    x = torch.randn(*shape, generator=torch.Generator().manual_seed(seed))
+    sp = torch.nn.functional.softplus
+    if name == "rising":                  # g > 0 in places
+        return x * 0.05 - 0.03
+    if name == "steep":                   # over 80 of decay inside a 16-token block
+        return -sp(x) * 12.0
+    return -sp(x) * 0.1
+
+
+@pytest.mark.parametrize("gate", ["gentle", "rising", "steep"])
+@pytest.mark.parametrize("H,T", [(72, 64), (72, 192), (69, 320)])
+def test_a_chain_does_not_depend_on_its_neighbours(gate, H, T):
+    announce(f"GDN bf16 slices {gate} H{H} T{T}")
+    d = make_delta_inputs(1, H, T, kind="gdn", dtype=torch.bfloat16, seed=H + T, h0_std=0.02)
+    d["g"] = _gate(gate, (1, H, T), T).float()
+    d = {n: t.to(DEV) for n, t in d.items()}
+
+    def run(n):
+        x = {k: t[:, :n].contiguous() for k, t in d.items()}
+        return gdn_chunk_forward(x["q"], x["k"], x["v"], x["beta"], x["g"], h0=x["h0"])
+
+    o, h = run(H)
+    torch.cuda.synchronize()
+    assert bool(torch.isfinite(o).all() and torch.isfinite(h).all())
+    for n in (40, 8):
+        on, hn = run(n)
+        torch.cuda.synchronize()
+        assert torch.equal(on, o[:, :n]) and torch.equal(hn, h[:, :n])
