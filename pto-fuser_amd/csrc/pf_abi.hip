@@ -52,8 +52,7 @@ double scan_us(long units, int chunks) {
 }
 
 // Segments of a bf16 chain.  A chain's time is its chunk count while chains leave CUs idle; in
-// segments it is the segment's length twice (its map, 2.5 us per chunk step on one workgroup per CU,
-// and the scan) plus a composition step of 1.9 us per segment, and 9 us for the two more launches.  The
+// segments it is the segment's length twice (its map, 2.45 or 3.35 us per chunk step, and the scan) plus a composition step of 1.9 us per segment, and 9 us for the two more launches.  The
 // times are per generation of workgroups, as measured; segments are taken where they come out 10 %
 // ahead.  Measured, whole forward, one chain against its segments: 4 chains x 512 chunks 577 -> 157 us,
 // 8 x 256 300 -> 132, 16 x 128 160 -> 119, 8 x 64 82 -> 59, 1 x 128 147 -> 68, 2 x 32 44 -> 42; not taken:
@@ -64,8 +63,8 @@ Segments gdn_segments(int BH, int NC, int dtype) {
   double t = 0.9 * scan_us(BH, NC);
   for (int want = 4; want <= 64 && want * 4 <= NC; want += want < 8 ? 2 : want / 4) {
     const int len = (NC + want - 1) / want, seg = (NC + len - 1) / len;
-    const double x = 9.0 + 2.5 * len * generations((long)BH * (2 * seg - 3)) + 1.9 * (seg - 2) +
-                     scan_us((long)BH * seg, len);
+    const double map = pf::seg_map_split(BH, seg) ? 2.45 * len : 3.35 * len * generations((long)BH * (seg - 1));
+    const double x = 9.0 + map + 1.9 * (seg - 2) + scan_us((long)BH * seg, len);
     if (x < t) {
       t = x;
       best = {seg, len};

@@ -39,6 +39,8 @@ struct SegMapArgs {
   int BH, NC;           // chains, chunks per chain
   int SEG, L;           // segments per chain, chunks per segment (the last may have fewer)
 };
+// D and M of a segment in workgroups of their own (the shorter chunk step), while those fit one generation.
+bool seg_map_split(int BH, int SEG);
 void seg_states_launch(const SegMapArgs& m, hipStream_t stream);
 
 }  // namespace pf

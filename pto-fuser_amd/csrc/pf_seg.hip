@@ -3,12 +3,18 @@
 #include <hip/hip_runtime.h>
 
 #include "pf_seg_scan.h"
+#include "pf_status.h"
 
 namespace pf {
 
+bool seg_map_split(int BH, int SEG) { return BH * (2 * SEG - 3) <= device_cu_count(); }
+
 void seg_states_launch(const SegMapArgs& m, hipStream_t stream) {
   const unsigned units = (unsigned)(m.BH * (m.SEG - 1));
-  seg_map_kernel<64, 128, 128><<<dim3((units + 7) / 8 * 16), dim3(512), 0, stream>>>(m);
+  if (seg_map_split(m.BH, m.SEG))
+    seg_map_kernel<64, 128, 128, 1><<<dim3((units + 7) / 8 * 16), dim3(512), 0, stream>>>(m);
+  else
+    seg_map_kernel<64, 128, 128, 2><<<dim3(units), dim3(512), 0, stream>>>(m);
   if (m.SEG > 2)
     seg_compose_kernel<128, 128><<<dim3((unsigned)((m.BH + 7) / 8 * 64)), dim3(256), 0, stream>>>(m.D, m.M, m.BH, m.SEG);
 }

@@ -13,14 +13,18 @@
 // where chains leave the chip idle or their length is the bound, not where every CU is busy
 // (gdn_segments in pf_abi.hip has the rule and its measurements).
 //
-// seg_map_kernel: state columns are independent, so a wave owns 16 of them for the whole segment and
+// seg_map_kernel: state columns are independent, so a wave owns 16 NT of them for the whole segment and
 // every product feeds the next from registers: S (packed pairs of D tiles) is the B operand of k S,
 // r = beta v - beta e^G (k S) that of T r, v_new e^{G_last - G} that of the update
-// S <- e^{G_last} S + k^T (.).  The eight waves of a workgroup (D or M of one segment) share only
-// the chunk's k, T, v and gate images in LDS (two), loaded into registers three chunks ahead.  Tile pair (2x, 2x + 1) holds rows (state
-// rows or tokens) 32x + 8g + 0..7 per lane group, so k and T rows are read as natural-order 16-byte
-// fragments and k^T by transposed reads of the same image.  fp32 state and accumulators, bf16
-// operands, as in the scan itself.
+// S <- e^{G_last} S + k^T (.).  Workgroups of eight waves: NT = 1, D or M of a segment each (the shorter
+// step, while they fit one generation); NT = 2, four waves on D and four on M (half the LDS reads).
+// M runs the same code with v masked to zero, so a chunk is straight-line code.  Waves share only the
+// chunk's k, T, v and gate images in LDS (two), loaded into registers two chunks ahead.  Tile pair (2x, 2x + 1) holds
+// rows (state rows or tokens) 32x + 8g + 0..7 per lane group, so k and T rows are read as
+// natural-order 16-byte fragments and k^T by transposed reads of the same image; a fragment read
+// serves all of the wave's column tiles.  fp32 state and accumulators, bf16 operands, as in the scan
+// itself.  A chunk step takes 2.4 us (NT = 1, 128 columns) or 3.3 us (NT = 2, 256 columns): 336 KB of LDS
+// reads, 76 products and about 300 vector instructions per wave at NT = 2, two waves per SIMD.
 #pragma once
 
 #include "pf_gfx950.h"
@@ -44,20 +48,29 @@ __device__ __forceinline__ constexpr int seg_m_index(int row, int col) {
 }
 
 struct SegImage {                                      // one chunk in LDS
-  bf16 ks[64 * 128], ts[64 * 64], vs[8 * 64 * 16];     // v: per wave [64][16]
+  bf16 ks[64 * 128], ts[64 * 64], vs[8 * 64 * 16];     // v: per 16 columns [64][16]
   struct {
     float BT[64], BEG[64], EL[64];                     // beta, beta e^G, e^{G_last - G}
   } gate[8];                                           // per wave: no branch around the tables
 };
 
-// D (MAP false) or M (MAP true) of segment `seg` of chain bh.  MAP is a template parameter so that the
-// chunk is straight-line code (a uniform branch around v splits it, and every LDS read is then waited
-// for where it is issued).
-template <int C, int DK, int DV, bool MAP>
-__device__ __forceinline__ void seg_map_run(const SegMapArgs& a, SegImage (&img)[2], int bh, int seg) {
+template <int C, int DK, int DV, int NT>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void seg_map_kernel(SegMapArgs a) {
+  static_assert(C == 64 && DK == 128 && DV == 128, "the forward's tile: C 64, dk = dv = 128");
+  __shared__ __attribute__((aligned(16))) SegImage img[2];
+  // NT = 2: one workgroup per segment; NT = 1: two, eight ids apart (one XCD: they read the same k and T)
+  const int bid = blockIdx.x;
+  const int unit = NT == 2 ? bid : bid / 16 * 8 + bid % 8;
+  if (unit >= a.BH * (a.SEG - 1)) return;
+  const int bh = unit / (a.SEG - 1), seg = unit % (a.SEG - 1);
   const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, c = lane & 15;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int col = 16 * w + c;
+  const bool map = NT == 2 ? w >= 4 : bid % 16 >= 8;   // M, else D
+  if (NT == 1 && map && seg == 0) return;              // the first segment's D is the state itself
+  const int wt = NT == 2 ? NT * (w & 3) : w;           // this wave's first column tile
+  const int col = 16 * wt + c;                         // this lane's column of tile nt: + 16 nt
+  const unsigned vmask = map ? 0u : ~0u;
   const size_t m0 = (size_t)bh * a.NC + (size_t)seg * a.L, t0 = m0 * C;
   const bf16* kg = a.k + t0 * DK;
   const bf16* vg = a.v + t0 * DV;
@@ -75,10 +88,8 @@ __device__ __forceinline__ void seg_map_run(const SegMapArgs& a, SegImage (&img)
 #pragma unroll
     for (int i = 0; i < 2; ++i) x.k[i] = *reinterpret_cast<const u32x4*>(kg + (size_t)ch * C * DK + (tid + 512 * i) * 8);
     x.t = *reinterpret_cast<const u32x4*>(tg + (size_t)ch * C * C + tid * 8);
-    if constexpr (!MAP) {
 #pragma unroll
-      for (int i = 0; i < 2; ++i) x.v[i] = *reinterpret_cast<const u32x4*>(vg + (size_t)ch * C * DV + (tid + 512 * i) * 8);
-    }
+    for (int i = 0; i < 2; ++i) x.v[i] = *reinterpret_cast<const u32x4*>(vg + (size_t)ch * C * DV + (tid + 512 * i) * 8);
     x.g = Gg[(size_t)ch * C + lane];
     x.b = Bg[(size_t)ch * C + lane];
   };
@@ -87,7 +98,7 @@ __device__ __forceinline__ void seg_map_run(const SegMapArgs& a, SegImage (&img)
     for (int i = 0; i < 2; ++i) {
       const int u = tid + 512 * i, row = u >> 4, s = u & 15;
       *reinterpret_cast<u32x4*>(im.ks + row * DK + 8 * seg_k_slot(row, s)) = x.k[i];
-      if constexpr (!MAP) *reinterpret_cast<u32x4*>(im.vs + (s >> 1) * C * 16 + row * 16 + 8 * (s & 1)) = x.v[i];
+      *reinterpret_cast<u32x4*>(im.vs + (s >> 1) * C * 16 + row * 16 + 8 * (s & 1)) = x.v[i];
     }
     *reinterpret_cast<u32x4*>(im.ts + (tid >> 3) * C + 8 * seg_t_slot(tid >> 3, tid & 7)) = x.t;
     const float gl = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x.g), C - 1));
@@ -97,125 +108,131 @@ __device__ __forceinline__ void seg_map_run(const SegMapArgs& a, SegImage (&img)
     return __expf(gl);                                 // the chunk's decay
   };
 
-  floatx4 S[8];
+  floatx4 S[8][NT];
 #pragma unroll
   for (int r = 0; r < 8; ++r)
 #pragma unroll
-    for (int ii = 0; ii < 4; ++ii) S[r][ii] = MAP && seg_row(r, g, ii) == col ? 1.f : 0.f;
-  if (!MAP && seg == 0 && a.h0) {                      // one branch around all loads
+    for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+      for (int ii = 0; ii < 4; ++ii) S[r][nt][ii] = map && seg_row(r, g, ii) == col + 16 * nt ? 1.f : 0.f;
+  if (!map && seg == 0 && a.h0) {                      // one branch around all loads
     const float* h = a.h0 + (size_t)bh * DK * DV + col;
 #pragma unroll
     for (int r = 0; r < 8; ++r)
 #pragma unroll
-      for (int ii = 0; ii < 4; ++ii) S[r][ii] = h[seg_row(r, g, ii) * DV];
+      for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+        for (int ii = 0; ii < 4; ++ii) S[r][nt][ii] = h[seg_row(r, g, ii) * DV + 16 * nt];
   }
 
   const int crow = 8 * (c >> 2) + (c & 3);             // + 32x + 4h: the row lane c supplies
   const int trow = 8 * g + (c >> 2);                   // transposed reads: + 32x + 4h
-  // chunk m in register set m % 3 until it is written to LDS, three chunks of lead
-  Regs r0, r1, r2;
+  // chunk m in register set m & 1 until it is written to LDS
+  Regs r0, r1;
   load(r0, 0);
   load(r1, 1);
-  load(r2, 2);
   float dl = store(img[0], r0), dl_next = 0.f;
-  load(r0, 3);
+  load(r0, 2);
   lds_barrier();
   auto chunk = [&](Regs& nx, int ch) {                 // nx holds chunk ch + 1
     const SegImage& im = img[ch & 1];
-    const bf16 *ks = im.ks, *ts = im.ts, *vs = im.vs;
-    bf16x8 Sb[4];
+    const bf16 *ks = im.ks, *ts = im.ts, *vs = im.vs + wt * C * 16;
+    bf16x8 Sb[4][NT];
 #pragma unroll
-    for (int kb = 0; kb < 4; ++kb) Sb[kb] = pack8(S[2 * kb], S[2 * kb + 1]);
+    for (int kb = 0; kb < 4; ++kb)
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) Sb[kb][nt] = pack8(S[2 * kb][nt], S[2 * kb + 1][nt]);
     // r = beta v - beta e^G (k S)
-    bf16x8 Rb[2];
+    bf16x8 Rb[2][NT];
 #pragma unroll
     for (int x = 0; x < 2; ++x) {
-      floatx4 r[2];
+      floatx4 r[2][NT];
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
-        floatx4 Y = zero4();
+        floatx4 Y[NT];
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) Y[nt] = zero4();
         const int row = 32 * x + 4 * h + crow;
 #pragma unroll
-        for (int kb = 0; kb < 4; ++kb)
-          Y = mfma_bf16(*reinterpret_cast<const bf16x8*>(ks + row * DK + 8 * seg_k_slot(row, 4 * kb + g)), Sb[kb], Y);
+        for (int kb = 0; kb < 4; ++kb) {
+          const bf16x8 kf = *reinterpret_cast<const bf16x8*>(ks + row * DK + 8 * seg_k_slot(row, 4 * kb + g));
+#pragma unroll
+          for (int nt = 0; nt < NT; ++nt) Y[nt] = mfma_bf16(kf, Sb[kb][nt], Y[nt]);
+        }
         const int t4 = 32 * x + 8 * g + 4 * h;
         const floatx4 beg = *reinterpret_cast<const floatx4*>(im.gate[w].BEG + t4);
-        if constexpr (MAP) {
+        const floatx4 bt = *reinterpret_cast<const floatx4*>(im.gate[w].BT + t4);
 #pragma unroll
-          for (int ii = 0; ii < 4; ++ii) r[h][ii] = -beg[ii] * Y[ii];
-        } else {
-          const floatx4 bt = *reinterpret_cast<const floatx4*>(im.gate[w].BT + t4);
-          const bf16x4 v4 = lds_read_tr(vs + w * C * 16 + (32 * x + 4 * h + trow) * 16 + 4 * (c & 3));
+        for (int nt = 0; nt < NT; ++nt) {
+          typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+          const u32x2 vx = __builtin_bit_cast(u32x2, lds_read_tr(vs + nt * C * 16 + (32 * x + 4 * h + trow) * 16 + 4 * (c & 3)));
+          const bf16x4 v4 = __builtin_bit_cast(bf16x4, u32x2{vx[0] & vmask, vx[1] & vmask});
 #pragma unroll
-          for (int ii = 0; ii < 4; ++ii) r[h][ii] = fmaf(-beg[ii], Y[ii], bt[ii] * (float)v4[ii]);
+          for (int ii = 0; ii < 4; ++ii) r[h][nt][ii] = fmaf(-beg[ii], Y[nt][ii], bt[ii] * (float)v4[ii]);
         }
       }
-      Rb[x] = pack8(r[0], r[1]);
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) Rb[x][nt] = pack8(r[0][nt], r[1][nt]);
     }
-    dl_next = store(img[(ch + 1) & 1], nx);                      // last read a barrier ago
-    load(nx, ch + 4);
+    dl_next = store(img[(ch + 1) & 1], nx);            // last read a barrier ago
+    load(nx, ch + 3);
     // v_new = T r (T lower triangular by 32-token blocks), scaled by e^{G_last - G}
-    bf16x8 Vb[2];
+    bf16x8 Vb[2][NT];
 #pragma unroll
     for (int x = 0; x < 2; ++x) {
-      floatx4 V[2];
+      floatx4 V[2][NT];
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
-        V[h] = zero4();
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) V[h][nt] = zero4();
         const int row = 32 * x + 4 * h + crow;
 #pragma unroll
-        for (int xb = 0; xb <= x; ++xb)
-          V[h] = mfma_bf16(*reinterpret_cast<const bf16x8*>(ts + row * C + 8 * seg_t_slot(row, 4 * xb + g)), Rb[xb], V[h]);
-        V[h] *= *reinterpret_cast<const floatx4*>(im.gate[w].EL + 32 * x + 8 * g + 4 * h);
+        for (int xb = 0; xb <= x; ++xb) {
+          const bf16x8 tf = *reinterpret_cast<const bf16x8*>(ts + row * C + 8 * seg_t_slot(row, 4 * xb + g));
+#pragma unroll
+          for (int nt = 0; nt < NT; ++nt) V[h][nt] = mfma_bf16(tf, Rb[xb][nt], V[h][nt]);
+        }
+        const floatx4 el = *reinterpret_cast<const floatx4*>(im.gate[w].EL + 32 * x + 8 * g + 4 * h);
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) V[h][nt] *= el;
       }
-      Vb[x] = pack8(V[0], V[1]);
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) Vb[x][nt] = pack8(V[0][nt], V[1][nt]);
     }
     // S <- e^{G_last} S + k^T (.)
 #pragma unroll
     for (int r = 0; r < 8; ++r) {
-      floatx4 acc = S[r] * dl;
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) S[r][nt] *= dl;
 #pragma unroll
       for (int x = 0; x < 2; ++x) {
         const int r0 = 32 * x + trow, off = 8 * seg_k_slot(trow, 4 * (r >> 1) + (c & 3)) + 4 * (r & 1);
         // rows r0 and r0 + 4 share their slot permutation (row bits 0, 1, 3, 4)
-        acc = mfma_bf16(cat8(lds_read_tr(ks + r0 * DK + off), lds_read_tr(ks + (r0 + 4) * DK + off)), Vb[x], acc);
+        const bf16x8 kt = cat8(lds_read_tr(ks + r0 * DK + off), lds_read_tr(ks + (r0 + 4) * DK + off));
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) S[r][nt] = mfma_bf16(kt, Vb[x][nt], S[r][nt]);
       }
-      S[r] = acc;
     }
     dl = dl_next;
     lds_barrier();                                     // the next image written, this one read
   };
   int ch = 0;
-  for (; ch + 2 < a.L; ch += 3) {
+  for (; ch + 1 < a.L; ch += 2) {
     chunk(r1, ch);
-    chunk(r2, ch + 1);
-    chunk(r0, ch + 2);
+    chunk(r0, ch + 1);
   }
   if (ch < a.L) chunk(r1, ch);
-  if (ch + 1 < a.L) chunk(r2, ch + 1);
-  float* out = (MAP ? a.M : a.D) + ((size_t)bh * (a.SEG - 1) + seg) * DK * DV;
+  if (map && seg == 0) return;
+  float* out = (map ? a.M : a.D) + (size_t)unit * DK * DV;
 #pragma unroll
   for (int r = 0; r < 8; ++r)
 #pragma unroll
-    for (int ii = 0; ii < 4; ++ii) {
-      const int row = seg_row(r, g, ii);
-      out[MAP ? seg_m_index(row, col) : row * DV + col] = S[r][ii];
-    }
-}
-
-template <int C, int DK, int DV>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
-void seg_map_kernel(SegMapArgs a) {
-  static_assert(C == 64 && DK == 128 && DV == 128, "the forward's tile: C 64, dk = dv = 128");
-  __shared__ __attribute__((aligned(16))) SegImage img[2];
-  // the workgroups of D and M of one segment on one XCD: they read the same k and T
-  const int units = a.BH * (a.SEG - 1), bid = blockIdx.x;
-  const int unit = (bid / 16) * 8 + bid % 8;
-  const bool map = bid % 16 >= 8;
-  if (unit >= units) return;
-  const int bh = unit / (a.SEG - 1), seg = unit % (a.SEG - 1);
-  if (!map) seg_map_run<C, DK, DV, false>(a, img, bh, seg);
-  else if (seg > 0) seg_map_run<C, DK, DV, true>(a, img, bh, seg);
+    for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+      for (int ii = 0; ii < 4; ++ii) {
+        const int row = seg_row(r, g, ii), cl = col + 16 * nt;
+        out[map ? seg_m_index(row, cl) : row * DV + cl] = S[r][nt][ii];
+      }
 }
 
 // H_{s+1} = D_s + M_s H_s for s = 1 .. SEG - 2 (H_1 = D_0 is final), written over D_s.  One workgroup per
