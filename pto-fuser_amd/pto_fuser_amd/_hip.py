@@ -12,6 +12,8 @@ import ctypes
 import os
 from typing import Optional
 
+import torch
+
 from . import _build
 
 PF_DTYPE_F32 = 0
@@ -122,5 +124,9 @@ def ptr(t) -> Optional[int]:
 
 
 def current_stream_handle(device=None) -> int:
-    import torch
-    return torch.cuda.current_stream(device).cuda_stream
+    """The current stream's hipStream_t.  Every launch asks for it, so for a device with an index
+    the handle is read directly, without the Stream object torch.cuda.current_stream builds."""
+    index = getattr(device, "index", None)
+    if index is None:
+        return torch.cuda.current_stream(device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(index)

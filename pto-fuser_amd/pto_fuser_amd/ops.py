@@ -26,19 +26,26 @@ SUPPORTED_C = (64, 128)   # the fused forwards run 64-token chunks; 128 regroups
 SUPPORTED_D = (128,)
 
 
+_DTYPE_CODES = {torch.float32: _hip.PF_DTYPE_F32, torch.bfloat16: _hip.PF_DTYPE_BF16}
+
+
 def _dtype_code(dtype: torch.dtype) -> int:
-    if dtype == torch.float32:
-        return _hip.PF_DTYPE_F32
-    if dtype == torch.bfloat16:
-        return _hip.PF_DTYPE_BF16
-    raise ValueError(f"unsupported operand dtype {dtype} (float32 or bfloat16)")
+    code = _DTYPE_CODES.get(dtype)
+    if code is None:
+        raise ValueError(f"unsupported operand dtype {dtype} (float32 or bfloat16)")
+    return code
 
 
 def _require(t: Optional[torch.Tensor], name: str, shape, dtype, device) -> None:
+    """``t`` (None passes) is a contiguous tensor of this shape, dtype and device.  A call makes one
+    such check per operand, so the passing case is one expression; the rest names what failed."""
     if t is None:
         return
     if not isinstance(t, torch.Tensor):
         raise ValueError(f"{name} must be a tensor")
+    if (t.shape == shape and t.dtype is dtype and t.get_device() == device.index
+            and t.is_contiguous()):
+        return
     if tuple(t.shape) != tuple(shape):
         raise ValueError(f"{name} has shape {tuple(t.shape)}, expected {tuple(shape)}")
     if t.dtype != dtype:
@@ -47,6 +54,17 @@ def _require(t: Optional[torch.Tensor], name: str, shape, dtype, device) -> None
         raise ValueError(f"{name} is on {t.device}, expected {device}")
     if not t.is_contiguous():
         raise ValueError(f"{name} must be contiguous")
+
+
+def _require_rows(t: Optional[torch.Tensor], name: str, shape, dtype, device) -> None:
+    """``t`` (None passes) flattens to ``shape``: a contiguous tensor with as many elements."""
+    if t is None:
+        return
+    numel = shape[0] * shape[1] if len(shape) == 2 else shape[0]
+    if (t.numel() == numel and t.dtype is dtype and t.get_device() == device.index
+            and t.is_contiguous()):
+        return
+    _require(t.reshape(shape) if t.is_contiguous() else t, name, shape, dtype, device)
 
 
 class GdnWorkspace:
@@ -73,30 +91,26 @@ class GdnWorkspace:
 _WORKSPACES: Dict[tuple, object] = {}
 
 
-def _stream_key(device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
-
-
-def _cached_workspace(key: tuple, make):
-    """The workspace cached under ``key`` (shape, device and the current stream), created on
-    first use.  One per stream: forwards of the same shape enqueued on two streams would
-    otherwise overwrite each other's intermediates.  Creating one allocates device memory, which
-    a HIP graph capture must not record: under capture a missing workspace raises (run the call
-    once on the capture stream before capturing, as graph.GraphReplayExecutor's warmup does)."""
+def _workspace(cls, B, H, T, C, DK, DV, code, device, stream):
+    """The ``cls`` workspace of a shape, device and stream, created on first use.  One per stream:
+    forwards of the same shape enqueued on two streams would otherwise overwrite each other's
+    intermediates.  Creating one allocates device memory, which a HIP graph capture must not
+    record: under capture a missing workspace raises (run the call once on the capture stream
+    before capturing, as graph.GraphReplayExecutor's warmup does)."""
+    key = (cls, B, H, T, C, DK, DV, code, device, stream)
     ws = _WORKSPACES.get(key)
     if ws is None:
         if torch.cuda.is_current_stream_capturing():
             raise RuntimeError("no workspace for this shape on the capturing stream: run the "
                                "forward once on that stream before capturing it")
-        ws = make()
-        _WORKSPACES[key] = ws
+        ws = _WORKSPACES[key] = cls(B, H, T, C, DK, DV, code, device)
     return ws
 
 
 def gdn_workspace(B, H, T, C, DK, DV, dtype: torch.dtype, device) -> GdnWorkspace:
-    code = _dtype_code(dtype)
-    key = ("gdn", B, H, T, C, DK, DV, code, str(device), _stream_key(device))
-    return _cached_workspace(key, lambda: GdnWorkspace(B, H, T, C, DK, DV, code, device))
+    device = torch.device(device)
+    return _workspace(GdnWorkspace, B, H, T, C, DK, DV, _dtype_code(dtype), device,
+                      _hip.current_stream_handle(device))
 
 
 class KdaWorkspace:
@@ -120,9 +134,9 @@ class KdaWorkspace:
 
 
 def kda_workspace(B, H, T, C, DK, DV, dtype: torch.dtype, device) -> KdaWorkspace:
-    code = _dtype_code(dtype)
-    key = ("kda", B, H, T, C, DK, DV, code, str(device), _stream_key(device))
-    return _cached_workspace(key, lambda: KdaWorkspace(B, H, T, C, DK, DV, code, device))
+    device = torch.device(device)
+    return _workspace(KdaWorkspace, B, H, T, C, DK, DV, _dtype_code(dtype), device,
+                      _hip.current_stream_handle(device))
 
 
 def release_workspaces() -> None:
@@ -166,19 +180,19 @@ def gdn_chunk_forward(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, beta: t
     _require(beta, "beta", (B, H, T), torch.float32, dev)
     _require(g, "g", (B, H, T), torch.float32, dev)
     _require(h0, "h0", (B, H, DK, DV), torch.float32, dev)
+    _require(out, "out", (B, H, T, DV), torch.float32, dev)
     o = out if out is not None else torch.empty(B, H, T, DV, device=dev, dtype=torch.float32)
-    _require(o, "out", (B, H, T, DV), torch.float32, dev)
     hf = None
     if output_final_state:
+        _require(final_out, "final_out", (B, H, DK, DV), torch.float32, dev)
         hf = final_out if final_out is not None else torch.empty(B, H, DK, DV, device=dev,
                                                                  dtype=torch.float32)
-        _require(hf, "final_out", (B, H, DK, DV), torch.float32, dev)
-    ws = workspace or gdn_workspace(B, H, T, C, DK, DV, q.dtype, dev)
+    stream = _hip.current_stream_handle(dev)
+    ws = workspace or _workspace(GdnWorkspace, B, H, T, C, DK, DV, code, dev, stream)
     sc = float(DK ** -0.5 if scale is None else scale)
-    lib = _hip.load()
-    st = lib.pf_gdn_exec(_hip.ptr(q), _hip.ptr(k), _hip.ptr(v), _hip.ptr(beta), _hip.ptr(g),
-                         _hip.ptr(h0), _hip.ptr(o), _hip.ptr(hf), B, H, T, C, DK, DV, code, sc,
-                         ws.handle, _hip.current_stream_handle(dev))
+    st = _hip.load().pf_gdn_exec(q.data_ptr(), k.data_ptr(), v.data_ptr(), beta.data_ptr(),
+                                 _hip.ptr(g), _hip.ptr(h0), o.data_ptr(), _hip.ptr(hf), B, H, T, C,
+                                 DK, DV, code, sc, ws.handle, stream)
     _hip.check("pf_gdn_exec", st)
     return o, hf
 
@@ -203,9 +217,8 @@ def kkt_inverse(k: torch.Tensor, g: Optional[torch.Tensor], beta: torch.Tensor,
     code = _dtype_code(k.dtype)
     if not k.is_contiguous():
         raise ValueError("k must be contiguous")
-    _require(beta.reshape(-1) if beta.is_contiguous() else beta, "beta", (n,), torch.float32, dev)
-    if g is not None:
-        _require(g.reshape(-1) if g.is_contiguous() else g, "g", (n,), torch.float32, dev)
+    _require_rows(beta, "beta", (n,), torch.float32, dev)
+    _require_rows(g, "g", (n,), torch.float32, dev)
     Tm = torch.empty(M, C, C, device=dev, dtype=torch.float32)
     A = torch.empty(M, C, C, device=dev, dtype=torch.float32) if return_A else None
     st = _hip.load().pf_kkt_inv_exec(_hip.ptr(k), _hip.ptr(g), _hip.ptr(beta), _hip.ptr(A),
@@ -254,13 +267,11 @@ def gated_qk(a: torch.Tensor, b: torch.Tensor, g: Optional[torch.Tensor] = None,
         raise ValueError(f"{n} rows do not split into chunks of {C} tokens x {H} heads")
     nc = n // (C * H)
     for name, t in (("a", a), ("b", b)):
-        _require(t.reshape(n, D) if t.is_contiguous() else t, name, (n, D), a.dtype, dev)
+        _require_rows(t, name, (n, D), a.dtype, dev)
     for name, t in (("a_scale", a_scale), ("b_scale", b_scale)):
-        if t is not None:
-            _require(t.reshape(n, D) if t.is_contiguous() else t, name, (n, D), torch.float32, dev)
+        _require_rows(t, name, (n, D), torch.float32, dev)
     for name, t in (("g", g), ("beta", beta)):
-        if t is not None:
-            _require(t.reshape(n) if t.is_contiguous() else t, name, (n,), torch.float32, dev)
+        _require_rows(t, name, (n,), torch.float32, dev)
     _require(mask, "mask", (C, C), torch.float32, dev)
     if out_dtype not in (torch.float32, torch.bfloat16):
         raise ValueError(f"out_dtype must be float32 or bfloat16, got {out_dtype}")
@@ -291,13 +302,11 @@ def qkv_flash(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: Optional[tor
         raise ValueError(f"{n} rows do not split into chunks of {C}")
     M = n // C
     for name, t in (("q", q), ("k", k), ("v", v)):
-        _require(t.reshape(n, D) if t.is_contiguous() else t, name, (n, D), q.dtype, dev)
+        _require_rows(t, name, (n, D), q.dtype, dev)
     for name, t in (("q_scale", q_scale), ("k_scale", k_scale)):
-        if t is not None:
-            _require(t.reshape(n, D) if t.is_contiguous() else t, name, (n, D), torch.float32, dev)
+        _require_rows(t, name, (n, D), torch.float32, dev)
     for name, t in (("g", g), ("beta", beta)):
-        if t is not None:
-            _require(t.reshape(n) if t.is_contiguous() else t, name, (n,), torch.float32, dev)
+        _require_rows(t, name, (n,), torch.float32, dev)
     o = torch.empty(M, C, D, device=dev, dtype=torch.float32)
     st = _hip.load().pf_qkv_flash_exec(
         _hip.ptr(q), _hip.ptr(k), _hip.ptr(v), _hip.ptr(q_scale), _hip.ptr(k_scale), _hip.ptr(g),
@@ -388,6 +397,7 @@ def kda_chunk_forward(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, beta: t
     dev = q.device
     if dev.type != "cuda":
         raise ValueError(f"q must be on a HIP device, got {dev}")
+    code = _dtype_code(q.dtype)
     _require(q, "q", (B, H, T, DK), q.dtype, dev)
     _require(k, "k", (B, H, T, DK), q.dtype, dev)
     _require(v, "v", (B, H, T, DV), q.dtype, dev)
@@ -396,18 +406,18 @@ def kda_chunk_forward(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, beta: t
         raise ValueError("g (the per-channel log decay [B,H,T,DK]) is required")
     _require(g, "g", (B, H, T, DK), torch.float32, dev)
     _require(h0, "h0", (B, H, DK, DV), torch.float32, dev)
+    _require(out, "out", (B, H, T, DV), torch.float32, dev)
     o = out if out is not None else torch.empty(B, H, T, DV, device=dev, dtype=torch.float32)
-    _require(o, "out", (B, H, T, DV), torch.float32, dev)
     hf = None
     if output_final_state:
+        _require(final_out, "final_out", (B, H, DK, DV), torch.float32, dev)
         hf = final_out if final_out is not None else torch.empty(B, H, DK, DV, device=dev,
                                                                  dtype=torch.float32)
-        _require(hf, "final_out", (B, H, DK, DV), torch.float32, dev)
-    ws = workspace or kda_workspace(B, H, T, C, DK, DV, q.dtype, dev)
+    stream = _hip.current_stream_handle(dev)
+    ws = workspace or _workspace(KdaWorkspace, B, H, T, C, DK, DV, code, dev, stream)
     sc = float(DK ** -0.5 if scale is None else scale)
-    lib = _hip.load()
-    st = lib.pf_kda_exec(_hip.ptr(q), _hip.ptr(k), _hip.ptr(v), _hip.ptr(beta), _hip.ptr(g),
-                         _hip.ptr(h0), _hip.ptr(o), _hip.ptr(hf), B, H, T, C, DK, DV,
-                         _dtype_code(q.dtype), sc, ws.handle, _hip.current_stream_handle(dev))
+    st = _hip.load().pf_kda_exec(q.data_ptr(), k.data_ptr(), v.data_ptr(), beta.data_ptr(),
+                                 g.data_ptr(), _hip.ptr(h0), o.data_ptr(), _hip.ptr(hf), B, H, T,
+                                 C, DK, DV, code, sc, ws.handle, stream)
     _hip.check("pf_kda_exec", st)
     return o, hf
