@@ -152,8 +152,15 @@ int pf_kda_exec(const void* q, const void* k, const void* v, const float* beta, 
   sa.BH = B * H;
   sa.NC = T / kChunk;
   constexpr int NLW = 4;
-  const unsigned grid = (unsigned)(B * H * (KD / 32));
-  pf::kda_scan_split_kernel<KC, KD, KD, NLW><<<dim3(grid), dim3(64 * (4 + NLW)), 0, s>>>(sa);
+  // 64-column slices where 32-column ones need a second generation of workgroups (one fits a CU): whole
+  // forward at 32 / 64 columns, 65 chains x 32 chunks 177 / 122 us, 96 x 32 181 / 150, 128 x 64
+  // 394 / 352, 512 x 8 238 / 206, but 64 x 64 203 / 228 and 32 x 128 283 / 343.  The same bits.
+  const bool wide = B * H * (KD / 32) > pf::device_cu_count();
+  const dim3 block(64 * (4 + NLW));
+  if (wide)
+    pf::kda_scan_split_kernel<KC, KD, KD, 4, NLW><<<dim3((unsigned)(B * H * (KD / 64))), block, 0, s>>>(sa);
+  else
+    pf::kda_scan_split_kernel<KC, KD, KD, 2, NLW><<<dim3((unsigned)(B * H * (KD / 32))), block, 0, s>>>(sa);
   return scope.status();
 }
 

@@ -2,7 +2,7 @@
 // split over four MFMA waves (one per SIMD) by token block and state row block, two workgroup
 // barriers per chunk.
 //
-// Workgroup = one chain bh x one slice of 32 state columns (NT = 2 column tiles of 16).  Stage 1
+// Workgroup = one chain bh x one slice of 32 or 64 state columns (NT = 2 or 4 column tiles of 16).  Stage 1
 // (kda_local_kernel) leaves per chunk the gated images W = T diag(beta) (k e^G),
 // TB = T diag(beta), QE = scale q e^G, KB = k e^-G and the chunk decay e^{G_last} per key
 // channel, so the recurrence needs no T r step:
@@ -41,7 +41,7 @@
 // the v tile row-major, the decay), W, v and the decay in the first phase, QE and KB in the
 // second.  TB has one LDS copy: it is read only in phase 1, so chunk c+1's TB is written in the
 // second phase of interval c.  The compute waves store their o rows
-// themselves: two 16-byte stores per lane, non-temporal, after lanes c and c + 8 swap the halves
+// themselves: NT 16-byte stores per lane, non-temporal, after lanes c and c + 8 swap the halves
 // of a token's 128-byte row so that every store instruction writes whole lines.
 #pragma once
 
@@ -55,7 +55,8 @@ template <int C, int DK, int NCOL>
 struct KdaSplitStage {
   static constexpr int KP = DK + 16;   // W, QE, KB rows: Swz<2,3>
   static constexpr int TP = C + 8;     // TB rows (the single copy outside the stage): Swz<3,1>
-  static constexpr int UP = NCOL + 8;  // v tile rows (row-major, read transposed)
+  // v tile rows (row-major, read transposed); 64-column rows are unpadded, which fits 160 KiB
+  static constexpr int UP = NCOL == 64 ? NCOL : NCOL + 8;
   bf16 ws[C * KP];
   bf16 qs[C * KP];
   bf16 ks[C * KP];
@@ -73,17 +74,17 @@ struct KdaSplitRegs {
   uint4 d;
 };
 
-template <int C, int DK, int DV, int NLW>
+template <int C, int DK, int DV, int NT, int NLW>
 __global__ __launch_bounds__(64 * (4 + NLW)) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void kda_scan_split_kernel(KdaScanArgs a) {
-  constexpr int NT = 2, NCOL = 16 * NT;
+  constexpr int NCOL = 16 * NT;
   using Stage = KdaSplitStage<C, DK, NCOL>;
   using Regs = KdaSplitRegs<NLW, NCOL>;
   constexpr int KP = Stage::KP, TP = Stage::TP, UP = Stage::UP;
   constexpr int NS = DV / NCOL;                 // slices per chain
   constexpr int FRAG = 64 * 8;                  // bf16 elements of one operand fragment
-  static_assert(C == 64 && DK == 128 && DV == 128 && NLW == 4,
-                "tile shapes of the KDA split scan kernel: C 64, DK = DV 128, 32 columns");
+  static_assert(C == 64 && DK == 128 && DV == 128 && (NT == 2 || NT == 4) && NLW == 4,
+                "tile shapes of the KDA split scan kernel: C 64, DK = DV 128, 32 or 64 columns");
 
   __shared__ __attribute__((aligned(16))) Stage st[2];
   __shared__ __attribute__((aligned(16))) bf16 TBs[C * TP];        // TB of the current chunk
@@ -357,25 +358,29 @@ void kda_scan_split_kernel(KdaScanArgs a) {
               OT[nt] = mfma_bf16(*reinterpret_cast<const bf16x8*>(VX + (kb * NT + nt) * FRAG + frag), pb, OT[nt]);
           }
         }
-        // lane (c, g) holds o[token tok0 + c][columns 16 nt + 4g .. +3]; a token's 32 columns
+        // lane (c, g) holds o[token tok0 + c][columns 16 nt + 4g .. +3]; 32 columns of a token
         // are one 128-byte line: lanes c and c + 8 of a row swap halves (DPP row rotate by 8) so
         // that each store instruction writes eight whole lines, tokens 0..7 then 8..15 of the
         // block, non-temporal (o is never read here)
         const bool hi = c >= 8;
-        floatx4 sa, sb;
 #pragma unroll
-        for (int ii = 0; ii < 4; ++ii) {
-          const float send = hi ? OT[0][ii] : OT[1][ii];
-          const float recv = __int_as_float(__builtin_amdgcn_update_dpp(
-              __float_as_int(send), __float_as_int(send), 0x128, 0xf, 0xf, false));   // row_ror:8
-          sa[ii] = hi ? recv : OT[0][ii];                // token c & 7, columns 16 hi + 4g ..
-          sb[ii] = hi ? OT[1][ii] : recv;                // token 8 + (c & 7), same columns
+        for (int p = 0; p < NT / 2; ++p) {
+          floatx4 sa, sb;
+#pragma unroll
+          for (int ii = 0; ii < 4; ++ii) {
+            const float v0 = OT[2 * p][ii], v1 = OT[2 * p + 1][ii];
+            const float send = hi ? v0 : v1;
+            const float recv = __int_as_float(__builtin_amdgcn_update_dpp(
+                __float_as_int(send), __float_as_int(send), 0x128, 0xf, 0xf, false));   // row_ror:8
+            sa[ii] = hi ? recv : v0;                     // token c & 7, columns 32 p + 16 hi + 4g ..
+            sb[ii] = hi ? v1 : recv;                     // token 8 + (c & 7), same columns
+          }
+          const uint32_t col = col0 + 32 * p + (hi ? 16 : 0) + 4 * g;
+          const uint32_t ra = (uint32_t)(((size_t)ch * C + tok0 + (c & 7)) * DV + col) * 4;
+          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, sa), ro, ra, 0, kCachePolicyNT);
+          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, sb), ro, ra + 8 * DV * 4, 0,
+                                                 kCachePolicyNT);
         }
-        const uint32_t col = col0 + (hi ? 16 : 0) + 4 * g;
-        const uint32_t ra = (uint32_t)(((size_t)ch * C + tok0 + (c & 7)) * DV + col) * 4;
-        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, sa), ro, ra, 0, kCachePolicyNT);
-        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, sb), ro, ra + 8 * DV * 4, 0,
-                                               kCachePolicyNT);
       }
       // S~ <- e^{G_last} (.) (S~ + KB^T v_new)  (the decay scales the state rows = key channels;
       // e^{G_last} KB^T is the (k e^{G_last - G})^T of the recurrence)

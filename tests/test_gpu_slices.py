@@ -1,12 +1,13 @@
 """The bf16 scan's column slices: 16, 32 and 64 columns, chosen by how many chains a call has.  A state
 column is computed the same way in all three, so a chain's outputs do not depend on how many chains
 run beside it: the first 40 and the first 8 of 72 chains give the same bits as within the 72, with
-every score-gate path, one chunk to five, and 72 and 69 chains (grouped by XCD and not)."""
+every score-gate path, one chunk to five, and 72 and 69 chains (grouped by XCD and not).  KDA likewise
+with its 32- and 64-column slices."""
 import pytest
 import torch
 
 from conftest import announce
-from pto_fuser_amd import gdn_chunk_forward
+from pto_fuser_amd import gdn_chunk_forward, kda_chunk_forward
 from pto_fuser_amd.forwards import make_delta_inputs
 
 pytestmark = pytest.mark.gpu
@@ -42,3 +43,19 @@ def test_a_chain_does_not_depend_on_its_neighbours(gate, H, T):
         on, hn = run(n)
         torch.cuda.synchronize()
         assert torch.equal(on, o[:, :n]) and torch.equal(hn, h[:, :n])
+
+
+@pytest.mark.parametrize("H,T", [(72, 64), (72, 192), (69, 320)])
+def test_a_kda_chain_does_not_depend_on_its_neighbours(H, T):
+    announce(f"KDA bf16 slices H{H} T{T}")
+    d = make_delta_inputs(1, H, T, kind="kda", dtype=torch.bfloat16, seed=H + T, h0_std=0.02, device=DEV)
+
+    def run(n):
+        x = {k: t[:, :n].contiguous() for k, t in d.items()}
+        return kda_chunk_forward(x["q"], x["k"], x["v"], x["beta"], x["g"], h0=x["h0"])
+
+    o, h = run(H)
+    on, hn = run(40)
+    torch.cuda.synchronize()
+    assert bool(torch.isfinite(o).all() and torch.isfinite(h).all())
+    assert torch.equal(on, o[:, :40]) and torch.equal(hn, h[:, :40])
