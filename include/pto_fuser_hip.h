@@ -128,7 +128,7 @@ int pf_gdn_scan_output_exec(const void* q, const void* k, const void* v, const f
  *   fp32 or NULL.  Supported: dtype PF_DTYPE_BF16 (bf16 MFMA) or PF_DTYPE_F32 (fp32
  *   operands and fp32 MFMA throughout), C = 64 or 128 (run as 64-token chunks),
  *   DK = DV = 128, T % C == 0, T <= 4 194 304.  The workspace holds the stage-1 images in the
- *   operand type.
+ *   operand type; bf16, few long chains: also the segments' state maps, used as by pf_gdn_exec.
  * ------------------------------------------------------------------------------------------ */
 size_t pf_kda_workspace_bytes(int B, int H, int T, int C, int DK, int DV, int dtype);
 void* pf_kda_setup(int B, int H, int T, int C, int DK, int DV, int dtype);

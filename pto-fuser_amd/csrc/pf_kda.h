@@ -283,6 +283,8 @@ struct KdaScanArgs {
   float* h_final;       // [BH, DK, DV] or null
   int BH;
   int NC;
+  const float* hseg;    // segmented chains, as ScanOutArgs: SEG segments of L chunks, segment s > 0 from
+  int SEG, L;           //   hseg[bh][s - 1]
 };
 
 }  // namespace pf

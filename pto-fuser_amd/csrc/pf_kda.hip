@@ -7,6 +7,7 @@
 #include "pf_kda.h"
 #include "pf_kda_scan.h"
 #include "pf_kda_f32.h"
+#include "pf_scan_args.h"
 #include "pf_status.h"
 #include "pf_workspace.h"
 
@@ -18,13 +19,59 @@ constexpr size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
 
 using KdaWorkspace = pf::Workspace;
 
+// How a chain of NC chunks is run: `seg` segments of `len` chunks (the last may have fewer).
+struct Segments {
+  int seg, len;
+};
+
+int generations(long wgs) { return (int)((wgs + pf::device_cu_count() - 1) / pf::device_cu_count()); }
+
+// Column slices of the bf16 scan, one workgroup per CU: 32 columns while four slices per unit (a chain
+// or a segment) fit one generation, else 64.  Whole forward at 32 / 64 columns: 65 chains x 32 chunks
+// 177 / 122 us, 96 x 32 181 / 150, 128 x 64 394 / 352, 512 x 8 238 / 206, but 64 x 64 203 / 228 and
+// 32 x 128 283 / 343.  The same bits.
+int slice_columns(long units) { return units * 4 <= pf::device_cu_count() ? 32 : 64; }
+
+// The scan's time: a chunk step of 1.25 us at 32 columns (1.8 at 64) alone on the chip and 0.4 (1.0) more
+// with every CU pulling its chunk images.
+double scan_us(long units, int chunks) {
+  const int cols = slice_columns(units);
+  const double wgs = (double)units * (128 / cols), full = wgs < pf::device_cu_count() ? wgs / pf::device_cu_count() : 1.0;
+  return (cols == 32 ? 1.25 + 0.4 * full : 1.8 + full) * chunks * generations((long)wgs);
+}
+
+// Segments of a bf16 chain, by the reasoning of gdn_segments: 2.3 us per chunk of a segment's map (only as
+// many segments as let every map run at once: more were never faster), 1.9 us per composition step,
+// 6 us for the launches, taken where that is 5 % ahead of whole chains.  Measured, whole forward, whole
+// chains against segments: 4 chains x 128 chunks 177 -> 83 us, 8 x 64 98 -> 70, 16 x 128 218 -> 152,
+// 24 x 128 258 -> 231, 32 x 256 555 -> 493, 1 x 128 170 -> 76; not taken: 32 x 64 (142, 142 in segments),
+// 16 x 32 (60, 61), 15 x 13 (32, 45).
+Segments kda_segments(int BH, int NC, int dtype) {
+  Segments best{1, NC};
+  if (dtype != PF_DTYPE_BF16 || NC < 16) return best;
+  double t = 0.95 * scan_us(BH, NC);
+  for (int want = 4; want <= 64 && want * 4 <= NC; want += want < 8 ? 2 : want / 4) {
+    const int len = (NC + want - 1) / want, seg = (NC + len - 1) / len;
+    if (!pf::seg_map_split(BH, seg)) break;
+    const double x = 6.0 + 2.3 * len + 1.9 * (seg - 2) + scan_us((long)BH * seg, len);
+    if (x < t) {
+      t = x;
+      best = {seg, len};
+    }
+  }
+  return best;
+}
+
 // Byte layout of the KDA workspace, M = B*H*T/C chunks:
 //   fp32 operands  [ W | U | QE | KR  (each M*C*128 fp32) | P (M*C*C fp32) | DEC (M*128 fp32) ]
-//   bf16 operands  [ W (M*C*128) | T diag(beta) (M*C*C) | QE | k e^-G (M*C*128 each) | DEC ]
+//   bf16 operands  [ W (M*C*128) | T diag(beta) (M*C*C) | QE | k e^-G (M*C*128 each) | DEC |
+//                    D, Mx (BH*(seg-1)*128*128 fp32 each; segmented chains only) ]
 // (bf16 stage 2 forms U and the score itself: nothing in P's place.)
 struct KdaLayout {
-  size_t w_off, u_off, q_off, k_off, p_off, d_off, total;
-  KdaLayout(size_t M, int C, int D, int dtype) {
+  size_t w_off, u_off, q_off, k_off, p_off, d_off, base, sd_off, sm_off, total;
+  KdaLayout(int BH, int NC, int dtype, Segments sg) {
+    constexpr size_t C = 64, D = 128;
+    const size_t M = (size_t)BH * NC;
     const bool b16 = dtype == PF_DTYPE_BF16;
     const size_t esize = b16 ? sizeof(bf16) : sizeof(float);
     const size_t tile = align256(M * C * D * esize);
@@ -35,9 +82,20 @@ struct KdaLayout {
     k_off = q_off + tile;
     p_off = k_off + tile;
     d_off = p_off + (b16 ? 0 : square);
-    total = d_off + align256(M * D * sizeof(float));
+    base = d_off + align256(M * D * sizeof(float));     // all an unsegmented run needs
+    sd_off = base;
+    sm_off = sd_off + (size_t)BH * (sg.seg - 1) * D * D * sizeof(float);
+    total = sm_off + (size_t)BH * (sg.seg - 1) * D * D * sizeof(float);
   }
 };
+
+// The workspace a shape asks for; the fp32 size is at least the bf16 one, as for GDN.
+size_t kda_workspace_total(int BH, int NC, int dtype) {
+  const size_t b16 = KdaLayout(BH, NC, PF_DTYPE_BF16, kda_segments(BH, NC, PF_DTYPE_BF16)).total;
+  if (dtype == PF_DTYPE_BF16) return b16;
+  const size_t f32 = KdaLayout(BH, NC, PF_DTYPE_F32, {1, NC}).total;
+  return f32 > b16 ? f32 : b16;
+}
 
 // bf16 operands (pf_kda.h) or fp32 operands (the fp32 kernels of pf_kda_f32.h); dk = dv = 128.
 // 64-token chunks in the kernels; a caller's chunk size of 128 runs them over T / 64 chunks (the
@@ -56,7 +114,7 @@ extern "C" {
 
 size_t pf_kda_workspace_bytes(int B, int H, int T, int C, int DK, int DV, int dtype) {
   if (!kda_shape_ok(B, H, T, C, DK, DV, dtype)) return 0;
-  return KdaLayout((size_t)B * H * (T / kChunk), kChunk, DK, dtype).total;
+  return kda_workspace_total(B * H, T / kChunk, dtype);
 }
 
 void* pf_kda_create(void) { return pf::workspace_create(); }
@@ -85,8 +143,11 @@ int pf_kda_exec(const void* q, const void* k, const void* v, const float* beta, 
   if (!kda_shape_ok(B, H, T, C, DK, DV, dtype)) return PF_ERR_ARG;
   const KdaWorkspace* w = static_cast<const KdaWorkspace*>(ws);
   const size_t M = (size_t)B * H * (T / kChunk);
-  const KdaLayout lay(M, kChunk, DK, dtype);
-  if (!w || !w->base || w->bytes < lay.total) return PF_ERR_WORKSPACE;
+  const int BH = B * H, NC = T / kChunk;
+  Segments sg = kda_segments(BH, NC, dtype);
+  if (!w || !w->base || w->bytes < KdaLayout(BH, NC, dtype, {1, NC}).base) return PF_ERR_WORKSPACE;
+  if (w->bytes < KdaLayout(BH, NC, dtype, sg).total) sg = {1, NC};   // a smaller buffer: whole chains
+  const KdaLayout lay(BH, NC, dtype, sg);
   if (!q || !k || !v || !beta || !g || !o) return PF_ERR_ARG;
   constexpr int KC = 64, KD = 128;
   char* base = static_cast<char*>(w->base);
@@ -139,7 +200,26 @@ int pf_kda_exec(const void* q, const void* k, const void* v, const float* beta, 
   const int st = scope.status();
   if (st != PF_OK) return st;
 
+  if (sg.seg > 1) {
+    pf::KdaSegMapArgs m{};
+    m.W = la.W;
+    m.TB = la.TB;
+    m.KB = la.KB;
+    m.v = static_cast<const bf16*>(v);
+    m.DEC = la.DEC;
+    m.h0 = h0;
+    m.D = reinterpret_cast<float*>(base + lay.sd_off);
+    m.M = reinterpret_cast<float*>(base + lay.sm_off);
+    m.BH = BH;
+    m.NC = NC;
+    m.SEG = sg.seg;
+    m.L = sg.len;
+    pf::kda_seg_states_launch(m, s);
+  }
   pf::KdaScanArgs sa{};
+  sa.hseg = reinterpret_cast<const float*>(base + lay.sd_off);
+  sa.SEG = sg.seg;
+  sa.L = sg.len;
   sa.W = la.W;
   sa.TB = la.TB;
   sa.v = static_cast<const bf16*>(v);
@@ -152,15 +232,11 @@ int pf_kda_exec(const void* q, const void* k, const void* v, const float* beta, 
   sa.BH = B * H;
   sa.NC = T / kChunk;
   constexpr int NLW = 4;
-  // 64-column slices where 32-column ones need a second generation of workgroups (one fits a CU): whole
-  // forward at 32 / 64 columns, 65 chains x 32 chunks 177 / 122 us, 96 x 32 181 / 150, 128 x 64
-  // 394 / 352, 512 x 8 238 / 206, but 64 x 64 203 / 228 and 32 x 128 283 / 343.  The same bits.
-  const bool wide = B * H * (KD / 32) > pf::device_cu_count();
-  const dim3 block(64 * (4 + NLW));
-  if (wide)
-    pf::kda_scan_split_kernel<KC, KD, KD, 4, NLW><<<dim3((unsigned)(B * H * (KD / 64))), block, 0, s>>>(sa);
-  else
-    pf::kda_scan_split_kernel<KC, KD, KD, 2, NLW><<<dim3((unsigned)(B * H * (KD / 32))), block, 0, s>>>(sa);
+  const long units = (long)BH * sg.seg;
+  const int cols = slice_columns(units);
+  const dim3 grid((unsigned)(units * (KD / cols))), block(64 * (4 + NLW));
+  if (cols == 64) pf::kda_scan_split_kernel<KC, KD, KD, 4, NLW><<<grid, block, 0, s>>>(sa);
+  else pf::kda_scan_split_kernel<KC, KD, KD, 2, NLW><<<grid, block, 0, s>>>(sa);
   return scope.status();
 }
 

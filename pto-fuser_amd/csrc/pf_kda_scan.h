@@ -2,7 +2,7 @@
 // split over four MFMA waves (one per SIMD) by token block and state row block, two workgroup
 // barriers per chunk.
 //
-// Workgroup = one chain bh x one slice of 32 or 64 state columns (NT = 2 or 4 column tiles of 16).  Stage 1
+// Workgroup = one chain bh (or one segment of it, pf_seg_scan.h) x one slice of 32 or 64 state columns (NT = 2 or 4 column tiles of 16).  Stage 1
 // (kda_local_kernel) leaves per chunk the gated images W = T diag(beta) (k e^G),
 // TB = T diag(beta), QE = scale q e^G, KB = k e^-G and the chunk decay e^{G_last} per key
 // channel, so the recurrence needs no T r step:
@@ -92,30 +92,32 @@ void kda_scan_split_kernel(KdaScanArgs a) {
   __shared__ __attribute__((aligned(16))) bf16 VX[2 * NT * FRAG];
   __shared__ __attribute__((aligned(16))) bf16 PX[3 * 64 * 4];   // P tiles (2,0) (3,0) (3,1)
 
-  int bh, slice;
+  int unit, slice;                              // unit: one segment of one chain
   const int bid = blockIdx.x;
-  if (a.BH % 8 == 0) {  // the slices of one chain share an XCD (dispatch is round-robin on XCDs)
+  if (a.BH * a.SEG % 8 == 0) {  // the slices of one unit share an XCD (dispatch is round-robin on XCDs)
     const int grp = bid / (8 * NS), within = bid % (8 * NS);
-    bh = grp * 8 + (within % 8);
+    unit = grp * 8 + (within % 8);
     slice = within / 8;
   } else {
-    bh = bid / NS;
+    unit = bid / NS;
     slice = bid % NS;
   }
+  const int bh = unit / a.SEG, seg = unit % a.SEG;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, g = lane >> 4, c = lane & 15;
-  const int NC = a.NC;
+  const int NC = min(a.L, a.NC - seg * a.L);    // this segment's chunks
   const int col0 = slice * NCOL;
   const uint32_t Tlen = (uint32_t)NC * C;
+  const size_t m0 = (size_t)bh * a.NC + (size_t)seg * a.L, t0 = m0 * C;   // its first chunk and token
 
   if (w >= 4) {
     // =========================== loader waves ===========================
     const int lt = tid - 256;                            // 0 .. 64*NLW-1
-    const __amdgpu_buffer_rsrc_t rw = make_rsrc(a.W + (size_t)bh * Tlen * DK, Tlen * DK * 2);
-    const __amdgpu_buffer_rsrc_t rq = make_rsrc(a.QE + (size_t)bh * Tlen * DK, Tlen * DK * 2);
-    const __amdgpu_buffer_rsrc_t rk = make_rsrc(a.KB + (size_t)bh * Tlen * DK, Tlen * DK * 2);
-    const __amdgpu_buffer_rsrc_t ru = make_rsrc(a.v + (size_t)bh * Tlen * DV, Tlen * DV * 2);
-    const __amdgpu_buffer_rsrc_t rtb = make_rsrc(a.TB + (size_t)bh * NC * C * C, (uint32_t)NC * C * C * 2);
-    const __amdgpu_buffer_rsrc_t rd = make_rsrc(a.DEC + (size_t)bh * NC * DK, (uint32_t)NC * DK * 4);
+    const __amdgpu_buffer_rsrc_t rw = make_rsrc(a.W + t0 * DK, Tlen * DK * 2);
+    const __amdgpu_buffer_rsrc_t rq = make_rsrc(a.QE + t0 * DK, Tlen * DK * 2);
+    const __amdgpu_buffer_rsrc_t rk = make_rsrc(a.KB + t0 * DK, Tlen * DK * 2);
+    const __amdgpu_buffer_rsrc_t ru = make_rsrc(a.v + t0 * DV, Tlen * DV * 2);
+    const __amdgpu_buffer_rsrc_t rtb = make_rsrc(a.TB + m0 * C * C, (uint32_t)NC * C * C * 2);
+    const __amdgpu_buffer_rsrc_t rd = make_rsrc(a.DEC + m0 * DK, (uint32_t)NC * DK * 4);
     // W / QE / KB rows (16 vectors of 8 per row): vec = lt & 15, a = lt >> 4; the vector index i
     // supplies the row bits that decide the swizzle's half swap, so the swap is compile-time:
     // row = a0 | a1<<1 | i0<<2 | a2<<3 | a3<<4 | i1<<5
@@ -225,7 +227,7 @@ void kda_scan_split_kernel(KdaScanArgs a) {
   } else {
     // =========================== compute waves ===========================
     const int cw = __builtin_amdgcn_readfirstlane(w);   // wave-uniform
-    const __amdgpu_buffer_rsrc_t ro = make_rsrc(a.o + (size_t)bh * Tlen * DV, Tlen * DV * 4);
+    const __amdgpu_buffer_rsrc_t ro = make_rsrc(a.o + t0 * DV, Tlen * DV * 4);
     const int tok0 = 16 * cw;                            // this wave's token block
     // per-lane LDS element offsets
     const int kq_rd = (tok0 + c) * KP + 4 * (g ^ ((c >> 2) & 3));          // W / QE rows
@@ -236,6 +238,8 @@ void kda_scan_split_kernel(KdaScanArgs a) {
     const int frag = lane * 8;                                             // lane's exchange slot
     const int xhalf = 4 * (cw & 1), xblk = cw >> 1;                        // this wave's VX slot
 
+    const float* h_in = seg ? a.hseg + ((size_t)bh * (a.SEG - 1) + seg - 1) * DK * DV
+                            : a.h0 ? a.h0 + (size_t)bh * DK * DV : nullptr;
     floatx4 S[2][NT];                                    // rows 32cw + 16r + 4g + i, column c
 #pragma unroll
     for (int r = 0; r < 2; ++r)
@@ -243,7 +247,7 @@ void kda_scan_split_kernel(KdaScanArgs a) {
       for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
         for (int ii = 0; ii < 4; ++ii)
-          S[r][nt][ii] = a.h0 ? a.h0[((size_t)bh * DK + 32 * cw + 16 * r + 4 * g + ii) * DV + col0 + 16 * nt + c] : 0.f;
+          S[r][nt][ii] = h_in ? h_in[(32 * cw + 16 * r + 4 * g + ii) * DV + col0 + 16 * nt + c] : 0.f;
     auto publish = [&]() {
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt)
@@ -406,7 +410,7 @@ void kda_scan_split_kernel(KdaScanArgs a) {
       publish();
       lds_barrier();                                     // B2
     }
-    if (a.h_final) {
+    if (a.h_final && seg == a.SEG - 1) {
 #pragma unroll
       for (int r = 0; r < 2; ++r)
 #pragma unroll

@@ -43,4 +43,18 @@ struct SegMapArgs {
 bool seg_map_split(int BH, int SEG);
 void seg_states_launch(const SegMapArgs& m, hipStream_t stream);
 
+// The same for the KDA forward (stage 1's images instead of k, T and the scalar gate).
+struct KdaSegMapArgs {
+  const bf16* W;        // [BH*NC, C, DK]
+  const bf16* TB;       // [BH*NC, C, C]
+  const bf16* KB;       // [BH*T, DK]
+  const bf16* v;        // [BH*T, DV]
+  const float* DEC;     // [BH*NC, DK]
+  const float* h0;      // [BH, DK, DV] or null
+  float* D;             // [BH, SEG - 1, DK, DV]
+  float* M;             // [BH, SEG - 1, DK, DK]
+  int BH, NC, SEG, L;
+};
+void kda_seg_states_launch(const KdaSegMapArgs& m, hipStream_t stream);
+
 }  // namespace pf

@@ -235,6 +235,150 @@ void seg_map_kernel(SegMapArgs a) {
       }
 }
 
+// The KDA form of seg_map_kernel: v_new = TB v - W S, S <- e^{G_last} (.) (S + KB^T v_new) over stage 1's
+// images (pf_kda.h); the organisation of NT = 1 (D or M of a segment per workgroup, 16 columns a wave), the
+// decay one factor per state row.  2.3-2.5 us a chunk step.  (32 columns a wave spill: the image is 114 KiB
+// and its prefetch half the registers.)
+struct KdaSegImage {
+  bf16 ws[64 * 128], ks[64 * 128], ts[64 * 64], vs[8 * 64 * 16];
+  float dec[128];
+};
+
+template <int C, int DK, int DV>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void kda_seg_map_kernel(KdaSegMapArgs a) {
+  static_assert(C == 64 && DK == 128 && DV == 128, "the forward's tile: C 64, dk = dv = 128");
+  __shared__ __attribute__((aligned(16))) KdaSegImage img[2];
+  const int bid = blockIdx.x;
+  const int unit = bid / 16 * 8 + bid % 8;             // D and M of a segment eight ids apart: one XCD
+  if (unit >= a.BH * (a.SEG - 1)) return;
+  const int bh = unit / (a.SEG - 1), seg = unit % (a.SEG - 1);
+  const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, c = lane & 15;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const bool map = bid % 16 >= 8;                      // M, else D
+  if (map && seg == 0) return;                         // the first segment's D is the state itself
+  const int col = 16 * w + c;                          // this lane's column
+  const unsigned vmask = map ? 0u : ~0u;
+  const size_t m0 = (size_t)bh * a.NC + (size_t)seg * a.L, t0 = m0 * C;
+
+  struct Regs {
+    u32x4 w[2], k[2], t, v[2];
+    floatx4 d;
+  };
+  auto load = [&](Regs& x, int ch) {
+    ch = min(ch, a.L - 1);                             // past the end: the last chunk again, unused
+    const size_t e = (t0 + (size_t)ch * C) * DK;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      x.w[i] = *reinterpret_cast<const u32x4*>(a.W + e + (tid + 512 * i) * 8);
+      x.k[i] = *reinterpret_cast<const u32x4*>(a.KB + e + (tid + 512 * i) * 8);
+      x.v[i] = *reinterpret_cast<const u32x4*>(a.v + e + (tid + 512 * i) * 8);
+    }
+    x.t = *reinterpret_cast<const u32x4*>(a.TB + (m0 + ch) * C * C + tid * 8);
+    x.d = *reinterpret_cast<const floatx4*>(a.DEC + (m0 + ch) * DK + 4 * (tid & 31));
+  };
+  auto store = [&](KdaSegImage& im, const Regs& x) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int u = tid + 512 * i, row = u >> 4, s = u & 15;
+      *reinterpret_cast<u32x4*>(im.ws + row * DK + 8 * seg_k_slot(row, s)) = x.w[i];
+      *reinterpret_cast<u32x4*>(im.ks + row * DK + 8 * seg_k_slot(row, s)) = x.k[i];
+      *reinterpret_cast<u32x4*>(im.vs + (s >> 1) * C * 16 + row * 16 + 8 * (s & 1)) = x.v[i];
+    }
+    *reinterpret_cast<u32x4*>(im.ts + (tid >> 3) * C + 8 * seg_t_slot(tid >> 3, tid & 7)) = x.t;
+    if (tid < 32) *reinterpret_cast<floatx4*>(im.dec + 4 * tid) = x.d;
+  };
+
+  floatx4 S[8];
+#pragma unroll
+  for (int r = 0; r < 8; ++r)
+#pragma unroll
+    for (int ii = 0; ii < 4; ++ii) S[r][ii] = map && seg_row(r, g, ii) == col ? 1.f : 0.f;
+  if (!map && seg == 0 && a.h0) {                      // one branch around all loads
+    const float* h = a.h0 + (size_t)bh * DK * DV + col;
+#pragma unroll
+    for (int r = 0; r < 8; ++r)
+#pragma unroll
+      for (int ii = 0; ii < 4; ++ii) S[r][ii] = h[seg_row(r, g, ii) * DV];
+  }
+
+  const int crow = 8 * (c >> 2) + (c & 3);             // + 32x + 4h: the row lane c supplies
+  const int trow = 8 * g + (c >> 2);                   // transposed reads: + 32x + 4h
+  Regs r0, r1;                                         // chunk m in set m & 1 until it is written to LDS
+  load(r0, 0);
+  load(r1, 1);
+  store(img[0], r0);
+  load(r0, 2);
+  lds_barrier();
+  auto chunk = [&](Regs& nx, int ch) {                 // nx holds chunk ch + 1
+    const KdaSegImage& im = img[ch & 1];
+    const bf16 *ws = im.ws, *ks = im.ks, *ts = im.ts, *vs = im.vs + w * C * 16;
+    bf16x8 Sb[4], Vt[2];
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb) Sb[kb] = pack8(S[2 * kb], S[2 * kb + 1]);
+    // v's tokens 32x + 8g .. +7 of this lane's column, zero for M
+#pragma unroll
+    for (int x = 0; x < 2; ++x) {
+      const bf16* vp = vs + (32 * x + trow) * 16 + 4 * (c & 3);
+      u32x4 vx = __builtin_bit_cast(u32x4, cat8(lds_read_tr(vp), lds_read_tr(vp + 4 * 16)));
+      vx &= u32x4{vmask, vmask, vmask, vmask};
+      Vt[x] = __builtin_bit_cast(bf16x8, vx);
+    }
+    // v_new = TB v - W S (TB lower triangular by 32-token blocks)
+    bf16x8 Vb[2];
+#pragma unroll
+    for (int x = 0; x < 2; ++x) {
+      floatx4 V[2];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        floatx4 Y = zero4(), U = zero4();
+        const int row = 32 * x + 4 * h + crow;
+#pragma unroll
+        for (int xb = 0; xb <= x; ++xb) {
+          const bf16x8 tf = *reinterpret_cast<const bf16x8*>(ts + row * C + 8 * seg_t_slot(row, 4 * xb + g));
+          U = mfma_bf16(tf, Vt[xb], U);
+        }
+#pragma unroll
+        for (int kb = 0; kb < 4; ++kb) {
+          const bf16x8 wf = *reinterpret_cast<const bf16x8*>(ws + row * DK + 8 * seg_k_slot(row, 4 * kb + g));
+          Y = mfma_bf16(wf, Sb[kb], Y);
+        }
+        V[h] = U - Y;
+      }
+      Vb[x] = pack8(V[0], V[1]);
+    }
+    store(img[(ch + 1) & 1], nx);                      // last read a barrier ago
+    load(nx, ch + 3);
+    // S <- e^{G_last} (.) (S + KB^T v_new)
+#pragma unroll
+    for (int r = 0; r < 8; ++r) {
+      const floatx4 d4 = *reinterpret_cast<const floatx4*>(im.dec + seg_row(r, g, 0));
+#pragma unroll
+      for (int x = 0; x < 2; ++x) {
+        const int r0 = 32 * x + trow, off = 8 * seg_k_slot(trow, 4 * (r >> 1) + (c & 3)) + 4 * (r & 1);
+        const bf16x8 kt = cat8(lds_read_tr(ks + r0 * DK + off), lds_read_tr(ks + (r0 + 4) * DK + off));
+        S[r] = mfma_bf16(kt, Vb[x], S[r]);
+      }
+      S[r] *= d4;
+    }
+    lds_barrier();                                     // the next image written, this one read
+  };
+  int ch = 0;
+  for (; ch + 1 < a.L; ch += 2) {
+    chunk(r1, ch);
+    chunk(r0, ch + 1);
+  }
+  if (ch < a.L) chunk(r1, ch);
+  float* out = (map ? a.M : a.D) + (size_t)unit * DK * DV;
+#pragma unroll
+  for (int r = 0; r < 8; ++r)
+#pragma unroll
+    for (int ii = 0; ii < 4; ++ii) {
+      const int row = seg_row(r, g, ii);
+      out[map ? seg_m_index(row, col) : row * DV + col] = S[r][ii];
+    }
+}
+
 // H_{s+1} = D_s + M_s H_s for s = 1 .. SEG - 2 (H_1 = D_0 is final), written over D_s.  One workgroup per
 // (chain, 16 columns); wave w forms rows 32w .. 32w+31 with fp32 products (two 16-row tiles, the
 // four-element K order of the D layout), its rows of M_s loaded a step ahead; H_s passes through LDS as

@@ -1,4 +1,4 @@
-"""Segmented chains of the bf16 GDN forward (few long chains): against the fp64 oracle where the segments
+"""Segmented chains of the bf16 GDN and KDA forwards (few long chains): against the fp64 oracle where the segments
 divide the chain and where the last one is shorter, with and without a gate and an initial state,
 against the same call on a workspace too small for segments (which runs whole chains), and with a
 NaN in one value column.  Bound of the forward tests: max abs 2e-2 on o and the final state."""
@@ -9,8 +9,8 @@ import pytest
 import torch
 
 from conftest import announce, record_error
-from oracle.gdn_oracle import gdn_reference
-from pto_fuser_amd import _hip, gdn_chunk_forward
+from oracle.gdn_oracle import gdn_reference, kda_reference
+from pto_fuser_amd import _hip, gdn_chunk_forward, kda_chunk_forward
 from pto_fuser_amd.forwards import as_oracle_inputs, make_delta_inputs
 
 pytestmark = pytest.mark.gpu
@@ -44,6 +44,28 @@ def test_segmented_forward(B, H, T, kind, h0_std):
     ro, rh = gdn_reference(x["q"], x["k"], x["v"], x["beta"], g, h0=x["h0"], C=64, dtype=np.float64)
     for name, got, ref in (("o", o, ro), ("h", h, rh)):
         e = record_error(f"segments {kind} B{B} H{H} T{T}", name, got.cpu().numpy(), ref, "max abs <= 0.02")
+        assert e["abs"] <= 2e-2, (name, e)
+
+
+@pytest.mark.parametrize("B,H,T,gate_scale,h0_std", [
+    (1, 1, 4096, 0.05, 0.02), (1, 2, 64 * 67, 0.3, None), (1, 3, 64 * 59, 0.002, 0.02)])
+def test_segmented_kda_forward(B, H, T, gate_scale, h0_std):
+    announce(f"segmented kda B{B} H{H} T{T} gate {gate_scale} h0={h0_std}")
+    lib = _hip.load()
+    chunks = B * H * T // 64                               # W, QE, KB, T diag(beta) and the decay
+    base = chunks * (3 * 64 * D * 2 + 64 * 64 * 2 + D * 4)
+    assert lib.pf_kda_workspace_bytes(B, H, T, 64, D, D, _hip.PF_DTYPE_BF16) > base + 4 * 256
+    inp = make_delta_inputs(B, H, T, kind="kda", dtype=torch.bfloat16, seed=T + H, h0_std=h0_std,
+                            gate_scale=gate_scale)
+    d = {n: (None if t is None else t.to(DEV)) for n, t in inp.items()}
+    o, h = kda_chunk_forward(d["q"], d["k"], d["v"], d["beta"], d["g"], h0=d["h0"])
+    o2, h2 = kda_chunk_forward(d["q"], d["k"], d["v"], d["beta"], d["g"], h0=d["h0"])
+    torch.cuda.synchronize()
+    assert torch.equal(o, o2) and torch.equal(h, h2)
+    x = as_oracle_inputs(inp)
+    ro, rh = kda_reference(x["q"], x["k"], x["v"], x["beta"], x["g"], h0=x["h0"], C=64, dtype=np.float64)
+    for name, got, ref in (("o", o, ro), ("h", h, rh)):
+        e = record_error(f"segments kda B{B} H{H} T{T}", name, got.cpu().numpy(), ref, "max abs <= 0.02")
         assert e["abs"] <= 2e-2, (name, e)
 
 
