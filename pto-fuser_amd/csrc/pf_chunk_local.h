@@ -150,10 +150,12 @@ __device__ __forceinline__ float quad_broadcast(float x, int p) {
 // block at its position — T_ii by the wave that has read all of A_ii, T10 / T32 by the wave
 // that just read A10 / A32, and T_LL a barrier after the X products read A_LL — and X lives in
 // the strictly-upper quadrant, which neither A nor T occupies.
+template <int GROUPS = 1>
 __device__ __forceinline__ void unit_lower_inverse64(float* As, float* Ts) {
   constexpr int CP = 64 + 4;
   const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, c = lane & 15;
-  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  if (GROUPS > 1) w &= 3;
   {  // wave w inverts diagonal block w: lane = column cc (of T) x row phase p (rows 4k + p)
     const int r = w, cc = lane >> 2, p = lane & 3;
     const float* Ab = As + (16 * r) * CP + 16 * r;
@@ -428,7 +430,7 @@ void chunk_local_kernel(ChunkLocalArgs a) {
 namespace pf {
 
 // Standalone opaque inverse: T = (I + A)^-1 for M strictly-lower C x C fp32 blocks (the upper
-// triangle and diagonal of A are ignored, as tril does).  One workgroup per block.
+// triangle and diagonal of A are ignored, as tril does).  One workgroup per block.  C <= 48.
 template <int C>
 __global__ __launch_bounds__(256) void tri_inv_kernel(const float* A, float* T, int M) {
   constexpr int CP = C + 4;
@@ -446,6 +448,77 @@ __global__ __launch_bounds__(256) void tri_inv_kernel(const float* A, float* T, 
   for (int e = tid; e < C * C; e += 256) {
     const int i = e / C, j = e % C;
     To[e] = (j <= i) ? Ts[i * CP + j] : 0.f;
+  }
+}
+
+// C = 64 and 128 on unit_lower_inverse64: 128 as [[T1, 0], [-T2 A21 T1, T2]], the two 64-row diagonal
+// blocks inverted side by side by four waves each, then X = A21 T1 and -T2 X, whose 16 x 16 tiles are dealt
+// two to a wave so that every wave has five products of each.  52 KB of LDS, three workgroups per CU;
+// A is read and T written in 16-byte vectors.  1024 blocks of 128: 22 us, 108 for the block-diagonal sweep
+// over two whole matrices in LDS (one workgroup per CU, 4-byte accesses); 4096 of 64: 20.5 us, 40.
+template <int C>
+__global__ __launch_bounds__(4 * C) void tri_inv_blocks_kernel(const float* A, float* T) {
+  static_assert(C == 64 || C == 128, "one or two 64-row diagonal blocks");
+  constexpr int CP = 64 + 4, NB = C / 64, MAT = 64 * CP;
+  __shared__ __attribute__((aligned(16))) float Ms[(NB == 2 ? 3 : 1) * MAT];   // A11, A22, A21
+  const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, c = lane & 15;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int blk = w >> 2, bt = tid & 255;                // diagonal block of this wave
+  const float* Ag = A + (size_t)blockIdx.x * C * C;
+  float* Tg = T + (size_t)blockIdx.x * C * C;
+  float* D = Ms + blk * MAT;
+  const size_t d0 = (size_t)(64 * blk) * C + 64 * blk;
+  const int r0 = bt >> 4, j0 = 4 * (bt & 15);            // rows r0 + 16 i, columns j0 .. j0+3
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int r = r0 + 16 * i;
+    floatx4 x = *reinterpret_cast<const floatx4*>(Ag + d0 + (size_t)r * C + j0);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) x[e] = j0 + e < r ? x[e] : 0.f;
+    *reinterpret_cast<floatx4*>(D + r * CP + j0) = x;
+  }
+  float* L = Ms + 2 * MAT;                               // A21, then X
+  if constexpr (NB == 2) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int r = (tid >> 4) + 32 * i;
+      *reinterpret_cast<floatx4*>(L + r * CP + j0) = *reinterpret_cast<const floatx4*>(Ag + (size_t)(64 + r) * C + j0);
+    }
+  }
+  lds_barrier();
+  unit_lower_inverse64<NB>(D, D);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int r = r0 + 16 * i;
+    floatx4 x = *reinterpret_cast<const floatx4*>(D + r * CP + j0);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) x[e] = j0 + e <= r ? x[e] : 0.f;   // above the diagonal: scratch
+    *reinterpret_cast<floatx4*>(Tg + d0 + (size_t)r * C + j0) = x;
+  }
+  if constexpr (NB == 2) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      *reinterpret_cast<floatx4*>(Tg + (size_t)((tid >> 4) + 32 * i) * C + 64 + j0) = zero4();
+    const int a = w >> 1, p0 = (w & 1) ? 1 : 0, p1 = (w & 1) ? 2 : 3;
+    floatx4 X[2];                                        // X tiles (a, p0), (a, p1): T1 lower triangular
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const int j = t ? p1 : p0;
+      X[t] = zero4();
+      for (int k = j; k < 4; ++k) X[t] = mm16<CP>(X[t], L, 16 * a, 16 * k, Ms, 16 * k, 16 * j, c, g);
+    }
+    lds_barrier();                                       // A21 is read: X takes its place
+#pragma unroll
+    for (int t = 0; t < 2; ++t) put16<CP>(L, 16 * a, 16 * (t ? p1 : p0), X[t], 1.f, c, g);
+    lds_barrier();
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {                        // tiles (p0, a), (p1, a) of -T2 X
+      const int i = t ? p1 : p0;
+      floatx4 Y = zero4();
+      for (int k = 0; k <= i; ++k) Y = mm16<CP>(Y, Ms + MAT, 16 * i, 16 * k, L, 16 * k, 16 * a, c, g);
+#pragma unroll
+      for (int ii = 0; ii < 4; ++ii) Tg[(size_t)(64 + 16 * i + 4 * g + ii) * C + 16 * a + c] = -Y[ii];
+    }
   }
 }
 
