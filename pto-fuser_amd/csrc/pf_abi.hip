@@ -200,9 +200,9 @@ void scan_output_launch(const void* q, const void* k, const void* v, const float
       default: pf::scan_split_kernel<C, DK, DV, 4, kSplitLoaderWaves><<<grid, block, 0, stream>>>(a); break;
     }
   } else {
-    // fp32: one workgroup per (chain, 16-column slice), every chunk split over four waves
+    // fp32: one workgroup per (chain, 16-column slice), every chunk split over eight waves
     // (pf_scan_split_f32.h)
-    pf::scan_split_f32_kernel<C, DK, DV><<<dim3((unsigned)(BH * (DV / 16))), dim3(256), 0, stream>>>(a);
+    pf::scan_split_f32_kernel<C, DK, DV><<<dim3((unsigned)(BH * (DV / 16))), dim3(512), 0, stream>>>(a);
   }
 }
 
