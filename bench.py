@@ -57,6 +57,7 @@ sys.path.insert(0, os.path.join(ROOT, "pto-fuser_amd"))
 sys.path.insert(0, ROOT)
 
 WORKLOAD = dict(B=4, H=16, T=4096, C=64, DK=128, DV=128)
+SCAN_THREADS = 512  # work items of a bf16 scan workgroup: four product waves, four loader waves
 SETTLE_S = 1.0      # untimed GPU work before the warmup steps (clock ramp)
 REPEATS = 5         # further runs of the timed loop, reported as a median beside `value`
 PEAK_HBM = 8.0e12          # MI355X HBM3E, bytes/s
@@ -135,15 +136,15 @@ def summarize_trace(trace_csv, lib_hash, out=None):
 
 def _counter_key(name, grid):
     """Record key of a dispatch in the counter passes: the headline's two kernels (the 32-column
-    scan and the 4096-chunk stage 1), the long-context secondary's two (the 16-column scan and
-    the 16384-chunk stage 1) and the KDA secondary's two; None for anything else (the other
+    scan and the 4096-chunk stage 1), the long-context secondary's two (the 64-column scan over
+    segments and the 16384-chunk stage 1) and the KDA secondary's two; None for anything else (the other
     secondaries, the calibration copies)."""
     W, L = WORKLOAD, LONG_WORKLOAD
     M = W["B"] * W["H"] * W["T"] // W["C"]
     ML = L["B"] * L["H"] * L["T"] // L["C"]
-    if "scan_split_kernel<64, 128, 128, 2," in name:
+    if "pf::scan_split_kernel<64, 128, 128, 2," in name:
         return "scan_output"
-    if "scan_split_kernel<64, 128, 128, 1," in name:
+    if "pf::scan_split_kernel<64, 128, 128, 4," in name:
         return "long_scan_output"
     bf16 = "DF16b" in name or "bf16" in name          # __bf16 as the demangler spells it
     if "chunk_local_kernel" in name and bf16 and grid == M * 256:
@@ -164,6 +165,7 @@ def summarize_counters(fetch_db, write_db, lib_hash, copy_mib, out=None):
     import sqlite3
     import statistics
     per, copy = {}, {}
+    long_grid = 0
     for counter, db in (("FETCH_SIZE", fetch_db), ("WRITE_SIZE", write_db)):
         con = sqlite3.connect(db)
         rows = con.execute("select kernel_name, grid_size, value from counters_collection "
@@ -177,6 +179,8 @@ def summarize_counters(fetch_db, write_db, lib_hash, copy_mib, out=None):
             key = _counter_key(name, grid)
             if key is not None:
                 vals.setdefault(key, []).append(v)
+            if key == "long_scan_output":
+                long_grid = grid
         for key, v in vals.items():
             per.setdefault(key, {})[counter] = round(statistics.mean(v), 2)
             per[key]["dispatches"] = len(v)
@@ -189,9 +193,13 @@ def summarize_counters(fetch_db, write_db, lib_hash, copy_mib, out=None):
     lmodel = stage_model(**{k: LONG_WORKLOAD[k] for k in ("B", "H", "T", "C", "DK", "DV")},
                          esize=2)
     h0_bytes = LONG_WORKLOAD["B"] * LONG_WORKLOAD["H"] * LONG_WORKLOAD["DK"] * LONG_WORKLOAD["DV"] * 4
+    # every segment of a chain reads the state it starts from: h0 or the composed one.  A segment is
+    # two workgroups (64 columns each) of SCAN_THREADS
+    segments = long_grid // (LONG_WORKLOAD["B"] * LONG_WORKLOAD["H"] * 2 * SCAN_THREADS)
     for k in ("chunk_local", "scan_output"):
         if "long_" + k in per:
-            model_bytes["long_" + k] = lmodel[k]["bytes"] + (h0_bytes if k == "scan_output" else 0)
+            model_bytes["long_" + k] = lmodel[k]["bytes"] + (
+                h0_bytes * segments if k == "scan_output" else 0)
     model_bytes.update({k: kda[k] for k in ("kda_local", "kda_scan") if k in per})
     rec = {"workload": "GDN forward B4 H16 T4096 C64 dk=dv=128, bf16 in (bench.py headline); "
                        "long-context GDN B1 H32 T32768 with h0 (long_*: bench.py "
@@ -319,7 +327,9 @@ def device_copy_GBps(mib: int = 256, reps: int = 20) -> float:
 
 
 def gdn_config_secondary(B, H, T, dtype_name, h0_std, steps, warmup, kind="gdn"):
-    """The fused forward at another configuration (GDN long context with h0; fp32 DeltaNet)."""
+    """The fused forward at another configuration (GDN long context with h0; fp32 DeltaNet).
+    ``bytes`` are those of the two stages over whole chains: what a chain in segments reads again
+    for its maps and moves as states (profiles/hbm_traffic_gdn_forward.md) is left out."""
     import torch
     from pto_fuser_amd.forwards import make_delta_inputs
     from pto_fuser_amd.ops import gdn_chunk_forward, gdn_workspace
