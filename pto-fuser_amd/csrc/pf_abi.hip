@@ -172,6 +172,7 @@ void scan_output_launch(const void* q, const void* k, const void* v, const float
   a.hseg = reinterpret_cast<const float*>(base + lay.d_off);
   a.SEG = sg.seg;
   a.L = sg.len;
+  a.h0_stride = DK * DV;
   if constexpr (std::is_same<E, bf16>::value) {
     if (sg.seg > 1) {
       pf::SegMapArgs m{};
@@ -187,7 +188,12 @@ void scan_output_launch(const void* q, const void* k, const void* v, const float
       m.NC = NC;
       m.SEG = sg.seg;
       m.L = sg.len;
+      m.keep_h0 = h0 && h0 == h_final;
       pf::seg_states_launch(m, stream);
+      if (m.keep_h0) {
+        a.h0 = m.M;
+        a.h0_stride = (size_t)(sg.seg - 1) * DK * DK;
+      }
     }
     const int units = BH * sg.seg;
     // bf16: one workgroup per (segment or whole chain, column slice); four MFMA waves split

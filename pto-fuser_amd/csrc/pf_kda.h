@@ -285,6 +285,7 @@ struct KdaScanArgs {
   int NC;
   const float* hseg;    // segmented chains, as ScanOutArgs: SEG segments of L chunks, segment s > 0 from
   int SEG, L;           //   hseg[bh][s - 1]
+  size_t h0_stride;
 };
 
 }  // namespace pf

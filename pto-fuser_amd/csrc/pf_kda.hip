@@ -200,6 +200,9 @@ int pf_kda_exec(const void* q, const void* k, const void* v, const float* beta, 
   const int st = scope.status();
   if (st != PF_OK) return st;
 
+  pf::KdaScanArgs sa{};
+  sa.h0 = h0;
+  sa.h0_stride = KD * KD;
   if (sg.seg > 1) {
     pf::KdaSegMapArgs m{};
     m.W = la.W;
@@ -214,9 +217,13 @@ int pf_kda_exec(const void* q, const void* k, const void* v, const float* beta, 
     m.NC = NC;
     m.SEG = sg.seg;
     m.L = sg.len;
+    m.keep_h0 = h0 && h0 == h_final;
     pf::kda_seg_states_launch(m, s);
+    if (m.keep_h0) {
+      sa.h0 = m.M;
+      sa.h0_stride = (size_t)(sg.seg - 1) * KD * KD;
+    }
   }
-  pf::KdaScanArgs sa{};
   sa.hseg = reinterpret_cast<const float*>(base + lay.sd_off);
   sa.SEG = sg.seg;
   sa.L = sg.len;
@@ -226,7 +233,6 @@ int pf_kda_exec(const void* q, const void* k, const void* v, const float* beta, 
   sa.QE = la.QE;
   sa.KB = la.KB;
   sa.DEC = la.DEC;
-  sa.h0 = h0;
   sa.o = o;
   sa.h_final = h_final;
   sa.BH = B * H;

@@ -21,9 +21,11 @@ struct ScanOutArgs {
   int NC;               // chunks per chain
   const float* scale;   // device scalar: the output scale (written by stage 1)
   // segmented chains (bf16): each chain runs as SEG segments of L chunks (the last may have fewer),
-  // segment s > 0 from the state hseg[bh][s - 1]; SEG = 1, L = NC otherwise
+  // segment s > 0 from the state hseg[bh][s - 1]; SEG = 1, L = NC otherwise.  h0_stride: elements between
+  // two chains' h0 (DK * DV, or more where h0 is the maps' copy of it)
   const float* hseg;    // [BH, SEG - 1, DK, DV]
   int SEG, L;
+  size_t h0_stride;
 };
 
 // Arguments of the segmented chains' first two steps (pf_seg_scan.h) and their launch (pf_seg.hip).
@@ -35,9 +37,11 @@ struct SegMapArgs {
   const bf16* Tm;       // [M, C, C] (I + A)^-1, from stage 1
   const float* h0;      // [BH, DK, DV] or null
   float* D;             // [BH, SEG - 1, DK, DV]
-  float* M;             // [BH, SEG - 1, DK, DK]   (segment 0's is not written)
+  float* M;             // [BH, SEG - 1, DK, DK]   (segment 0's slot: the copy of h0, or not written)
   int BH, NC;           // chains, chunks per chain
   int SEG, L;           // segments per chain, chunks per segment (the last may have fewer)
+  int keep_h0;          // copy h0 to M's slots of segment 0: the final state is written over h0 itself, by
+                        // another workgroup than the one that starts from it
 };
 // D and M of a segment in workgroups of their own (the shorter chunk step), while those fit one generation.
 bool seg_map_split(int BH, int SEG);
@@ -53,7 +57,7 @@ struct KdaSegMapArgs {
   const float* h0;      // [BH, DK, DV] or null
   float* D;             // [BH, SEG - 1, DK, DV]
   float* M;             // [BH, SEG - 1, DK, DK]
-  int BH, NC, SEG, L;
+  int BH, NC, SEG, L, keep_h0;
 };
 void kda_seg_states_launch(const KdaSegMapArgs& m, hipStream_t stream);
 

@@ -351,7 +351,7 @@ void scan_split_kernel(ScanOutArgs a) {
     const int xhalf = 4 * (cw & 1), xblk = cw >> 1;                        // this wave's RX/VX slot
 
     const float* h_in = seg ? a.hseg + ((size_t)bh * (a.SEG - 1) + seg - 1) * DK * DV
-                            : a.h0 ? a.h0 + (size_t)bh * DK * DV : nullptr;
+                            : a.h0 ? a.h0 + (size_t)bh * a.h0_stride : nullptr;
     floatx4 S[2][NT];                                    // rows 32cw + 16r + 4g + i, column c
 #pragma unroll
     for (int r = 0; r < 2; ++r)

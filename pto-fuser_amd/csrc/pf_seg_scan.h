@@ -123,6 +123,15 @@ void seg_map_kernel(SegMapArgs a) {
       for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
         for (int ii = 0; ii < 4; ++ii) S[r][nt][ii] = h[seg_row(r, g, ii) * DV + 16 * nt];
+    if (a.keep_h0) {
+      float* keep = a.M + (size_t)unit * DK * DK + col;
+#pragma unroll
+      for (int r = 0; r < 8; ++r)
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+          for (int ii = 0; ii < 4; ++ii) keep[seg_row(r, g, ii) * DV + 16 * nt] = S[r][nt][ii];
+    }
   }
 
   const int crow = 8 * (c >> 2) + (c & 3);             // + 32x + 4h: the row lane c supplies
@@ -300,6 +309,13 @@ void kda_seg_map_kernel(KdaSegMapArgs a) {
     for (int r = 0; r < 8; ++r)
 #pragma unroll
       for (int ii = 0; ii < 4; ++ii) S[r][ii] = h[seg_row(r, g, ii) * DV];
+    if (a.keep_h0) {
+      float* keep = a.M + (size_t)unit * DK * DK + col;
+#pragma unroll
+      for (int r = 0; r < 8; ++r)
+#pragma unroll
+        for (int ii = 0; ii < 4; ++ii) keep[seg_row(r, g, ii) * DV] = S[r][ii];
+    }
   }
 
   const int crow = 8 * (c >> 2) + (c & 3);             // + 32x + 4h: the row lane c supplies

@@ -106,3 +106,20 @@ def test_nan_stays_in_its_column_and_behind_its_token():
     assert not bad[0, 1].any() and not bad[0, 0, :tok // 64 * 64].any()
     others = [c for c in range(D) if c != col]
     assert not bad[0, 0][:, others].any() and not torch.isnan(h)[0, 0][:, others].any()
+
+
+@pytest.mark.parametrize("op,B,H,T", [
+    ("gdn", 1, 9, 64 * 97), ("gdn", 4, 5, 64 * 107), ("kda", 1, 2, 64 * 67), ("kda", 1, 10, 64 * 65)])
+def test_state_updated_in_place(op, B, H, T):
+    """final_out is h0 itself: the first segment starts from h0 in one workgroup while the last segment's
+    writes the final state over it, so the call keeps a copy of h0.  The same bits as with two tensors, in
+    both map layouts (9 and 20 chains) and at both KDA slice widths."""
+    announce(f"in-place state, segmented {op} B{B} H{H} T{T}")
+    d = make_delta_inputs(B, H, T, kind=op, dtype=torch.bfloat16, seed=T + H, h0_std=0.5, device=DEV)
+    fn = gdn_chunk_forward if op == "gdn" else kda_chunk_forward
+    o, h = fn(d["q"], d["k"], d["v"], d["beta"], d["g"], h0=d["h0"])
+    state = d["h0"].clone()
+    o2, h2 = fn(d["q"], d["k"], d["v"], d["beta"], d["g"], h0=state, final_out=state)
+    torch.cuda.synchronize()
+    assert h2.data_ptr() == state.data_ptr()
+    assert torch.equal(o, o2) and torch.equal(h, h2)
