@@ -122,9 +122,17 @@ void scan_split_kernel(ScanOutArgs a) {
     unit = bid / NS;
     slice = bid % NS;
   }
-  const int bh = unit / a.SEG, seg = unit % a.SEG;
+  int bh = unit, seg = 0, NC = a.NC;            // NC: this segment's chunks
+  if (a.SEG > 1) {
+    bh = unit / a.SEG;
+    seg = unit % a.SEG;
+    // a chain whose maps left fp32 range (seg_compose_kernel) is run whole, by its first unit
+    const float mark =
+        a.hseg[((size_t)bh * (a.SEG - 1) + a.SEG - 2) * DK * DV + slice * NCOL + (threadIdx.x & (NCOL - 1))];
+    if (!__any(!__builtin_isfinite(mark))) NC = min(a.L, a.NC - seg * a.L);
+    else if (seg) return;
+  }
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, g = lane >> 4, c = lane & 15;
-  const int NC = min(a.L, a.NC - seg * a.L);    // this segment's chunks
   const int col0 = slice * NCOL;
   const uint32_t Tlen = (uint32_t)NC * C;
   const size_t m0 = (size_t)bh * a.NC + (size_t)seg * a.L, t0 = m0 * C;   // its first chunk and token
@@ -583,7 +591,7 @@ void scan_split_kernel(ScanOutArgs a) {
       publish();
       lds_barrier();                                     // B3
     }
-    if (a.h_final && seg == a.SEG - 1) {
+    if (a.h_final && seg * a.L + NC == a.NC) {           // this unit ran the chain's last chunk
 #pragma unroll
       for (int r = 0; r < 2; ++r)
 #pragma unroll

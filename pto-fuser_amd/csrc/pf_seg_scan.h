@@ -399,11 +399,17 @@ void kda_seg_map_kernel(KdaSegMapArgs a) {
 // (chain, 16 columns); wave w forms rows 32w .. 32w+31 with fp32 products (two 16-row tiles, the
 // four-element K order of the D layout), its rows of M_s loaded a step ahead; H_s passes through LDS as
 // D tiles.
+//
+// A segment's map can leave fp32 range where the states it is applied to do not (they are zero, or small):
+// then Inf * 0 is NaN.  A state that is not finite stays so in every row of its column through the later
+// products, so the last one shows it; its row 0 is set to NaN in all of the slice's columns, which is
+// where the scan looks before it splits the chain.
 template <int DK, int DV>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
 void seg_compose_kernel(float* D, const float* M, int BH, int SEG) {
   constexpr int NS = DV / 16;
   __shared__ __attribute__((aligned(16))) floatx4 H[2][8 * 64];
+  __shared__ int bad[4];
   // the slices of one chain on one XCD: they read the same M
   const int bh = (blockIdx.x / (8 * NS)) * 8 + blockIdx.x % 8, col0 = 16 * (blockIdx.x % (8 * NS) / 8);
   if (bh >= BH) return;
@@ -437,6 +443,7 @@ void seg_compose_kernel(float* D, const float* M, int BH, int SEG) {
     H[1][(2 * w + r) * 64 + lane] = x;
   }
   lds_barrier();
+  floatx4 last[2];                                     // this wave's rows of the newest state
   auto step = [&](Step& x, int s) {
     const floatx4* h = H[s & 1];
     floatx4 acc[2][2] = {{x.d[0], zero4()}, {x.d[1], zero4()}}, hv[8];
@@ -455,6 +462,7 @@ void seg_compose_kernel(float* D, const float* M, int BH, int SEG) {
     for (int r = 0; r < 2; ++r) {
       const floatx4 y = acc[r][0] + acc[r][1];
       H[(s + 1) & 1][(2 * w + r) * 64 + lane] = y;
+      last[r] = y;
 #pragma unroll
       for (int ii = 0; ii < 4; ++ii) Dc[((size_t)s * DK + 32 * w + 16 * r + 4 * g + ii) * DV] = y[ii];
     }
@@ -469,6 +477,16 @@ void seg_compose_kernel(float* D, const float* M, int BH, int SEG) {
   }
   if (s < SEG - 1) step(st[0], s);
   if (s + 1 < SEG - 1) step(st[1], s + 1);
+  bool off = false;
+#pragma unroll
+  for (int r = 0; r < 2; ++r)
+#pragma unroll
+    for (int ii = 0; ii < 4; ++ii) off = off || !__builtin_isfinite(last[r][ii]);
+  const bool any_off = __any(off);
+  if (lane == 0) bad[w] = any_off;
+  lds_barrier();
+  if (w == 0 && g == 0 && (bad[0] | bad[1] | bad[2] | bad[3]))
+    Dc[(size_t)(SEG - 2) * DK * DV] = __builtin_nanf("");   // row 0, which this lane stored
 }
 
 }  // namespace pf

@@ -10,7 +10,7 @@ import torch
 
 from conftest import announce, record_error
 from oracle.gdn_oracle import gdn_reference, kda_reference
-from pto_fuser_amd import _hip, gdn_chunk_forward, kda_chunk_forward
+from pto_fuser_amd import _hip, gdn_chunk_forward, kda_chunk_forward, ops
 from pto_fuser_amd.forwards import as_oracle_inputs, make_delta_inputs
 
 pytestmark = pytest.mark.gpu
@@ -123,3 +123,34 @@ def test_state_updated_in_place(op, B, H, T):
     torch.cuda.synchronize()
     assert h2.data_ptr() == state.data_ptr()
     assert torch.equal(o, o2) and torch.equal(h, h2)
+
+
+def _forward(op, d, whole=False, **kw):
+    """The forward; ``whole`` runs it on a workspace made for as many one-chunk chains, which has no
+    room for segments."""
+    fn, cls = (gdn_chunk_forward, ops.GdnWorkspace) if op == "gdn" else (kda_chunk_forward, ops.KdaWorkspace)
+    B, H, T, _ = d["q"].shape
+    ws = cls(B, H * T // 64, 64, 64, D, D, _hip.PF_DTYPE_BF16, DEV) if whole else None
+    out = fn(d["q"], d["k"], d["v"], d["beta"], d["g"], h0=d["h0"], workspace=ws, **kw)
+    torch.cuda.synchronize()
+    return out
+
+
+@pytest.mark.parametrize("op,B,H,T", [("gdn", 1, 2, 64 * 256), ("kda", 1, 2, 64 * 64), ("kda", 1, 10, 64 * 65)])
+def test_maps_outside_fp32_range(op, B, H, T):
+    """A segment's map overflows (long keys make the recurrence grow by about e^15 per chunk; KDA: gates
+    that rise by e^16 per chunk) while the state it is applied to is exactly zero: v is zero up to the
+    last two chunks.  The chain is then run whole: finite, and the whole chain's bits."""
+    announce(f"segment maps outside fp32 range {op} B{B} H{H} T{T}")
+    d = make_delta_inputs(B, H, T, kind=op, dtype=torch.bfloat16, seed=T, device=DEV)
+    d["v"][:, :, :T - 128] = 0
+    if op == "gdn":
+        d["k"] = (d["k"].float() * 5).bfloat16()
+    else:
+        d["g"].fill_(0.25)
+    assert d["h0"] is None
+    o, h = _forward(op, d)
+    assert bool(torch.isfinite(o).all() and torch.isfinite(h).all())
+    assert bool((o[:, :, :T - 128] == 0).all()) and float(o.abs().max()) > 0
+    wo, wh = _forward(op, d, whole=True)
+    assert torch.equal(o, wo) and torch.equal(h, wh)
