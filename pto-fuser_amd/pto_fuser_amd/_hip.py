@@ -124,9 +124,9 @@ def ptr(t) -> Optional[int]:
 
 
 def current_stream_handle(device=None) -> int:
-    """The current stream's hipStream_t.  Every launch asks for it, so for a device with an index
-    the handle is read directly, without the Stream object torch.cuda.current_stream builds."""
-    index = getattr(device, "index", None)
-    if index is None:
-        return torch.cuda.current_stream(device).cuda_stream
-    return torch._C._cuda_getCurrentRawStream(index)
+    """The current stream's hipStream_t.  Every launch asks for it, so for a HIP ``torch.device`` with
+    an index the handle is read directly, without the Stream object torch.cuda.current_stream builds;
+    whatever else names a device (a string, an index, None) goes through that."""
+    if isinstance(device, torch.device) and device.type == "cuda" and device.index is not None:
+        return torch._C._cuda_getCurrentRawStream(device.index)
+    return torch.cuda.current_stream(device).cuda_stream

@@ -7,6 +7,7 @@ import os
 import re
 
 import pytest
+import torch
 
 from pto_fuser_amd import _build, _hip
 
@@ -209,3 +210,22 @@ def test_ops_validate_on_host():
         kda_chunk_forward(qb.half(), qb.half(), qb.half(), torch.zeros(1, 1, 128), gk)
     with pytest.raises(ValueError, match="multiple of the chunk size"):
         kda_chunk_forward(qb[:, :, :96], qb[:, :, :96], qb[:, :, :96], torch.zeros(1, 1, 96), gk[:, :, :96])
+
+
+@pytest.mark.parametrize("device", [None, 0, "cuda", "cuda:0", torch.device("cuda"), torch.device("cuda:0")])
+def test_stream_handle_of_every_device_form(monkeypatch, device):
+    """A device given as a string or an index names the same stream as the torch.device does; a CPU device
+    with an index does not pass for the GPU of that index."""
+    class Stream:
+        cuda_stream = 7
+
+    def current_stream(dev=None):
+        if dev is not None and not isinstance(dev, int) and torch.device(dev).type != "cuda":
+            raise ValueError(f"Expected a cuda device, but got: {dev}")
+        return Stream
+
+    monkeypatch.setattr(torch.cuda, "current_stream", current_stream)
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda index: 7 + int(index), raising=False)
+    assert _hip.current_stream_handle(device) == 7
+    with pytest.raises(ValueError):
+        _hip.current_stream_handle(torch.device("cpu", 0))
