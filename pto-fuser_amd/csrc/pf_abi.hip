@@ -14,12 +14,14 @@
 #include "pf_scan_args.h"
 #include "pf_scan_split.h"
 #include "pf_scan_split_f32.h"
+#include "pf_segments.h"
 
 namespace {
 
 constexpr int kSplitLoaderWaves = 4;   // loader waves of the bf16 split scan kernel
 
 using pf::bf16;
+using pf::Segments;
 
 using GdnWorkspace = pf::Workspace;
 
@@ -28,50 +30,6 @@ constexpr size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
 size_t elem_size(int dtype) { return dtype == PF_DTYPE_BF16 ? 2 : 4; }
 
 bool valid_dtype(int dtype) { return dtype == PF_DTYPE_F32 || dtype == PF_DTYPE_BF16; }
-
-// How a chain of NC chunks is run: `seg` segments of `len` chunks (the last may have fewer).
-struct Segments {
-  int seg, len;
-};
-
-int generations(long wgs) { return (int)((wgs + pf::device_cu_count() - 1) / pf::device_cu_count()); }
-
-// Column slices of the bf16 scan, one workgroup per CU: 16 columns (a chunk step of 1.2 us) while eight
-// slices per unit fit one generation of workgroups, 32 (1.45 us) while four do, else 64 (2.0-2.3 us,
-// half the workgroups of 32 and half their reads of k, q and T).  Whole forward at 16 / 32 / 64 columns:
-// 32 chains x 128 chunks 176 / 193 / 272 us, 64 x 64 178 / 113 / 150, 65 x 64 339 / 250 / 150,
-// 96 x 64 265 / 207 / 160, 128 x 64 349 / 240 / 194, 192 x 32 283 / 180 / 164, 512 x 8 235 / 157 / 116.
-// The three give the same bits.
-int slice_columns(long units) {
-  const int cus = pf::device_cu_count();
-  return units * 8 <= cus ? 16 : units * 4 <= cus ? 32 : 64;
-}
-double scan_us(long units, int chunks) {
-  const int cols = slice_columns(units);
-  return (cols == 16 ? 1.2 : cols == 32 ? 1.45 : 2.25) * chunks * generations(units * (128 / cols));
-}
-
-// Segments of a bf16 chain.  A chain's time is its chunk count while chains leave CUs idle; in
-// segments it is the segment's length twice (its map, 2.45 or 3.35 us per chunk step, and the scan) plus a composition step of 1.9 us per segment, and 9 us for the two more launches.  The
-// times are per generation of workgroups, as measured; segments are taken where they come out 10 %
-// ahead.  Measured, whole forward, one chain against its segments: 4 chains x 512 chunks 577 -> 157 us,
-// 8 x 256 300 -> 132, 16 x 128 160 -> 119, 8 x 64 82 -> 59, 1 x 128 147 -> 68, 2 x 32 44 -> 42; not taken:
-// 32 x 128 (173, 190 in segments), 15 x 23 (37, 53), 32 x 512 (666, 693).
-Segments gdn_segments(int BH, int NC, int dtype) {
-  Segments best{1, NC};
-  if (dtype != PF_DTYPE_BF16 || NC < 16) return best;
-  double t = 0.9 * scan_us(BH, NC);
-  for (int want = 4; want <= 64 && want * 4 <= NC; want += want < 8 ? 2 : want / 4) {
-    const int len = (NC + want - 1) / want, seg = (NC + len - 1) / len;
-    const double map = pf::seg_map_split(BH, seg) ? 2.45 * len : 3.35 * len * generations((long)BH * (seg - 1));
-    const double x = 9.0 + map + 1.9 * (seg - 2) + scan_us((long)BH * seg, len);
-    if (x < t) {
-      t = x;
-      best = {seg, len};
-    }
-  }
-  return best;
-}
 
 // Byte layout of the fused-forward workspace, M = BH * NC chunks:
 //   [ T (M*C*C E) | P (M*C*C E, pre-scaled; fp32 only) | G (M*C fp32) | output scale (fp32, 256 B) |
@@ -94,10 +52,10 @@ struct GdnLayout {
   }
 };
 
-// The workspace a shape asks for.  The fp32 size is at least the bf16 one, so that a handle reserved
-// for fp32 serves both types of a shape without growing.
+// The workspace a shape asks for: arithmetic, for an MI355X, whatever device is present.  The fp32 size is
+// at least the bf16 one, so that a handle reserved for fp32 serves both types of a shape without growing.
 size_t gdn_workspace_total(int BH, int NC, int dtype) {
-  const size_t b16 = GdnLayout(BH, NC, PF_DTYPE_BF16, gdn_segments(BH, NC, PF_DTYPE_BF16)).total;
+  const size_t b16 = GdnLayout(BH, NC, PF_DTYPE_BF16, pf::gdn_segments(BH, NC, pf::kCus)).total;
   if (dtype == PF_DTYPE_BF16) return b16;
   const size_t f32 = GdnLayout(BH, NC, PF_DTYPE_F32, {1, NC}).total;
   return f32 > b16 ? f32 : b16;
@@ -152,7 +110,8 @@ void scan_output_launch(const void* q, const void* k, const void* v, const float
                        char* base, size_t bytes, hipStream_t stream) {
   constexpr int C = 64, DK = 128, DV = 128;
   constexpr int dtype = std::is_same<E, bf16>::value ? PF_DTYPE_BF16 : PF_DTYPE_F32;
-  Segments sg = gdn_segments(BH, NC, dtype);
+  Segments sg{1, NC};
+  if (dtype == PF_DTYPE_BF16) sg = pf::gdn_segments(BH, NC, pf::device_cu_count());
   if (GdnLayout(BH, NC, dtype, sg).total > bytes) sg = {1, NC};   // a smaller buffer: whole chains
   const GdnLayout lay(BH, NC, dtype, sg);
   pf::ScanOutArgs a{};
@@ -198,7 +157,7 @@ void scan_output_launch(const void* q, const void* k, const void* v, const float
     const int units = BH * sg.seg;
     // bf16: one workgroup per (segment or whole chain, column slice); four MFMA waves split
     // every chunk (pf_scan_split.h)
-    const int cols = slice_columns(units);
+    const int cols = pf::gdn_slice_columns(units, pf::device_cu_count());
     const dim3 grid((unsigned)(units * (DV / cols))), block(64 * (4 + kSplitLoaderWaves));
     switch (cols) {
       case 16: pf::scan_split_kernel<C, DK, DV, 1, kSplitLoaderWaves><<<grid, block, 0, stream>>>(a); break;

@@ -8,6 +8,7 @@
 #include "pf_kda_scan.h"
 #include "pf_kda_f32.h"
 #include "pf_scan_args.h"
+#include "pf_segments.h"
 #include "pf_status.h"
 #include "pf_workspace.h"
 
@@ -18,49 +19,7 @@ using pf::bf16;
 constexpr size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
 
 using KdaWorkspace = pf::Workspace;
-
-// How a chain of NC chunks is run: `seg` segments of `len` chunks (the last may have fewer).
-struct Segments {
-  int seg, len;
-};
-
-int generations(long wgs) { return (int)((wgs + pf::device_cu_count() - 1) / pf::device_cu_count()); }
-
-// Column slices of the bf16 scan, one workgroup per CU: 32 columns while four slices per unit (a chain
-// or a segment) fit one generation, else 64.  Whole forward at 32 / 64 columns: 65 chains x 32 chunks
-// 177 / 122 us, 96 x 32 181 / 150, 128 x 64 394 / 352, 512 x 8 238 / 206, but 64 x 64 203 / 228 and
-// 32 x 128 283 / 343.  The same bits.
-int slice_columns(long units) { return units * 4 <= pf::device_cu_count() ? 32 : 64; }
-
-// The scan's time: a chunk step of 1.25 us at 32 columns (1.8 at 64) alone on the chip and 0.4 (1.0) more
-// with every CU pulling its chunk images.
-double scan_us(long units, int chunks) {
-  const int cols = slice_columns(units);
-  const double wgs = (double)units * (128 / cols), full = wgs < pf::device_cu_count() ? wgs / pf::device_cu_count() : 1.0;
-  return (cols == 32 ? 1.25 + 0.4 * full : 1.8 + full) * chunks * generations((long)wgs);
-}
-
-// Segments of a bf16 chain, by the reasoning of gdn_segments: 2.3 us per chunk of a segment's map (only as
-// many segments as let every map run at once: more were never faster), 1.9 us per composition step,
-// 6 us for the launches, taken where that is 5 % ahead of whole chains.  Measured, whole forward, whole
-// chains against segments: 4 chains x 128 chunks 177 -> 83 us, 8 x 64 98 -> 70, 16 x 128 218 -> 152,
-// 24 x 128 258 -> 231, 32 x 256 555 -> 493, 1 x 128 170 -> 76; not taken: 32 x 64 (142, 142 in segments),
-// 16 x 32 (60, 61), 15 x 13 (32, 45).
-Segments kda_segments(int BH, int NC, int dtype) {
-  Segments best{1, NC};
-  if (dtype != PF_DTYPE_BF16 || NC < 16) return best;
-  double t = 0.95 * scan_us(BH, NC);
-  for (int want = 4; want <= 64 && want * 4 <= NC; want += want < 8 ? 2 : want / 4) {
-    const int len = (NC + want - 1) / want, seg = (NC + len - 1) / len;
-    if (!pf::seg_map_split(BH, seg)) break;
-    const double x = 6.0 + 2.3 * len + 1.9 * (seg - 2) + scan_us((long)BH * seg, len);
-    if (x < t) {
-      t = x;
-      best = {seg, len};
-    }
-  }
-  return best;
-}
+using pf::Segments;
 
 // Byte layout of the KDA workspace, M = B*H*T/C chunks:
 //   fp32 operands  [ W | U | QE | KR  (each M*C*128 fp32) | P (M*C*C fp32) | DEC (M*128 fp32) ]
@@ -91,7 +50,7 @@ struct KdaLayout {
 
 // The workspace a shape asks for; the fp32 size is at least the bf16 one, as for GDN.
 size_t kda_workspace_total(int BH, int NC, int dtype) {
-  const size_t b16 = KdaLayout(BH, NC, PF_DTYPE_BF16, kda_segments(BH, NC, PF_DTYPE_BF16)).total;
+  const size_t b16 = KdaLayout(BH, NC, PF_DTYPE_BF16, pf::kda_segments(BH, NC, pf::kCus)).total;
   if (dtype == PF_DTYPE_BF16) return b16;
   const size_t f32 = KdaLayout(BH, NC, PF_DTYPE_F32, {1, NC}).total;
   return f32 > b16 ? f32 : b16;
@@ -144,7 +103,8 @@ int pf_kda_exec(const void* q, const void* k, const void* v, const float* beta, 
   const KdaWorkspace* w = static_cast<const KdaWorkspace*>(ws);
   const size_t M = (size_t)B * H * (T / kChunk);
   const int BH = B * H, NC = T / kChunk;
-  Segments sg = kda_segments(BH, NC, dtype);
+  Segments sg{1, NC};
+  if (dtype == PF_DTYPE_BF16) sg = pf::kda_segments(BH, NC, pf::device_cu_count());
   if (!w || !w->base || w->bytes < KdaLayout(BH, NC, dtype, {1, NC}).base) return PF_ERR_WORKSPACE;
   if (w->bytes < KdaLayout(BH, NC, dtype, sg).total) sg = {1, NC};   // a smaller buffer: whole chains
   const KdaLayout lay(BH, NC, dtype, sg);
@@ -239,7 +199,7 @@ int pf_kda_exec(const void* q, const void* k, const void* v, const float* beta, 
   sa.NC = T / kChunk;
   constexpr int NLW = 4;
   const long units = (long)BH * sg.seg;
-  const int cols = slice_columns(units);
+  const int cols = pf::kda_slice_columns(units, pf::device_cu_count());
   const dim3 grid((unsigned)(units * (KD / cols))), block(64 * (4 + NLW));
   if (cols == 64) pf::kda_scan_split_kernel<KC, KD, KD, 4, NLW><<<grid, block, 0, s>>>(sa);
   else pf::kda_scan_split_kernel<KC, KD, KD, 2, NLW><<<grid, block, 0, s>>>(sa);

@@ -43,8 +43,6 @@ struct SegMapArgs {
   int keep_h0;          // copy h0 to M's slots of segment 0: the final state is written over h0 itself, by
                         // another workgroup than the one that starts from it
 };
-// D and M of a segment in workgroups of their own (the shorter chunk step), while those fit one generation.
-bool seg_map_split(int BH, int SEG);
 void seg_states_launch(const SegMapArgs& m, hipStream_t stream);
 
 // The same for the KDA forward (stage 1's images instead of k, T and the scalar gate).

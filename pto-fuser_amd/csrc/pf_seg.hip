@@ -3,11 +3,10 @@
 #include <hip/hip_runtime.h>
 
 #include "pf_seg_scan.h"
+#include "pf_segments.h"
 #include "pf_status.h"
 
 namespace pf {
-
-bool seg_map_split(int BH, int SEG) { return BH * (2 * SEG - 3) <= device_cu_count(); }
 
 namespace {
 void compose_launch(float* D, const float* M, int BH, int SEG, hipStream_t stream) {
@@ -18,7 +17,7 @@ void compose_launch(float* D, const float* M, int BH, int SEG, hipStream_t strea
 
 void seg_states_launch(const SegMapArgs& m, hipStream_t stream) {
   const unsigned units = (unsigned)(m.BH * (m.SEG - 1));
-  if (seg_map_split(m.BH, m.SEG))
+  if (seg_map_split(m.BH, m.SEG, device_cu_count()))
     seg_map_kernel<64, 128, 128, 1><<<dim3((units + 7) / 8 * 16), dim3(512), 0, stream>>>(m);
   else
     seg_map_kernel<64, 128, 128, 2><<<dim3(units), dim3(512), 0, stream>>>(m);

@@ -11,7 +11,7 @@
 //
 // Step 1 repeats the state part of the chunk loop on 256 columns instead of 128, so segments pay
 // where chains leave the chip idle or their length is the bound, not where every CU is busy
-// (gdn_segments in pf_abi.hip has the rule and its measurements).
+// (pf_segments.h has the rule and its measurements).
 //
 // seg_map_kernel: state columns are independent, so a wave owns 16 NT of them for the whole segment and
 // every product feeds the next from registers: S (packed pairs of D tiles) is the B operand of k S,

@@ -5,6 +5,8 @@ launches a kernel."""
 import glob
 import os
 import re
+import subprocess
+import sys
 
 import pytest
 import torch
@@ -95,6 +97,23 @@ def test_gdn_workspace_of_segmented_chains():
     for B, H, T in ((1, 1, 64), (1, 1, 1024), (1, 4, 1 << 15), (1, 8, 4096), (2, 5, 5120), (4, 16, 4096),
                     (1, 1, 1 << 22), (1, 32, 1 << 15)):
         assert size(B, H, T, _hip.PF_DTYPE_F32) >= size(B, H, T, _hip.PF_DTYPE_BF16) > 0
+
+
+def test_workspace_sizes_start_no_runtime(lib):
+    """Sizes are arithmetic: a process that only asks for them (before it forks, say) does not start the HIP
+    runtime.  Every HIP call is logged at this level; the last one is there to show that."""
+    code = ("import ctypes, sys\n"
+            "lib = ctypes.CDLL(sys.argv[1])\n"
+            "for f in (lib.pf_gdn_workspace_bytes, lib.pf_kda_workspace_bytes):\n"
+            "    f.restype, f.argtypes = ctypes.c_size_t, [ctypes.c_int] * 7\n"
+            "    assert f(1, 4, 32768, 64, 128, 128, 0) >= f(1, 4, 32768, 64, 128, 128, 1) > 0\n"
+            "print('sized', file=sys.stderr, flush=True)\n"
+            "lib.hipGetDeviceCount(ctypes.byref(ctypes.c_int()))\n")
+    run = subprocess.run([sys.executable, "-c", code, _hip.lib_path()], capture_output=True, text=True,
+                         env={**os.environ, "AMD_LOG_LEVEL": "3"}, timeout=120)
+    assert run.returncode == 0, run.stderr[-2000:]
+    before, after = run.stderr.split("sized", 1)
+    assert "hipGetDevice" in after and "hip" not in before, before[-2000:]
 
 
 @pytest.mark.parametrize("B,H,T,C", [(1, 1, 64, 64), (4, 16, 4096, 64), (1, 32, 32768, 128),
