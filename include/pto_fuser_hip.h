@@ -67,8 +67,10 @@ size_t pf_gdn_workspace_bytes(int B, int H, int T, int C, int DK, int DV, int dt
 void* pf_gdn_setup(int B, int H, int T, int C, int DK, int DV, int dtype);
 /* The same workspace in two steps, for a registry whose setup takes no arguments (the
  * reference's FusedKernel calls setup_sym() bare, fused.py:102-107): pf_gdn_create returns an
- * empty handle (allocates nothing); pf_gdn_reserve grows it to the shape's size (PF_OK, PF_ERR_ARG
- * for an unsupported shape, PF_ERR_ALLOC).  A reserve that does not grow allocates nothing and is
+ * empty handle (allocates nothing); pf_gdn_reserve grows it to the shape's size if it does not
+ * hold what the shape's whole chains need, which rises with the number of chunks (PF_OK, PF_ERR_ARG
+ * for an unsupported shape, PF_ERR_ALLOC): a handle never grows for segments alone, and where it has no
+ * room for them the call runs whole chains.  A reserve that does not grow allocates nothing and is
  * safe under HIP graph capture; one that grows waits for the device and must run outside it.
  * Growing frees the old buffer: a HIP graph captured on the handle before a growth still
  * addresses it and must be captured again.  The fp32 size of a shape covers its bf16 size, so

@@ -264,7 +264,8 @@ void* pf_gdn_create(void) { return pf::workspace_create(); }
 int pf_gdn_reserve(void* ws, int B, int H, int T, int C, int DK, int DV, int dtype) {
   const size_t bytes = pf_gdn_workspace_bytes(B, H, T, C, DK, DV, dtype);
   if (bytes == 0) return PF_ERR_ARG;
-  return pf::workspace_reserve(static_cast<GdnWorkspace*>(ws), bytes);
+  const int NC = T / kChunk;
+  return pf::workspace_reserve(static_cast<GdnWorkspace*>(ws), GdnLayout(B * H, NC, dtype, {1, NC}).base, bytes);
 }
 
 void* pf_gdn_setup(int B, int H, int T, int C, int DK, int DV, int dtype) {

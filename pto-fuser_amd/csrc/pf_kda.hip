@@ -81,7 +81,8 @@ void* pf_kda_create(void) { return pf::workspace_create(); }
 int pf_kda_reserve(void* ws, int B, int H, int T, int C, int DK, int DV, int dtype) {
   const size_t bytes = pf_kda_workspace_bytes(B, H, T, C, DK, DV, dtype);
   if (bytes == 0) return PF_ERR_ARG;
-  return pf::workspace_reserve(static_cast<KdaWorkspace*>(ws), bytes);
+  const int NC = T / kChunk;
+  return pf::workspace_reserve(static_cast<KdaWorkspace*>(ws), KdaLayout(B * H, NC, dtype, {1, NC}).base, bytes);
 }
 
 void* pf_kda_setup(int B, int H, int T, int C, int DK, int DV, int dtype) {

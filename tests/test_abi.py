@@ -116,6 +116,42 @@ def test_workspace_sizes_start_no_runtime(lib):
     assert "hipGetDevice" in after and "hip" not in before, before[-2000:]
 
 
+_FAKE_HIP = """#include <stdlib.h>
+int mallocs, frees;
+int hipMalloc(void** p, size_t n) { ++mallocs; *p = malloc(1); return 0; }
+int hipFree(void* p) { ++frees; free(p); return 0; }
+int hipDeviceSynchronize(void) { return 0; }
+"""
+
+
+@pytest.mark.parametrize("op", ["gdn", "kda"])
+def test_a_shape_of_fewer_chunks_never_grows_a_handle(lib, tmp_path, op):
+    """After a reserve for the most chunks a caller uses, a reserve for fewer allocates and frees nothing, also
+    where those chains would run in segments and a fresh handle of theirs is larger: a graph captured
+    on the handle keeps its buffer.  The library's allocations are counted in a process of its own."""
+    src, so = tmp_path / "fake.c", tmp_path / "fake.so"
+    src.write_text(_FAKE_HIP)
+    subprocess.run(["gcc", "-shared", "-fPIC", str(src), "-o", str(so)], check=True)
+    code = f"""
+import ctypes, sys
+fake = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+lib = ctypes.CDLL(sys.argv[2])
+size, reserve, create = lib.pf_{op}_workspace_bytes, lib.pf_{op}_reserve, lib.pf_{op}_create
+size.restype, size.argtypes = ctypes.c_size_t, [ctypes.c_int] * 7
+reserve.argtypes, create.restype = [ctypes.c_void_p] + [ctypes.c_int] * 7, ctypes.c_void_p
+count = lambda: (ctypes.c_int.in_dll(fake, "mallocs").value, ctypes.c_int.in_dll(fake, "frees").value)
+ws = create()
+large, small = (1, 64, 64 * 32, 64, 128, 128, 1), (1, 4, 64 * 500, 64, 128, 128, 1)
+assert size(*small) > size(*large), "the shape of fewer chunks is the larger workspace"
+assert reserve(ws, *large) == 0 and count() == (1, 0), count()
+assert reserve(ws, *small) == 0 and count() == (1, 0), count()
+assert reserve(ws, 1, 64, 64 * 64, 64, 128, 128, 1) == 0 and count() == (2, 1), count()
+"""
+    run = subprocess.run([sys.executable, "-c", code, str(so), _hip.lib_path()], capture_output=True, text=True,
+                         timeout=120)
+    assert run.returncode == 0, run.stderr[-2000:]
+
+
 @pytest.mark.parametrize("B,H,T,C", [(1, 1, 64, 64), (4, 16, 4096, 64), (1, 32, 32768, 128),
                                      (3, 5, 192, 64)])
 def test_fp32_workspace_holds_bf16(lib, B, H, T, C):
