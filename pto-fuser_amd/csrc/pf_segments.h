@@ -63,30 +63,34 @@ inline Segments best_segments(int NC, double limit, Time&& time) {
 
 // Segments of a bf16 GDN chain.  A chain's time is its chunk count while chains leave CUs idle; in
 // segments it is the segment's length twice (its map, 2.45 or 3.35 us per chunk step, and the scan) plus a
-// composition step of 1.9 us per segment, and 9 us for the two more launches.  The times are per
-// generation of workgroups, as measured; segments are taken where they come out 10 % ahead.  Measured, whole
-// forward, one chain against its segments: 4 chains x 512 chunks 577 -> 157 us, 8 x 256 300 -> 132,
-// 16 x 128 160 -> 119, 8 x 64 82 -> 59, 1 x 128 147 -> 68, 2 x 32 44 -> 42; not taken: 32 x 128 (173, 190 in
-// segments), 15 x 23 (37, 53), 32 x 512 (666, 693).
+// composition step of 1.9 us per segment, 9 us for the two more launches, and what short segments of
+// many chains lose at their starts (2 us per chain and chunk of length).  No more segments than let every
+// map run in one generation of workgroups, which also bounds their states and maps to 128 KiB per CU.  They
+// are taken where they come out 5 % ahead.  Whole forward, whole chains and the segments taken (us):
+//   1 chain x 128 chunks 149, 69;  4 x 512 578, 153;  8 x 64 82, 60;  8 x 256 301, 128;  16 x 128 160, 109;
+//   32 x 512 692, 567;  1 x 32 42.7, 40.6;  20 x 96 125, 104
+// and what the segments would have taken where chains stay whole:
+//   12 x 40 55.2, 56.4;  33 x 192 286, 311;  64 x 256 434, 552
 inline Segments gdn_segments(int BH, int NC, int cus) {
-  return best_segments(NC, 0.9 * gdn_scan_us(BH, NC, cus), [&](Segments s) {
-    const double map = seg_map_split(BH, s.seg, cus)
-                           ? 2.45 * s.len
-                           : 3.35 * s.len * generations((long)BH * (s.seg - 1), cus);
-    return 9.0 + map + 1.9 * (s.seg - 2) + gdn_scan_us((long)BH * s.seg, s.len, cus);
+  return best_segments(NC, 0.95 * gdn_scan_us(BH, NC, cus), [&](Segments s) {
+    if ((long)BH * (s.seg - 1) > cus) return -1.0;
+    const double map = (seg_map_split(BH, s.seg, cus) ? 2.45 : 3.35) * s.len;
+    return 9.0 + 2.0 * BH / s.len + map + 1.9 * (s.seg - 2) + gdn_scan_us((long)BH * s.seg, s.len, cus);
   });
 }
 
-// Segments of a bf16 KDA chain, by the same reasoning: 2.3 us per chunk of a segment's map (only as many
-// segments as let every map run at once: more were never faster), 1.9 us per composition step, 6 us
-// for the launches, taken where that is 5 % ahead of whole chains.  Measured, whole forward, whole chains
-// against segments: 4 chains x 128 chunks 177 -> 83 us, 8 x 64 98 -> 70, 16 x 128 218 -> 152, 24 x 128
-// 258 -> 231, 32 x 256 555 -> 493, 1 x 128 170 -> 76; not taken: 32 x 64 (142, 142 in segments), 16 x 32
-// (60, 61), 15 x 13 (32, 45).
+// Segments of a bf16 KDA chain, by the same reasoning: 2.3 us per chunk of a segment's map (D and M in
+// workgroups of their own, and only as many segments as let those run at once: more were never faster),
+// 10 us for the launches, taken where that is ahead of whole chains.  Whole forward, whole chains and the
+// segments taken (us):
+//   1 chain x 128 chunks 168, 76;  4 x 128 176, 84;  8 x 64 98, 71;  16 x 128 220, 154;  24 x 128 258, 232;
+//   32 x 256 555, 497
+// and what the segments would have taken where chains stay whole:
+//   9 x 24 45.7, 50.1;  16 x 32 59.8, 62.9;  32 x 64 142, 143
 inline Segments kda_segments(int BH, int NC, int cus) {
-  return best_segments(NC, 0.95 * kda_scan_us(BH, NC, cus), [&](Segments s) {
+  return best_segments(NC, kda_scan_us(BH, NC, cus), [&](Segments s) {
     if (!seg_map_split(BH, s.seg, cus)) return -1.0;
-    return 6.0 + 2.3 * s.len + 1.9 * (s.seg - 2) + kda_scan_us((long)BH * s.seg, s.len, cus);
+    return 10.0 + 2.0 * BH / s.len + 2.3 * s.len + 1.9 * (s.seg - 2) + kda_scan_us((long)BH * s.seg, s.len, cus);
   });
 }
 

@@ -116,6 +116,35 @@ def test_workspace_sizes_start_no_runtime(lib):
     assert "hipGetDevice" in after and "hip" not in before, before[-2000:]
 
 
+def _segments(lib, op, chains, chunks):
+    """Segments per chain that the workspace of a bf16 shape holds (1: whole chains)."""
+    size = lib.pf_gdn_workspace_bytes if op == "gdn" else lib.pf_kda_workspace_bytes
+    extra = size(1, chains, 64 * chunks, 64, 128, 128, 1) - size(1, chains * chunks, 64, 64, 128, 128, 1)
+    assert extra % (chains * 2 * 128 * 128 * 4) == 0
+    return 1 + extra // (chains * 2 * 128 * 128 * 4)
+
+
+@pytest.mark.parametrize("op,chains,chunks,segmented", [
+    ("gdn", 1, 128, True), ("gdn", 4, 512, True), ("gdn", 8, 64, True), ("gdn", 8, 256, True),
+    ("gdn", 16, 128, True), ("gdn", 32, 512, True), ("gdn", 1, 32, True), ("gdn", 20, 96, True),
+    ("gdn", 12, 40, False), ("gdn", 33, 192, False), ("gdn", 64, 256, False), ("gdn", 15, 23, False),
+    ("kda", 1, 128, True), ("kda", 4, 128, True), ("kda", 8, 64, True), ("kda", 16, 128, True),
+    ("kda", 24, 128, True), ("kda", 32, 256, True),
+    ("kda", 9, 24, False), ("kda", 8, 28, False), ("kda", 16, 32, False), ("kda", 32, 64, False)])
+def test_chains_run_in_segments_where_that_was_faster(lib, op, chains, chunks, segmented):
+    """The rule's decisions at shapes measured both ways (the times are beside the rule)."""
+    assert (_segments(lib, op, chains, chunks) > 1) == segmented
+
+
+def test_segment_states_are_bounded(lib):
+    """The segments' states and maps never take more than 32 MiB (GDN) or 16 MiB (KDA) beside what whole
+    chains need: their maps run in one generation of workgroups."""
+    for op, mib in (("gdn", 32), ("kda", 16)):
+        for chains in (1, 3, 8, 16, 17, 36, 64, 100, 132, 256, 300):
+            for chunks in (16, 67, 128, 500, 512, 5040, 65536):
+                assert (_segments(lib, op, chains, chunks) - 1) * chains * 2 * 128 * 128 * 4 <= mib << 20
+
+
 _FAKE_HIP = """#include <stdlib.h>
 int mallocs, frees;
 int hipMalloc(void** p, size_t n) { ++mallocs; *p = malloc(1); return 0; }
