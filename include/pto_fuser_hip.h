@@ -86,9 +86,10 @@ void pf_gdn_teardown(void* ws);
 /* The same forward with no workspace argument and no allocation of any kind: no counterpart in
  * the reference.  It is for callers that cannot allocate device memory (code under HIP graph
  * capture, tight serving loops, harnesses that forbid allocation).  Its workspace is a
- * file-scope device array of 40 MiB (bf16: up to 4 964 chunks of 64 tokens, the B4 H16 T4096
- * headline included; fp32: up to 1 270); a larger input returns PF_ERR_SCRATCH and launches
- * nothing.  The array's device address is looked up once per device on the first call there
+ * file-scope device array: 40 MiB for what whole chains need (bf16: up to 4 964 chunks of 64 tokens,
+ * the B4 H16 T4096 headline included; fp32: up to 1 270) and 32 MiB for the states and maps of
+ * segments, so that the call gives the bits of pf_gdn_exec on a workspace of its shape; a larger input
+ * returns PF_ERR_SCRATCH and launches nothing.  The array's device address is looked up once per device on the first call there
  * (make that call outside any graph capture).  Every call on one GPU shares that GPU's array:
  * calls that overlap on one GPU (different streams, or threads) race; serialise them.  Same
  * arguments as pf_gdn_exec otherwise. */

@@ -197,10 +197,14 @@ int gdn_check(int B, int H, int T, int C, int DK, int DV, int dtype, const void*
 }
 
 // ---- the allocation-free forward ---------------------------------------------------------
-// Its workspace is this file-scope array, 40 MiB: the bf16 headline shape (B4 H16 T4096, 4096
-// chunks: T 32 MiB, G 1 MiB) fits with room to spare; bf16 up to 4 964 chunks of 64 tokens, fp32
-// (T and P) up to 1 270.  Every GPU the library runs on holds one copy until the process ends.
-constexpr size_t kStaticScratchBytes = size_t(40) << 20;
+// Its workspace is this file-scope array.  40 MiB are what whole chains may need: the bf16 headline shape
+// (B4 H16 T4096, 4096 chunks: T 32 MiB, G 1 MiB) fits with room to spare; bf16 up to 4 964 chunks of 64
+// tokens, fp32 (T and P) up to 1 270.  32 MiB more hold the states and maps of whatever runs in segments
+// (at most 128 KiB for each of the 256 workgroups of a generation of maps), so that an accepted call takes
+// the route it takes on a workspace of its shape.  Every GPU the library runs on holds one copy until the
+// process ends.
+constexpr size_t kStaticChainBytes = size_t(40) << 20;
+constexpr size_t kStaticScratchBytes = kStaticChainBytes + (size_t(pf::kCus) << 17);
 static __device__ __align__(256) unsigned char scratch[kStaticScratchBytes];
 
 // Device address of `scratch` on the current device, resolved once per device with
@@ -330,7 +334,7 @@ int pf_gdn_exec_static(const void* q, const void* k, const void* v, const float*
                        const float* g, const float* h0, float* o, float* h_final, int B, int H,
                        int T, int C, int DK, int DV, int dtype, float scale, void* stream) {
   if (!gdn_shape_ok(B, H, T, C, DK, DV, dtype)) return PF_ERR_ARG;
-  if (GdnLayout(B * H, T / kChunk, dtype, {1, T / kChunk}).base > kStaticScratchBytes)
+  if (GdnLayout(B * H, T / kChunk, dtype, {1, T / kChunk}).base > kStaticChainBytes)
     return PF_ERR_SCRATCH;
   if (!q || !k || !v || !beta || !o) return PF_ERR_ARG;
   int st = PF_OK;
