@@ -15,9 +15,10 @@
 // by one rule: chunk m = c*H + h, token i of it lives at row (c*C + i)*H + h.  H = 1 is the native
 // layout.  Gates follow the same rule with row length 1, scores with row length C.
 //
-// gfx950 mapping.  256-thread workgroups (4 waves), one per chunk.  A wave owns whole 16-token query
-// blocks: their rows go straight from HBM into its registers as MFMA operands (no other wave reads
-// them); only the key side (and v) is staged in LDS, unpadded with XOR-permuted 16-byte slots.
+// gfx950 mapping (chunks of 64 and 128 tokens; of 16 and 32: pf_stages_small.h).  256-thread workgroups
+// (4 waves), one per chunk.  A wave owns whole 16-token query blocks: their rows go straight from HBM into
+// its registers as MFMA operands (no other wave reads them); only the key side (and v) is staged in LDS,
+// unpadded with XOR-permuted 16-byte slots.
 // Every score tile is formed transposed, P^T = k_jb q_ib^T, so a lane holds P[16 ib + c][16 jb + 4g ..
 // +3]: four consecutive columns of one row, which is a vector to store (gated_qk) and, two tiles
 // together, the B operand of o^T = v^T P^T as it stands (qkv_flash; v^T by transposed reads of the
@@ -106,9 +107,10 @@ struct GatedQkArgs {
 
 template <typename E, int C, int D, bool MASK>
 __global__ __launch_bounds__(256) void gated_qk_kernel(GatedQkArgs p) {
+  static_assert(C >= 64, "smaller chunks: pf_stages_small.h");
   typedef typename VecT<E>::T V;
   constexpr int VE = Vec16<E>::N, SLOTS = D / VE, NB = C / 16, NKB = D / Mfma<E>::KB;
-  constexpr int NBW = (NB + 3) / 4, NV = (C * SLOTS + 255) / 256;
+  constexpr int NBW = NB / 4, NV = C * SLOTS / 256;
   __shared__ __attribute__((aligned(16))) E sb[C * D];
   __shared__ __attribute__((aligned(16))) float Gs[C], Ls[C];
   const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, c = lane & 15;
@@ -122,7 +124,7 @@ __global__ __launch_bounds__(256) void gated_qk_kernel(GatedQkArgs p) {
 
   V br[NV], q[NBW][NKB];
   auto b_off = [&](int i) {
-    const int u = tid + 256 * i;                       // vectors past the tile repeat its last one
+    const int u = tid + 256 * i;                       // always in the tile; see the guard below
     return (min(u, C * SLOTS - 1) / SLOTS) * rs + (u % SLOTS) * VE;
   };
   auto a_off = [&](int s, int kb) {
@@ -152,10 +154,11 @@ __global__ __launch_bounds__(256) void gated_qk_kernel(GatedQkArgs p) {
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
     const int u = tid + 256 * i, row = u / SLOTS;
-    if (C * SLOTS >= 256 * (i + 1) || u < C * SLOTS)
-      *reinterpret_cast<V*>(sb + row * D + VE * key_slot<E, D>(row, u % SLOTS)) = br[i];
+    *reinterpret_cast<V*>(sb + row * D + VE * key_slot<E, D>(row, u % SLOTS)) = br[i];
   }
   lds_barrier();
+  // Never taken, as the min of the row offsets never acts (C >= 64).  Both shape what the compiler makes of
+  // the score tiles: without them fp32 scores at C = D = 128 took up to 1.4 times as long (4096 chunks).
   if (w >= NB) return;
   const size_t lrs = (size_t)p.H * C, lbase = ((size_t)ch * C * p.H + h) * C;
 #pragma unroll
@@ -194,10 +197,6 @@ __global__ __launch_bounds__(256) void gated_qk_kernel(GatedQkArgs p) {
         const u32x2 e1 = __builtin_amdgcn_permlane16_swap(x[1], y[1], false, false);
         *reinterpret_cast<u32x4*>(L + 32 * jp + 16 * (g & 1) + 8 * (g >> 1)) = u32x4{e0[0], e1[0], e0[1], e1[1]};
       }
-      if constexpr (NB == 1) {
-        const floatx4 t0 = tile(0);
-        store4(L + 4 * g, t0[0], t0[1], t0[2], t0[3]);
-      }
     }
   }
 }
@@ -217,10 +216,11 @@ template <typename E, int C, int D>
 __global__ __launch_bounds__(256)
 __attribute__((amdgpu_waves_per_eu(C * D * sizeof(E) > 32 * 1024 ? 1 : 2, 8)))
 void qkv_flash_kernel(QkvFlashArgs p) {
+  static_assert(C >= 64, "smaller chunks: pf_stages_small.h");
   typedef typename VecT<E>::T V;
   constexpr bool B16 = sizeof(E) == 2;
   constexpr int VE = Vec16<E>::N, SLOTS = D / VE, NB = C / 16, NKB = D / Mfma<E>::KB;
-  constexpr int NBW = (NB + 3) / 4, NV = (C * SLOTS + 255) / 256;
+  constexpr int NBW = NB / 4, NV = C * SLOTS / 256;
   __shared__ __attribute__((aligned(16))) E sk[C * D];
   __shared__ __attribute__((aligned(16))) E sv[C * D];
   __shared__ __attribute__((aligned(16))) float Gs[C], Ls[C];
@@ -264,13 +264,12 @@ void qkv_flash_kernel(QkvFlashArgs p) {
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
     const int u = tid + 256 * i, row = u / SLOTS;
-    if (C * SLOTS >= 256 * (i + 1) || u < C * SLOTS)
-      *reinterpret_cast<V*>(sk + row * D + VE * key_slot<E, D>(row, u % SLOTS)) = kr[i];
+    *reinterpret_cast<V*>(sk + row * D + VE * key_slot<E, D>(row, u % SLOTS)) = kr[i];
   }
   lds_barrier();
 
   // the score rows of this wave's query blocks, in the operand type
-  constexpr int NP = B16 ? (NB + 1) / 2 : NB;
+  constexpr int NP = B16 ? NB / 2 : NB;
   typedef typename std::conditional<B16, bf16x8, floatx4>::type PV;
   PV P[NBW][NP];
 #pragma unroll
@@ -298,11 +297,10 @@ void qkv_flash_kernel(QkvFlashArgs p) {
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
     const int u = tid + 256 * i, row = u / SLOTS;
-    if (C * SLOTS >= 256 * (i + 1) || u < C * SLOTS)
-      *reinterpret_cast<V*>(sv + row * D + VE * val_slot<E, D>(row, u % SLOTS)) = vr[i];
+    *reinterpret_cast<V*>(sv + row * D + VE * val_slot<E, D>(row, u % SLOTS)) = vr[i];
   }
   lds_barrier();
-  if (w >= NB) return;
+  if (w >= NB) return;                                 // never taken, as in gated_qk_kernel
   // o^T tiles: lane (c, g) gets o[16 ib + c][16 r + 4g .. +3]
 #pragma unroll
   for (int s = 0; s < NBW; ++s) {

@@ -5,6 +5,7 @@
 
 #include "../../include/pto_fuser_hip.h"
 #include "pf_stages.h"
+#include "pf_stages_small.h"
 #include "pf_state_scan.h"
 #include "pf_status.h"
 
@@ -48,8 +49,13 @@ struct GatedQkLaunch {
   template <typename E, int C, int D>
   int operator()() {
     pf::LaunchScope scope;
-    if (a.mask) pf::gated_qk_kernel<E, C, D, true><<<dim3(grid), dim3(256), 0, s>>>(a);
-    else pf::gated_qk_kernel<E, C, D, false><<<dim3(grid), dim3(256), 0, s>>>(a);
+    if constexpr (C < 64) {
+      if (a.mask) pf::gated_qk_small_kernel<E, C, D, true><<<dim3(grid), dim3(256), 0, s>>>(a);
+      else pf::gated_qk_small_kernel<E, C, D, false><<<dim3(grid), dim3(256), 0, s>>>(a);
+    } else {
+      if (a.mask) pf::gated_qk_kernel<E, C, D, true><<<dim3(grid), dim3(256), 0, s>>>(a);
+      else pf::gated_qk_kernel<E, C, D, false><<<dim3(grid), dim3(256), 0, s>>>(a);
+    }
     return scope.status();
   }
 };
@@ -61,7 +67,8 @@ struct QkvFlashLaunch {
   template <typename E, int C, int D>
   int operator()() {
     pf::LaunchScope scope;
-    pf::qkv_flash_kernel<E, C, D><<<dim3(grid), dim3(256), 0, s>>>(a);
+    if constexpr (C < 64) pf::qkv_flash_small_kernel<E, C, D><<<dim3(grid), dim3(256), 0, s>>>(a);
+    else pf::qkv_flash_kernel<E, C, D><<<dim3(grid), dim3(256), 0, s>>>(a);
     return scope.status();
   }
 };

@@ -94,3 +94,57 @@ def test_qkv_flash_tiles(dtype, C, D, scaled):
         ref = gated_qk_reference(_np(q), _np(k), g, beta, causal=True, dtype=np.float64) @ _np(v)
     tol = 1e-4 if dtype == torch.float32 else 1e-2
     assert max_rel(_np(o), ref) <= tol, max_rel(_np(o), ref)
+
+
+SMALL = [(torch.float32, 16), (torch.float32, 32), (torch.bfloat16, 32)]
+
+
+@pytest.mark.parametrize("M", [1, 2, 259])
+@pytest.mark.parametrize("dtype,C", SMALL)
+def test_small_chunks(dtype, C, M):
+    """Chunks of 16 and 32 tokens have one or two query blocks, whose work the four waves share: key blocks of
+    the score (gated, and with prescales and an explicit mask; both output types), columns of o."""
+    D, tol = (64 if M % 2 else 128), (1e-4 if dtype == torch.float32 else 1e-2)
+    announce(f"small chunks C={C} D={D} M={M} {dtype}")
+    rng = np.random.default_rng(C + M)
+    a, b, v = (_rows(rng, (M, C, D), dtype, s) for s in (0.2, 0.2, 1.0))
+    G = np.cumsum(-np.log1p(np.exp(rng.standard_normal((M, C)))) * 0.1, axis=1).astype(np.float32)
+    beta = (1 / (1 + np.exp(-rng.standard_normal((M, C))))).astype(np.float32)
+    sa, sb = (rng.random((M, C, D)).astype(np.float32) + 0.5 for _ in range(2))
+    mask = ((rng.random((C, C)) < 0.5) * rng.random((C, C))).astype(np.float32)
+    ad, bd = a.to(DEV), b.to(DEV)
+    for out16 in (False, True):
+        od = torch.bfloat16 if out16 else torch.float32
+        gated = gated_qk(ad, bd, _dev(G), _dev(beta), chunk_size=C, causal=True, out_dtype=od)
+        masked = gated_qk(ad, bd, chunk_size=C, mask=_dev(mask), a_scale=_dev(sa), b_scale=_dev(sb), out_dtype=od)
+        torch.cuda.synchronize()
+        ref = gated_qk_reference(_np(a), _np(b), G, beta, causal=True, dtype=np.float64)
+        bound = tol + (2 ** -8 if out16 else 0)
+        assert max_rel(_np(gated).reshape(ref.shape), ref) <= bound
+        mref = np.matmul(_np(a) * sa, (_np(b) * sb).transpose(0, 2, 1)) * mask
+        assert max_rel(_np(masked).reshape(mref.shape), mref) <= bound
+    o = qkv_flash(ad, bd, v.to(DEV), _dev(G), _dev(beta), chunk_size=C)
+    scaled = qkv_flash(ad, bd, v.to(DEV), chunk_size=C, q_scale=_dev(sa), k_scale=_dev(sb))
+    torch.cuda.synchronize()
+    assert max_rel(_np(o), ref @ _np(v)) <= tol
+    sref = np.tril(np.matmul(_np(a) * sa, (_np(b) * sb).transpose(0, 2, 1))) @ _np(v)
+    assert max_rel(_np(scaled), sref) <= tol
+
+
+@pytest.mark.parametrize("nc,H", [(1, 3), (65, 4)])
+def test_small_chunks_of_interleaved_heads(nc, H):
+    """Small chunks in the token layout: the staged query and key rows lie H rows apart."""
+    C, D = 16, 128
+    announce(f"small chunks C={C} nc={nc} H={H} heads interleaved")
+    rng = np.random.default_rng(nc)
+    a, b = (_rows(rng, (nc * C * H, D), torch.float32) for _ in range(2))
+    g = (-np.cumsum(rng.random((nc, C, H)), axis=1) * 0.1).astype(np.float32)
+    L = gated_qk(a.to(DEV), b.to(DEV), _dev(g.reshape(-1)), chunk_size=C, heads=H, causal=False)
+    torch.cuda.synchronize()
+
+    def chunks(x):
+        return x.reshape(nc, C, H, -1).transpose(0, 2, 1, 3).reshape(nc * H, C, -1)
+
+    ref = gated_qk_reference(chunks(_np(a)), chunks(_np(b)), chunks(g)[..., 0], np.ones((nc * H, C)), causal=False,
+                             dtype=np.float64)
+    assert max_rel(chunks(_np(L)), ref) <= 1e-4
