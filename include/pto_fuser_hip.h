@@ -56,7 +56,7 @@ const char* pf_source_hash(void);
  *   summed within each chunk of C tokens by the kernel); h0 [B,H,DK,DV] fp32 or NULL (zero);
  *   o [B,H,T,DV] fp32 (scaled by `scale`); h_final [B,H,DK,DV] fp32 or NULL.
  *   Supported: C = 64 or 128, DK = DV = 128, T % C == 0, T <= 4 194 304 (per-chain addressing is
- *   32-bit; a longer sequence is PF_ERR_ARG).  The kernels run 64-token chunks; C = 128
+ *   32-bit; a longer sequence is PF_ERR_ARG), B * H <= 2^24 (more chains do not fit the memory).  The kernels run 64-token chunks; C = 128
  *   (the reference's chunk) is served by them over T / 64 chunks — the chunked forward's result
  *   does not depend on the chunk size, only the blocking of its arithmetic does.
  *   bf16 operands, few long chains: a chain runs as segments side by side, joined through their
@@ -130,7 +130,7 @@ int pf_gdn_scan_output_exec(const void* q, const void* k, const void* v, const f
  *   h0 [B,H,DK,DV] fp32 or NULL; o [B,H,T,DV] fp32 (scaled by `scale`); h_final [B,H,DK,DV]
  *   fp32 or NULL.  Supported: dtype PF_DTYPE_BF16 (bf16 MFMA) or PF_DTYPE_F32 (fp32
  *   operands and fp32 MFMA throughout), C = 64 or 128 (run as 64-token chunks),
- *   DK = DV = 128, T % C == 0, T <= 4 194 304.  The workspace holds the stage-1 images in the
+ *   DK = DV = 128, T % C == 0, T <= 4 194 304, B * H <= 2^24.  The workspace holds the stage-1 images in the
  *   operand type; bf16, few long chains: also the segments' state maps, used as by pf_gdn_exec.
  * ------------------------------------------------------------------------------------------ */
 size_t pf_kda_workspace_bytes(int B, int H, int T, int C, int DK, int DV, int dtype);

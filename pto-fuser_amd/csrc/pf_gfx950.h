@@ -16,6 +16,9 @@ constexpr int kCachePolicyNT = 2;
 // are addressed through one buffer descriptor, whose byte range and offsets are 32-bit; the limit
 // keeps them below 2^31.
 constexpr int kMaxChainTokens = 1 << 22;
+// Chains of a call: counts of chains and of their workgroups are 32-bit.  (One chunk each of this many is over
+// 1 TB of operands.)
+constexpr long kMaxChains = 1L << 24;
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base, uint32_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)bytes, 0x00020000);

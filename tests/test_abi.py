@@ -141,8 +141,18 @@ def test_segment_states_are_bounded(lib):
     chains need: their maps run in one generation of workgroups."""
     for op, mib in (("gdn", 32), ("kda", 16)):
         for chains in (1, 3, 8, 16, 17, 36, 64, 100, 132, 256, 300):
-            for chunks in (16, 67, 128, 500, 512, 5040, 65536):
+            for chunks in (16, 67, 128, 500, 512, 5040, 50000):
                 assert (_segments(lib, op, chains, chunks) - 1) * chains * 2 * 128 * 128 * 4 <= mib << 20
+
+
+@pytest.mark.parametrize("op", ["gdn", "kda"])
+def test_chain_counts_do_not_wrap(lib, op):
+    """B * H past 32 bits is refused: it may not come out as a small workspace that a call would accept."""
+    size = lib.pf_gdn_workspace_bytes if op == "gdn" else lib.pf_kda_workspace_bytes
+    for B, H in ((1 << 16, 1 << 16), ((1 << 16) + 1, (1 << 16) + 1), (1 << 20, 1 << 12), (1 << 15, 1 << 16)):
+        assert size(B, H, 64, 64, 128, 128, 1) == 0
+        assert size(B, H, 64, 64, 128, 128, 0) == 0
+    assert size(1 << 12, 1 << 12, 64, 64, 128, 128, 1) >= (1 << 24) * 64 * 64 * 2
 
 
 _FAKE_HIP = """#include <stdlib.h>
