@@ -283,8 +283,8 @@ struct KdaScanArgs {
   float* h_final;       // [BH, DK, DV] or null
   int BH;
   int NC;
-  const float* hseg;    // segmented chains, as ScanOutArgs: SEG segments of L chunks, segment s > 0 from
-  int SEG, L;           //   hseg[bh][s - 1]
+  int SEG, L;           // segmented chains, as ScanOutArgs: SEG segments of L chunks, segment s > 0 from
+  const float* hseg;    //   hseg[bh][s - 1]
   size_t h0_stride;
 };
 

@@ -19,12 +19,12 @@ struct ScanOutArgs {
   float* h_final;       // [BH, DK, DV] or null
   int BH;
   int NC;               // chunks per chain
-  const float* scale;   // device scalar: the output scale (written by stage 1)
   // segmented chains (bf16): each chain runs as SEG segments of L chunks (the last may have fewer),
-  // segment s > 0 from the state hseg[bh][s - 1]; SEG = 1, L = NC otherwise.  h0_stride: elements between
-  // two chains' h0 (DK * DV, or more where h0 is the maps' copy of it)
-  const float* hseg;    // [BH, SEG - 1, DK, DV]
+  // segment s > 0 from the state hseg[bh][s - 1]; SEG = 1, L = NC otherwise.  h0_stride (SEG > 1): elements
+  // between two chains' h0 (DK * DV, or more where h0 is the maps' copy of it)
   int SEG, L;
+  const float* scale;   // device scalar: the output scale (written by stage 1)
+  const float* hseg;    // [BH, SEG - 1, DK, DV]
   size_t h0_stride;
 };
 

@@ -123,9 +123,11 @@ void scan_split_kernel(ScanOutArgs a) {
     slice = bid % NS;
   }
   int bh = unit, seg = 0, NC = a.NC;            // NC: this segment's chunks
+  size_t h0_stride = DK * DV;
   if (a.SEG > 1) {
     bh = unit / a.SEG;
     seg = unit % a.SEG;
+    h0_stride = a.h0_stride;
     // a chain whose maps left fp32 range (seg_compose_kernel) is run whole, by its first unit
     const float mark =
         a.hseg[((size_t)bh * (a.SEG - 1) + a.SEG - 2) * DK * DV + slice * NCOL + (threadIdx.x & (NCOL - 1))];
@@ -359,7 +361,7 @@ void scan_split_kernel(ScanOutArgs a) {
     const int xhalf = 4 * (cw & 1), xblk = cw >> 1;                        // this wave's RX/VX slot
 
     const float* h_in = seg ? a.hseg + ((size_t)bh * (a.SEG - 1) + seg - 1) * DK * DV
-                            : a.h0 ? a.h0 + (size_t)bh * a.h0_stride : nullptr;
+                            : a.h0 ? a.h0 + bh * h0_stride : nullptr;
     floatx4 S[2][NT];                                    // rows 32cw + 16r + 4g + i, column c
 #pragma unroll
     for (int r = 0; r < 2; ++r)
