@@ -14,7 +14,7 @@ import torch
 from conftest import announce, record_error
 from oracle.gdn_oracle import (deltanet_reference, gdn_reference, max_abs, max_rel,
                                tri_inv_reference, within_chunk_cumsum)
-from pto_fuser_amd import gdn_chunk_forward, kkt_inverse, tri_inv
+from pto_fuser_amd import _hip, gdn_chunk_forward, kkt_inverse, ops, tri_inv
 from pto_fuser_amd.forwards import as_oracle_inputs, make_delta_inputs
 
 pytestmark = pytest.mark.gpu
@@ -151,11 +151,12 @@ def test_gdn_bf16_score_gates(name):
     _check(f"GDN bf16 score gates {name}", o, h, o_ref, h_ref, bf16=True)
 
 
-# The scan launcher takes 32-column state slices (four workgroups per chain) when B*H >= 64, the
-# headline's instantiation, and 16-column slices below that; the tests above at B*H <= 6 run the
-# 16-column kernel.  The cases below run the 32-column one at its edges: one, two and three
+# The scan launcher takes 16-column state slices up to B*H = 32, 32-column ones (four workgroups per
+# chain, the headline's instantiation) up to 64 and 64-column ones above; the tests above at B*H <= 6
+# run the 16-column kernel.  The cases below run the 32-column one at its edges: one, two and three
 # chunks per chain (the loaders' end-of-chain clamps), a nonzero h0, both score-gate paths, and
-# B*H not a multiple of 8 (the slice mapping without XCD grouping).
+# B*H not a multiple of 8 (the slice mapping without XCD grouping); and the 64-column one without
+# that grouping.
 @pytest.mark.parametrize("T", [64, 128, 192, 1024])
 def test_gdn_bf16_wide_slices_h0(T):
     B, H = 4, 16
@@ -181,13 +182,24 @@ def test_gdn_bf16_wide_slices_score_gates(name):
 
 @pytest.mark.parametrize("B,H,T", [(3, 22, 512), (5, 13, 192)])
 def test_gdn_bf16_wide_slices_unaligned_chains(B, H, T):
-    """B*H = 66 and 65: 32-column slices, chains not grouped by XCD (B*H % 8 != 0)."""
-    announce(f"GDN bf16 B{B} H{H} T{T} h0 (32-col, B*H % 8 != 0)")
+    """B*H = 66 and 65: 64-column slices, chains not grouped by XCD (B*H % 8 != 0)."""
+    announce(f"GDN bf16 B{B} H{H} T{T} h0 (64-col, B*H % 8 != 0)")
     inp = make_delta_inputs(B, H, T, kind="gdn", dtype=torch.bfloat16, seed=B * 50 + H,
                             h0_std=0.02)
     o, h = _run(inp)
     o_ref, h_ref = _oracle(inp)
-    _check(f"GDN bf16 B{B} H{H} T{T} h0 (32-col)", o, h, o_ref, h_ref, bf16=True)
+    _check(f"GDN bf16 B{B} H{H} T{T} h0 (64-col)", o, h, o_ref, h_ref, bf16=True)
+
+
+@pytest.mark.parametrize("B,H,T,kind", [(5, 7, 64, "gdn"), (5, 7, 320, "gdn"), (2, 31, 192, "gdn"),
+                                        (3, 11, 128, "deltanet")])
+def test_gdn_bf16_32_column_slices_unaligned_chains(B, H, T, kind):
+    """B*H = 35, 62 and 33: 32-column slices, chains not grouped by XCD (B*H % 8 != 0)."""
+    announce(f"{kind} bf16 B{B} H{H} T{T} h0 (32-col, B*H % 8 != 0)")
+    inp = make_delta_inputs(B, H, T, kind=kind, dtype=torch.bfloat16, seed=B * 90 + H, h0_std=0.02)
+    o, h = _run(inp)
+    o_ref, h_ref = _oracle(inp)
+    _check(f"{kind} bf16 B{B} H{H} T{T} h0 (32-col)", o, h, o_ref, h_ref, bf16=True)
 
 
 @pytest.mark.parametrize("B,H,T", [(16, 32, 128), (7, 73, 192)])
@@ -219,7 +231,8 @@ def test_deltanet_bf16_fused(B, H, T):
 def test_deltanet_bf16_longest_chain():
     """No decay at the longest chain the forward takes in one call at this size (T = 32768,
     512 chunks) with h0: the state's bf16 rounding never washes out, so this is where its error
-    builds up most; it levels off near 1e-2 on h (|h| up to ~3)."""
+    builds up most; it levels off near 1e-2 on h (|h| up to ~3).  The call runs in segments; the next
+    test runs the chains whole."""
     announce("DeltaNet bf16 fused B1 H2 T32768 h0")
     inp = make_delta_inputs(1, 2, 32768, kind="deltanet", dtype=torch.bfloat16, seed=3, h0_std=0.02)
     o, h = _run(inp)
@@ -227,6 +240,24 @@ def test_deltanet_bf16_longest_chain():
     ref = deltanet_reference(x["q"], x["k"], x["v"], x["beta"], C=64, h0=x["h0"], dtype=np.float64)
     _check("DeltaNet bf16 fused B1 H2 T32768 h0", o, h, ref["o"].reshape(o.shape), ref["final"],
            bf16=True)
+
+
+def test_deltanet_bf16_longest_chain_whole():
+    """The same as one sequence of 512 chunk steps per chain, on a workspace that holds what whole
+    chains need and no segments: the rounding of the whole chain is within the bound too."""
+    B, H, T = 1, 2, 32768
+    announce(f"DeltaNet bf16 fused B{B} H{H} T{T} h0, whole chains")
+    inp = make_delta_inputs(B, H, T, kind="deltanet", dtype=torch.bfloat16, seed=3, h0_std=0.02)
+    d = {n: (None if t is None else t.to(DEV)) for n, t in inp.items()}
+    ws = ops.GdnWorkspace(B, H * T // 64, 64, 64, 128, 128, _hip.PF_DTYPE_BF16, torch.device(DEV))
+    seg, _ = gdn_chunk_forward(d["q"], d["k"], d["v"], d["beta"], None, h0=d["h0"])
+    o, h = gdn_chunk_forward(d["q"], d["k"], d["v"], d["beta"], None, h0=d["h0"], workspace=ws)
+    torch.cuda.synchronize()
+    assert not torch.equal(o, seg)                       # the other route ran
+    x = as_oracle_inputs(inp)
+    ref = deltanet_reference(x["q"], x["k"], x["v"], x["beta"], C=64, h0=x["h0"], dtype=np.float64)
+    _check(f"DeltaNet bf16 fused B{B} H{H} T{T} h0 whole", o.cpu().numpy(), h.cpu().numpy(),
+           ref["o"].reshape(o.shape), ref["final"], bf16=True)
 
 
 def test_gdn_bf16_config2():
@@ -283,8 +314,8 @@ def test_gdn_deterministic():
 def test_gdn_state_passing_config4():
     """Size-independent property at the long-context shape (config 4, with h0): running [0,T)
     equals running [0,T/2) and then [T/2,T) from the first half's final state.  Both runs see
-    the same bf16 operands; they differ only in where the kernel's deferred state factor is
-    folded back in, so the difference stays far below the oracle tolerance (5e-3 abs)."""
+    the same bf16 operands; they differ in where a segment starts and where the kernel's deferred
+    state factor is folded back in, so the difference stays far below the oracle tolerance (5e-3 abs)."""
     announce("GDN bf16 state passing B1 H32 T32768 h0")
     inp = make_delta_inputs(1, 32, 32768, kind="gdn", dtype=torch.bfloat16, seed=4, h0_std=0.02)
     d = {n: (None if t is None else t.to(DEV)) for n, t in inp.items()}

@@ -1,8 +1,10 @@
 """The bf16 scan's column slices: 16, 32 and 64 columns, chosen by how many chains a call has.  A state
-column is computed the same way in all three, so a chain's outputs do not depend on how many chains
-run beside it: the first 40 and the first 8 of 72 chains give the same bits as within the 72, with
-every score-gate path, one chunk to five, and 72 and 69 chains (grouped by XCD and not).  KDA likewise
-with its 32- and 64-column slices."""
+column is computed the same way in all three, so while chains run whole a chain's outputs do not
+depend on how many run beside it: the first 40 and the first 8 of 72 chains give the same bits as
+within the 72, with every score-gate path, one chunk to five, and 72 and 69 chains (grouped by XCD
+and not).  KDA likewise with its 32- and 64-column slices.  (Long chains that are few run in segments,
+and how many segments depends on how many chains there are: there the same chain alone and in a batch
+differs by its bf16 rounding; test_gpu_segments.py has them.)"""
 import pytest
 import torch
 

@@ -1,6 +1,6 @@
 """A seeded random sweep of the fused forwards against the oracle: GDN, DeltaNet (g = None) and
 KDA, bf16 and fp32 operands, chunk size 64 or 128, with and without h0, gate scales from none to
-steep, B·H from 1 to 66 (so both scan instantiations, the XCD-aware and the plain chain mapping)
+steep, B·H from 1 to 66 (so every scan instantiation, the XCD-aware and the plain chain mapping)
 and chains of 1 to 24 chunks.  The cases are drawn once from a fixed seed, so every run and every
 failure names the same shapes.  Bounds as in the other parity tests: bf16 inputs max abs err
 <= 2e-2, fp32 max rel err <= 1e-4, on o and the final state.  Oracle:
