@@ -472,7 +472,7 @@ __global__ __launch_bounds__(4 * C) void tri_inv_blocks_kernel(const float* A, f
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int r = r0 + 16 * i;
-    floatx4 x = *reinterpret_cast<const floatx4*>(Ag + d0 + (size_t)r * C + j0);
+    floatx4 x = *reinterpret_cast<const floatx4_any*>(Ag + d0 + (size_t)r * C + j0);
 #pragma unroll
     for (int e = 0; e < 4; ++e) x[e] = j0 + e < r ? x[e] : 0.f;
     *reinterpret_cast<floatx4*>(D + r * CP + j0) = x;
@@ -482,7 +482,7 @@ __global__ __launch_bounds__(4 * C) void tri_inv_blocks_kernel(const float* A, f
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       const int r = (tid >> 4) + 32 * i;
-      *reinterpret_cast<floatx4*>(L + r * CP + j0) = *reinterpret_cast<const floatx4*>(Ag + (size_t)(64 + r) * C + j0);
+      *reinterpret_cast<floatx4*>(L + r * CP + j0) = *reinterpret_cast<const floatx4_any*>(Ag + (size_t)(64 + r) * C + j0);
     }
   }
   lds_barrier();
@@ -493,12 +493,12 @@ __global__ __launch_bounds__(4 * C) void tri_inv_blocks_kernel(const float* A, f
     floatx4 x = *reinterpret_cast<const floatx4*>(D + r * CP + j0);
 #pragma unroll
     for (int e = 0; e < 4; ++e) x[e] = j0 + e <= r ? x[e] : 0.f;   // above the diagonal: scratch
-    *reinterpret_cast<floatx4*>(Tg + d0 + (size_t)r * C + j0) = x;
+    *reinterpret_cast<floatx4_any*>(Tg + d0 + (size_t)r * C + j0) = x;
   }
   if constexpr (NB == 2) {
 #pragma unroll
     for (int i = 0; i < 2; ++i)
-      *reinterpret_cast<floatx4*>(Tg + (size_t)((tid >> 4) + 32 * i) * C + 64 + j0) = zero4();
+      *reinterpret_cast<floatx4_any*>(Tg + (size_t)((tid >> 4) + 32 * i) * C + 64 + j0) = zero4();
     const int a = w >> 1, p0 = (w & 1) ? 1 : 0, p1 = (w & 1) ? 2 : 3;
     floatx4 X[2];                                        // X tiles (a, p0), (a, p1): T1 lower triangular
 #pragma unroll

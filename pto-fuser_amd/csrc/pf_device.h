@@ -32,11 +32,11 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));   // one 16-byte vector
-
-constexpr int kWave = 64;
-
-__device__ __forceinline__ int lane_id() { return threadIdx.x & 63; }
-__device__ __forceinline__ int wave_id() { return threadIdx.x >> 6; }
+// The same at a caller's address that promises an element's alignment only (a contiguous view that starts
+// inside a buffer): one instruction all the same, since global accesses need no more.
+typedef float floatx4_any __attribute__((ext_vector_type(4), aligned(4)));
+typedef unsigned int u32x4_any __attribute__((ext_vector_type(4), aligned(2)));
+typedef __bf16 bf16x4_any __attribute__((ext_vector_type(4), aligned(2)));
 
 __device__ __forceinline__ float to_f32(float x) { return x; }
 __device__ __forceinline__ float to_f32(bf16 x) { return (float)x; }

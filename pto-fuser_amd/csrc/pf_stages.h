@@ -182,7 +182,7 @@ __global__ __launch_bounds__(256) void gated_qk_kernel(GatedQkArgs p) {
     if (p.out_f32) {
 #pragma unroll
       for (int jb = 0; jb < NB; ++jb)
-        *reinterpret_cast<floatx4*>(static_cast<float*>(p.L) + row + 16 * jb + 4 * g) = tile(jb);
+        *reinterpret_cast<floatx4_any*>(static_cast<float*>(p.L) + row + 16 * jb + 4 * g) = tile(jb);
     } else {
       bf16* L = static_cast<bf16*>(p.L) + row;
 #pragma unroll
@@ -195,7 +195,7 @@ __global__ __launch_bounds__(256) void gated_qk_kernel(GatedQkArgs p) {
         const u32x2 y = __builtin_bit_cast(u32x2, bf16x4{(bf16)t1[0], (bf16)t1[1], (bf16)t1[2], (bf16)t1[3]});
         const u32x2 e0 = __builtin_amdgcn_permlane16_swap(x[0], y[0], false, false);
         const u32x2 e1 = __builtin_amdgcn_permlane16_swap(x[1], y[1], false, false);
-        *reinterpret_cast<u32x4*>(L + 32 * jp + 16 * (g & 1) + 8 * (g >> 1)) = u32x4{e0[0], e1[0], e0[1], e1[1]};
+        *reinterpret_cast<u32x4_any*>(L + 32 * jp + 16 * (g & 1) + 8 * (g >> 1)) = u32x4{e0[0], e1[0], e0[1], e1[1]};
       }
     }
   }
@@ -327,7 +327,7 @@ void qkv_flash_kernel(QkvFlashArgs p) {
           }
         }
       }
-      *reinterpret_cast<floatx4*>(o + 16 * r) = acc;
+      *reinterpret_cast<floatx4_any*>(o + 16 * r) = acc;
     }
   }
 }

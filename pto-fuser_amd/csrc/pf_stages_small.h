@@ -60,7 +60,7 @@ __global__ __launch_bounds__(256) void gated_qk_small_kernel(GatedQkArgs p) {
   for (int i = 0; i < NV; ++i) ar[i] = load_vec(ag, off(i));
   const int i = 16 * ib + c, j0 = 16 * jb + 4 * g;     // this lane's row and first column of its tile
   floatx4 mask = zero4();
-  if (MASK && jb < NB) mask = *reinterpret_cast<const floatx4*>(p.mask + i * C + j0);
+  if (MASK && jb < NB) mask = *reinterpret_cast<const floatx4_any*>(p.mask + i * C + j0);
   if (p.b_scale) {
 #pragma unroll
     for (int i = 0; i < NV; ++i) prescale<E>(br[i], p.b_scale + base, off(i));
@@ -92,8 +92,8 @@ __global__ __launch_bounds__(256) void gated_qk_small_kernel(GatedQkArgs p) {
     }
   }
   const size_t e = (((size_t)ch * C + i) * p.H + h) * C + j0;
-  if (p.out_f32) *reinterpret_cast<floatx4*>(static_cast<float*>(p.L) + e) = out;
-  else store4(static_cast<bf16*>(p.L) + e, out[0], out[1], out[2], out[3]);
+  if (p.out_f32) *reinterpret_cast<floatx4_any*>(static_cast<float*>(p.L) + e) = out;
+  else *reinterpret_cast<bf16x4_any*>(static_cast<bf16*>(p.L) + e) = bf16x4_any{(bf16)out[0], (bf16)out[1], (bf16)out[2], (bf16)out[3]};
 }
 
 template <typename E, int C, int D>
@@ -195,7 +195,7 @@ void qkv_flash_small_kernel(QkvFlashArgs p) {
         }
       }
     }
-    *reinterpret_cast<floatx4*>(o + 16 * r) = acc;
+    *reinterpret_cast<floatx4_any*>(o + 16 * r) = acc;
   }
 }
 

@@ -130,7 +130,7 @@ void scan_state_kernel(ScanStateArgs p) {
 #pragma unroll
     for (int i = 0; i < NU; ++i) {
       const int x = min(tid + 256 * i, U_VECS - 1);     // lanes past the tile repeat its last vector
-      ur[i] = *reinterpret_cast<const u32x4*>(ug + t0 + (size_t)(x / UVR) * rs + slice * NCOL + (x % UVR) * VE);
+      ur[i] = *reinterpret_cast<const u32x4_any*>(ug + t0 + (size_t)(x / UVR) * rs + slice * NCOL + (x % UVR) * VE);
     }
 #pragma unroll
     for (int i = 0; i < NV; ++i)
@@ -179,7 +179,7 @@ void scan_state_kernel(ScanStateArgs p) {
 #pragma unroll
         for (int r = 0; r < RB; ++r) {
           const bf16x4 t = lds_read_tr(x + n * D + 8 * scan_x_slot<D>(n, 2 * r + ((c & 3) >> 1)) + 4 * (c & 1));
-          *reinterpret_cast<bf16x4*>(ho + (size_t)(16 * r + c) * D + slice * NCOL + 16 * w + 4 * g) = t;
+          *reinterpret_cast<bf16x4_any*>(ho + (size_t)(16 * r + c) * D + slice * NCOL + 16 * w + 4 * g) = t;
         }
         return;
       }
@@ -209,7 +209,7 @@ void scan_state_kernel(ScanStateArgs p) {
     if constexpr (!PERDIM) dec1 = p.decay[(size_t)bh * p.NC + ch];
     auto load_decay = [&](int r) {
       if constexpr (PERDIM)
-        if (r < RB) dec[r] = *reinterpret_cast<const floatx4*>(p.decay + ((size_t)bh * p.NC + ch) * D + scan_row<E>(r, g, 0));
+        if (r < RB) dec[r] = *reinterpret_cast<const floatx4_any*>(p.decay + ((size_t)bh * p.NC + ch) * D + scan_row<E>(r, g, 0));
     };
     auto decayed = [&](int r) {
       if constexpr (PERDIM) return S[r] * dec[r];
