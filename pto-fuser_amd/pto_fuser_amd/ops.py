@@ -107,8 +107,13 @@ def _workspace(cls, B, H, T, C, DK, DV, code, device, stream):
     return ws
 
 
+def _named_device(device):
+    """One key for every form that names a device; None stays the current one."""
+    return None if device is None else torch.device(device)
+
+
 def gdn_workspace(B, H, T, C, DK, DV, dtype: torch.dtype, device) -> GdnWorkspace:
-    device = torch.device(device)
+    device = _named_device(device)
     return _workspace(GdnWorkspace, B, H, T, C, DK, DV, _dtype_code(dtype), device,
                       _hip.current_stream_handle(device))
 
@@ -134,7 +139,7 @@ class KdaWorkspace:
 
 
 def kda_workspace(B, H, T, C, DK, DV, dtype: torch.dtype, device) -> KdaWorkspace:
-    device = torch.device(device)
+    device = _named_device(device)
     return _workspace(KdaWorkspace, B, H, T, C, DK, DV, _dtype_code(dtype), device,
                       _hip.current_stream_handle(device))
 

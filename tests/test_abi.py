@@ -323,3 +323,28 @@ def test_stream_handle_of_every_device_form(monkeypatch, device):
     assert _hip.current_stream_handle(device) == 7
     with pytest.raises(ValueError):
         _hip.current_stream_handle(torch.device("cpu", 0))
+
+
+@pytest.mark.parametrize("name", ["gdn", "kda"])
+def test_workspaces_of_every_device_form(monkeypatch, name):
+    """A workspace can be asked for by device, string, index or None (the current device); the forms that
+    name one device share it."""
+    from pto_fuser_amd import ops
+    made = []
+
+    class Fake:
+        def __init__(self, *args):
+            made.append(args[-1])
+
+        def close(self):
+            pass
+
+    monkeypatch.setattr(ops, name.capitalize() + "Workspace", Fake)
+    monkeypatch.setattr(ops, "_WORKSPACES", {})
+    monkeypatch.setattr(ops._hip, "current_stream_handle", lambda device=None: 7)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    get = getattr(ops, name + "_workspace")
+    one = [get(1, 1, 64, 64, 128, 128, torch.float32, dev) for dev in ("cuda:0", 0, torch.device("cuda", 0))]
+    assert one[0] is one[1] is one[2]
+    current = get(1, 1, 64, 64, 128, 128, torch.float32, None)
+    assert isinstance(current, Fake) and made == [torch.device("cuda:0"), None]
