@@ -60,8 +60,13 @@ const char* pf_source_hash(void);
  *   (the reference's chunk) is served by them over T / 64 chunks — the chunked forward's result
  *   does not depend on the chunk size, only the blocking of its arithmetic does.
  *   bf16 operands, few long chains: a chain runs as segments side by side, joined through their
- *   state maps, when the workspace holds those (pf_gdn_workspace_bytes and pf_gdn_setup include them);
- *   on a smaller workspace the same call runs whole chains.
+ *   state maps, when the workspace holds those (pf_gdn_workspace_bytes and pf_gdn_setup include them,
+ *   at most 32 MiB); on a smaller workspace the same call runs whole chains.  Segments round to bf16 in
+ *   other places, and their number follows from the number of chains and chunks: from 29 chunks on, a
+ *   chain's result in a call of few chains and in one of many differs by that rounding (about 1e-3
+ *   of its norm; as far from float64 either way).  A workspace reserved for as many one-chunk chains
+ *   (B, H * T / 64, 64) has no room for segments: on it a chain's bits never depend on its neighbours.
+ *   h0 may be h_final itself (the state updated in place).
  * ------------------------------------------------------------------------------------------ */
 size_t pf_gdn_workspace_bytes(int B, int H, int T, int C, int DK, int DV, int dtype);
 void* pf_gdn_setup(int B, int H, int T, int C, int DK, int DV, int dtype);

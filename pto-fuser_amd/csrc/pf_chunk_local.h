@@ -144,7 +144,11 @@ __device__ __forceinline__ float quad_broadcast(float x, int p) {
 //      / lower-right quadrants: the four 16 x 16 tiles of X = A_LL T_L (one per wave) go to the
 //      unused strictly-upper quadrant of As, then the four tiles of -T_R X.
 // The off-diagonal part is three levels of at most two dependent 16 x 16 products each (a
-// block-diagonal sweep would end in a chain of four).  Must be called by all 256 threads.
+// block-diagonal sweep would end in a chain of four).
+//
+// Called by all 256 * GROUPS threads of the workgroup: every 256 of them (four waves) invert a block of
+// their own, each with its own As and Ts, and the barriers are the workgroup's, so that GROUPS blocks
+// go through the levels side by side.
 //
 // Ts may equal As (in place): every block of T is written only after the last read of the A
 // block at its position — T_ii by the wave that has read all of A_ii, T10 / T32 by the wave

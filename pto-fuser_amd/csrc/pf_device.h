@@ -106,13 +106,6 @@ __device__ __forceinline__ void store4(float* p, float a, float b, float c, floa
   *reinterpret_cast<floatx4*>(p) = floatx4{a, b, c, d};
 }
 
-// Four consecutive elements as fp32.
-__device__ __forceinline__ floatx4 load4f(const bf16* p) {
-  const bf16x4 v = *reinterpret_cast<const bf16x4*>(p);
-  return floatx4{(float)v[0], (float)v[1], (float)v[2], (float)v[3]};
-}
-__device__ __forceinline__ floatx4 load4f(const float* p) { return *reinterpret_cast<const floatx4*>(p); }
-
 // 16-byte vector type of an element type (8 bf16 or 4 fp32).
 template <typename E> struct Vec16;
 template <> struct Vec16<bf16> { typedef uint4 T; static constexpr int N = 8; };

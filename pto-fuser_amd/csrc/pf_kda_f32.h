@@ -1,6 +1,5 @@
 // KDA forward for fp32 operands: the two stages of the bf16 kernels (pf_kda.h) with fp32 tiles and
-// the fp32 MFMA (v_mfma_f32_16x16x4f32), written for exactness rather than throughput (no config
-// of the benchmark runs KDA in fp32).  Mathematics (examples/attention/_kda_full.py:42-76), per
+// the fp32 MFMA (v_mfma_f32_16x16x4f32).  Mathematics (examples/attention/_kda_full.py:42-76), per
 // chain and chunk of C tokens, G = within-chunk cumsum of g [C, dk], a = k e^G, b = k e^-G:
 //
 //   A = strictly_lower(beta_i (a b^T)_ij),  T = (I + A)^-1,  W = T diag(beta) a,  U = T diag(beta) v
@@ -250,7 +249,7 @@ struct KdaScanF32Args {
 // and KR rows, so it loads those slices itself and refills them after its own last read, with no
 // barrier; P is written between the barriers (its readers are past the first one), U after the
 // second.  Two barriers per chunk, the next chunk's loads in flight across both.  Bound by the chunk
-// step's chain, 3.6 us, of which the fp32 products take 1.4 (32 chains x 32 chunks: 115-123 us; 480
+// step's chain, 3.25 us, of which the fp32 products take 1.4 (32 chains x 32 chunks: 104 us; 480
 // for the earlier two-wave form, which copied every image with the products waiting).
 template <int C, int DK, int DV>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))

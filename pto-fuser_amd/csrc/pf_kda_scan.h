@@ -50,7 +50,7 @@
 
 namespace pf {
 
-// LDS image of one KDA chunk (C = 64, DK = 128, NCOL = 32 columns).
+// LDS image of one KDA chunk (C = 64, DK = 128, NCOL = 32 or 64 columns).
 template <int C, int DK, int NCOL>
 struct KdaSplitStage {
   static constexpr int KP = DK + 16;   // W, QE, KB rows: Swz<2,3>

@@ -104,8 +104,8 @@ void qkv_flash_small_kernel(QkvFlashArgs p) {
   constexpr bool B16 = sizeof(E) == 2;
   constexpr int VE = Sh::VE, SLOTS = Sh::SLOTS, NB = Sh::NB, NV = Sh::NV;
   constexpr int NP = B16 ? (NB + 1) / 2 : NB, NR = D / 16 / Sh::PARTS;
-  // fp32 rows of 32 tokens: v takes the query rows' place in LDS, which with three tiles allowed half as many
-  // workgroups on a CU (2048 chunks of 32 x 128 with prescales: 32.0 us, 29.7 shared)
+  // fp32 rows of 32 tokens: v takes the query rows' place in LDS, which lets a CU hold one or two workgroups
+  // more (2048 chunks of 32 x 128 with prescales: 32.0 us with three tiles, 29.7 with two)
   constexpr bool SHARE = !B16 && C == 32;
   typedef typename std::conditional<B16, bf16x8, floatx4>::type PV;
   __shared__ __attribute__((aligned(16))) E sk[C * D];

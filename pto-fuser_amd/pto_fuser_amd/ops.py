@@ -164,7 +164,12 @@ def gdn_chunk_forward(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, beta: t
     per-token log decay, summed within chunks by the kernel; None = DeltaNet); h0 [B,H,DK,DV]
     float32 or None.  Returns (o [B,H,T,DV] float32 scaled by ``scale`` (default DK^-1/2),
     h_final [B,H,DK,DV] float32 or None).  chunk_size 64 or 128: both run the 64-token kernels
-    (the result does not depend on the chunk size); T must be a multiple of it."""
+    (the result does not depend on the chunk size); T must be a multiple of it.
+
+    bfloat16, few long sequences: each runs as segments side by side, whose number follows from how
+    many sequences there are, so the same sequence alone and in a batch differs by its bfloat16
+    rounding.  With ``workspace=GdnWorkspace(B, H * T // 64, 64, 64, DK, DV, ...)``, which has no
+    room for segments, its bits do not depend on the batch."""
     if q.dim() != 4:
         raise ValueError(f"q must be [B,H,T,DK], got shape {tuple(q.shape)}")
     B, H, T, DK = q.shape
@@ -386,7 +391,7 @@ def kda_chunk_forward(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, beta: t
     g [B,H,T,DK] float32 (the per-token, per-channel log decay, summed within chunks by the
     kernel); h0 [B,H,DK,DV] float32 or None.  Returns (o [B,H,T,DV] float32 scaled by ``scale``
     (default DK^-1/2), h_final [B,H,DK,DV] float32 or None).  chunk_size 64 or 128 (both run
-    64-token chunks)."""
+    64-token chunks).  Few long bfloat16 sequences run in segments, as in gdn_chunk_forward."""
     if q.dim() != 4:
         raise ValueError(f"q must be [B,H,T,DK], got shape {tuple(q.shape)}")
     B, H, T, DK = q.shape

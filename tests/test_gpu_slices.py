@@ -9,7 +9,7 @@ import pytest
 import torch
 
 from conftest import announce
-from pto_fuser_amd import gdn_chunk_forward, kda_chunk_forward
+from pto_fuser_amd import _hip, gdn_chunk_forward, kda_chunk_forward, ops
 from pto_fuser_amd.forwards import make_delta_inputs
 
 pytestmark = pytest.mark.gpu
@@ -61,3 +61,25 @@ def test_a_kda_chain_does_not_depend_on_its_neighbours(H, T):
     torch.cuda.synchronize()
     assert bool(torch.isfinite(o).all() and torch.isfinite(h).all())
     assert torch.equal(on, o[:, :40]) and torch.equal(hn, h[:, :40])
+
+
+@pytest.mark.parametrize("op", ["gdn", "kda"])
+def test_long_chains_on_a_workspace_without_segments(op):
+    """Where few chains would run in segments, a workspace made for as many one-chunk chains keeps them whole:
+    again the bits they have in a batch."""
+    H, T = 72, 64 * 45
+    announce(f"{op} whole long chains H{H} T{T}")
+    fn, cls = (gdn_chunk_forward, ops.GdnWorkspace) if op == "gdn" else (kda_chunk_forward, ops.KdaWorkspace)
+    d = make_delta_inputs(1, H, T, kind=op, dtype=torch.bfloat16, seed=H + T, h0_std=0.02, device=DEV)
+
+    def run(n, whole):
+        x = {k: t[:, :n].contiguous() for k, t in d.items()}
+        ws = cls(1, n * T // 64, 64, 64, 128, 128, _hip.PF_DTYPE_BF16, DEV) if whole else None
+        out = fn(x["q"], x["k"], x["v"], x["beta"], x["g"], h0=x["h0"], workspace=ws)
+        torch.cuda.synchronize()
+        return out
+
+    o, h = run(H, False)                                 # 72 chains run whole
+    on, hn = run(8, True)
+    assert torch.equal(on, o[:, :8]) and torch.equal(hn, h[:, :8])
+    assert not torch.equal(run(8, False)[0], on)         # in segments otherwise
